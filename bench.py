@@ -776,10 +776,10 @@ def bench_lindblad_matrix(args, torch):
                                f"sqrt(0.05) a and sqrt(0.02) a^dag a, {n} initial states per launch, {nsteps} RK4 "
                                f"steps (dt {dt}), <n> and <x> every step; a step is one call (upload, launch, "
                                "download)", "instances": n, "d": d},
-        "roofline": {"bound": "mfma", "kernel": "lindblad_matrix_kernel", "launch_ms": launch_ms,
+        "roofline": {"bound": "mfma", "kernel": "lindblad_product_kernel (8 launches per step)", "launch_ms": launch_ms,
                      "flops_per_launch": flops, "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None,
-                     "note": "FP64 VALU FMAs; the MI355X FP64 vector and matrix peaks are equal"},
+                     "note": "FP64 MFMA; flops of the dense products (exactly zero 16 x 16 operator blocks are skipped)"},
         "trace_deviation": trace_dev,
     }
     if not args.no_cpu:
