@@ -244,6 +244,18 @@ int pyqed_liouville_run(int32_t N, int32_t nterm, const void* A, int32_t n_inst,
                         const double* field, int64_t nsteps, double dt, int32_t n_obs, const void* obs,
                         void* obs_out, void* rho_out, int64_t save_every, void* stream);
 
+/* pyqed_liouville_run with a workspace (device, >= pyqed_liouville_work_bytes, which is 0 when a run has no
+ * use for one; keep_states says whether rho_out is given).  With a workspace and a constant generator
+ * (nterm == 1) the states of many steps are formed at once by powers of the RK4 step matrix I + D,
+ * D = z + z^2/2 + z^3/6 + z^4/24, z = A dt -- the polynomial that the four stages of phys.py:1051-1063
+ * evaluate; other runs, and work == NULL, are pyqed_liouville_run. */
+int pyqed_liouville_work_bytes(int32_t N, int32_t nterm, int32_t n_inst, int64_t nsteps, int32_t n_obs,
+                               int32_t keep_states, int64_t save_every, int64_t* bytes);
+int pyqed_liouville_run_work(int32_t N, int32_t nterm, const void* A, int32_t n_inst, void* rho,
+                             const double* field, int64_t nsteps, double dt, int32_t n_obs, const void* obs,
+                             void* obs_out, void* rho_out, int64_t save_every, void* work, int64_t work_bytes,
+                             void* stream);
+
 /* ------------------------------------------------------------------ Lindblad, matrix form
  * Batched propagation of rho (d x d, row-major) under the Lindblad equation for any d (the
  * Liouville-space entry point above holds the N x N generator and serves N = d*d <= 1024):

@@ -1,0 +1,398 @@
+// Liouville-space RK4 of a constant generator by powers of its step matrix.
+//
+// With a generator that does not change, one RK4 step of pyqed/phys.py:1051-1063 is a fixed matrix,
+//   v' = v + D v,   D = z + z^2/2 + z^3/6 + z^4/24,   z = A dt,
+// and 2^j steps are v + D_j v with D_{j+1} = 2 D_j + D_j D_j.  The step-by-step kernel (liouville.hip) is a
+// chain of 4 nsteps dependent matrix-vector products on one workgroup; here the states of all steps are the
+// rows of matrix products: rows [2^j, 2^{j+1}) are rows [0, 2^j) advanced by D_j, and once kCap rows are
+// there every further launch makes kCap rows at a time from the last ones.  A quarter of the flops (one
+// product per step in place of four), about nsteps / kCap + 9 launches, and every CU has tiles to form.
+//
+// The increment form keeps FP64 accuracy: D is O(dt), so its rounding enters v at O(dt) of an ulp, and a
+// state is reached through log2(kCap) + nsteps / kCap additions instead of nsteps.  Against an extended-
+// precision run, over Lindblad systems of d = 2..24 and Redfield oscillators of d = 3..20 with 50..1000
+// steps, the relative error is 0.8e-16..1.3e-15, on geometric mean 0.74 times the stepping kernel's
+// (0.24..0.6 times for small |A dt|, up to 1.96 times at |A dt| = 0.075 and N = 256).  kCap bounds the powers:
+// the entries of D_j for a mode that this dt makes unstable grow like |P|^(2^j) and must stay finite even
+// if the state never excites that mode (0 x Inf would be NaN where stepping gives 0); |P|^64 overflows only
+// beyond |lambda dt| of about 35, twelve times the stability limit of RK4.
+//
+// States are rows, so the matrices are kept transposed (G_j = D_j^T): v' = v + v G.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstring>
+#include <string>
+
+#include "common.h"
+
+using namespace pqa;
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kCap = 64;            // largest number of steps in one power
+constexpr int64_t kTilesFull = 1024;  // wavefront tiles that give every SIMD of the chip one
+constexpr int64_t kScratchBytes = int64_t(256) << 20;  // states kept when the caller keeps none
+
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// One launch: the row task (rows s_in .. s_in + cnt - 1 of every instance times G, added to themselves, into
+// rows s + shift) in workgroups [0, row_blocks), then the matrix task (out = addc * add + X B, all N x N).
+struct PwParams {
+  int N, cnt, n_inst, row_blocks;
+  int64_t s_in, shift;
+  const double2* G;
+  const double2* v0;  // row 0 of instance i at v0 + i N
+  double2* V;         // row s >= 1 at V + i strideI + (s - 1) N
+  int64_t strideI;
+  const double2* X;   // matrix task
+  const double2* B;
+  const double2* add;
+  double2* out;
+  double2* w;         // set when X B = zt zt: also writes w = 1/2 + zt/6 + (X B)/24
+  double addc;
+};
+
+__device__ __forceinline__ const double2* row_ptr(const PwParams& p, int64_t inst, int64_t s) {
+  return s == 0 ? p.v0 + inst * p.N : p.V + inst * p.strideI + (s - 1) * p.N;
+}
+
+// Tiles of 16 R x 16 R per wavefront on v_mfma_f64_16x16x4_f64 (four real products per complex one), operands
+// read straight from memory (L2) in the MFMA layout, one 16-deep k-block ahead.
+//   SPLIT 4: a workgroup is one tile, its k-blocks dealt to the four wavefronts and summed through LDS in a
+//            fixed order: small launches, where the chain length counts
+//   SPLIT 1: a workgroup is four tiles; R = 2 halves the operand loads per product for launches that fill
+//            the chip
+template <int R, int SPLIT>
+__global__ __launch_bounds__(kThreads, R == 2 ? 2 : 4) void liouville_power_kernel(PwParams p) {
+  __shared__ double2 red[SPLIT == 4 ? 4 * 256 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, gi = lane & 15, gk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int N = p.N, ntc = (N + 16 * R - 1) / (16 * R);
+  const bool rows = (int)blockIdx.x < p.row_blocks;
+  const int blk = rows ? (int)blockIdx.x : (int)blockIdx.x - p.row_blocks;
+  const int wt = SPLIT == 4 ? blk : blk * 4 + wv;
+  const int nrow = rows ? p.cnt * p.n_inst : N;
+  const int tr = wt / ntc * (16 * R), tc = (wt % ntc) * (16 * R);
+  if (tr >= nrow) return;  // SPLIT 1: the tail of the last workgroup
+  // row r of the task's left operand
+  auto src = [&](int r) __attribute__((always_inline)) -> const double2* {
+    if (!rows) return p.X + r * N;
+    const int i = (int)((unsigned)r / (unsigned)p.cnt);
+    return row_ptr(p, i, p.s_in + (r - i * p.cnt));
+  };
+  const double2* ap[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) ap[u] = src(min(tr + 16 * u + gi, nrow - 1));
+  const double2* Bm = rows ? p.G : p.B;
+  struct Frag {
+    double2 a[4][R], b[4][R];
+  };
+  auto load = [&](int kb, Frag& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int k = 16 * kb + 4 * c + gk;
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int j = tc + 16 * u + gi;
+        f.a[c][u] = k < N ? ap[u][k] : make_double2(0.0, 0.0);
+        f.b[c][u] = k < N && j < N ? Bm[(unsigned)(k * N + j)] : make_double2(0.0, 0.0);
+      }
+    }
+  };
+  doublex4 sr[R][R], si[R][R];
+#pragma unroll
+  for (int u = 0; u < R; ++u)
+#pragma unroll
+    for (int v = 0; v < R; ++v) sr[u][v] = si[u][v] = doublex4{0.0, 0.0, 0.0, 0.0};
+  auto multiply = [&](const Frag& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int u = 0; u < R; ++u)
+#pragma unroll
+        for (int v = 0; v < R; ++v) {
+          const double2 a = f.a[c][u], b = f.b[c][v];
+          sr[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, sr[u][v], 0, 0, 0);
+          si[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, si[u][v], 0, 0, 0);
+          sr[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, sr[u][v], 0, 0, 0);
+          si[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, si[u][v], 0, 0, 0);
+        }
+  };
+  const int nkb = (N + 15) / 16;
+  {
+    Frag f0, f1;
+    int kb = SPLIT == 4 ? wv : 0;
+    if (kb < nkb) load(kb, f0);
+#pragma unroll 1
+    while (kb < nkb) {
+      if (kb + SPLIT < nkb) load(kb + SPLIT, f1);
+      multiply(f0);
+      kb += SPLIT;
+      if (kb >= nkb) break;
+      if (kb + SPLIT < nkb) load(kb + SPLIT, f0);
+      multiply(f1);
+      kb += SPLIT;
+    }
+  }
+  // MFMA output: register r of lane (gk, gi) holds element (4 r + gk, gi) of its 16 x 16 tile
+  auto finish = [&](int r, int j, double2 v) __attribute__((always_inline)) {
+    if (r >= nrow || j >= N) return;
+    if (rows) {
+      const int i = (int)((unsigned)r / (unsigned)p.cnt);
+      const int64_t s = p.s_in + (r - i * p.cnt);
+      const double2 x = row_ptr(p, i, s)[j];
+      p.V[i * p.strideI + (s + p.shift - 1) * N + j] = make_double2(x.x + v.x, x.y + v.y);
+    } else {
+      const unsigned e = (unsigned)(r * N + j);
+      if (p.w) {
+        const double2 z = p.X[e];
+        p.w[e] = make_double2((r == j ? 0.5 : 0.0) + (z.x / 6.0 + v.x / 24.0), z.y / 6.0 + v.y / 24.0);
+      }
+      if (p.add) {
+        const double2 x = p.add[e];
+        v.x = fma(p.addc, x.x, v.x);
+        v.y = fma(p.addc, x.y, v.y);
+      }
+      p.out[e] = v;
+    }
+  };
+  if constexpr (SPLIT == 4) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wv * 256 + (4 * r + gk) * 16 + gi] = make_double2(sr[0][0][r], si[0][0][r]);
+    __syncthreads();
+    double2 v = red[tid];
+#pragma unroll
+    for (int s = 1; s < 4; ++s) {
+      v.x += red[s * 256 + tid].x;
+      v.y += red[s * 256 + tid].y;
+    }
+    finish(tr + (tid >> 4), tc + (tid & 15), v);
+  } else {
+#pragma unroll
+    for (int u = 0; u < R; ++u)
+#pragma unroll
+      for (int v = 0; v < R; ++v)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          finish(tr + 16 * u + 4 * r + gk, tc + 16 * v + gi, make_double2(sr[u][v][r], si[u][v][r]));
+  }
+}
+
+// zt = dt A^T
+__global__ __launch_bounds__(kThreads) void liouville_step_kernel(int N, const double2* A, double dt, double2* zt) {
+  __shared__ double2 t[16][17];
+  const int nt = (N + 15) / 16, bi = blockIdx.x / nt * 16, bj = blockIdx.x % nt * 16;
+  const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+  if (bi + r < N && bj + c < N) t[r][c] = A[(int64_t)(bi + r) * N + bj + c];
+  __syncthreads();
+  if (bj + r < N && bi + c < N) zt[(int64_t)(bj + r) * N + bi + c] = make_double2(dt * t[c][r].x, dt * t[c][r].y);
+}
+
+// observables of rows s = s0 .. s0 + cnt - 1 of every instance, gsz lanes (a power of two, at most 64) to a
+// row: Tr(O rho) = sum_e obs[o][e] v[e]; row s goes to obs_out row t0 + s
+__global__ __launch_bounds__(kThreads) void liouville_observe_kernel(PwParams p, int gsz, int n_obs, const double2* obs,
+                                                                     double2* obs_out, int64_t out_rows, int64_t t0) {
+  const int li = threadIdx.x % gsz;
+  const int64_t r = blockIdx.x * (int64_t)(kThreads / gsz) + threadIdx.x / gsz;
+  const bool live = r < (int64_t)p.cnt * p.n_inst;
+  const int64_t i = live ? r / p.cnt : 0, s = live ? p.s_in + (r - i * p.cnt) : p.s_in;
+  const double2* v = row_ptr(p, i, s);
+  for (int o = 0; o < n_obs; ++o) {
+    double re = 0.0, im = 0.0;
+    for (int e = li; e < p.N; e += gsz) {
+      const double2 a = obs[(int64_t)o * p.N + e], x = v[e];
+      re += a.x * x.x - a.y * x.y;
+      im += a.x * x.y + a.y * x.x;
+    }
+    for (int w = gsz / 2; w > 0; w >>= 1) {
+      re += __shfl_xor(re, w, gsz);
+      im += __shfl_xor(im, w, gsz);
+    }
+    if (live && li == 0) obs_out[(i * out_rows + t0 + s) * n_obs + o] = make_double2(re, im);
+  }
+}
+
+// row s of every instance into out [n_inst][N]
+__global__ __launch_bounds__(kThreads) void liouville_row_kernel(PwParams p, int64_t s, double2* out) {
+  for (int64_t e = blockIdx.x * (int64_t)kThreads + threadIdx.x; e < (int64_t)p.n_inst * p.N; e += (int64_t)gridDim.x * kThreads) {
+    const int64_t i = e / p.N;
+    out[e] = row_ptr(p, i, s)[e - i * p.N];
+  }
+}
+
+struct Shape {
+  int levels;       // powers kept: 1, 2, .. 2^(levels - 1) steps
+  int64_t seg;      // states kept at a time (rows 1..seg) in the workspace; 0: in the caller's rho_out
+  int64_t bytes;
+};
+
+// Is a run served here, and what does it need?  The power path pays for forming and squaring N x N matrices
+// (about 8 products of N^3) and for a dozen launches, 45-60 us in all up to N = 64; the stepping kernel takes
+// 2 us a step up to N = 9, 5 us at 16, 16 us at 64, 115 us at 256 and 1.9 ms at 1024 (one workgroup per
+// instance streaming A from L2 four times).  Measured, stepping against powers: N = 9, 32 steps 110 / 58 us;
+// N = 25, 8 steps 63 / 49; N = 64, 8 steps 149 / 47, 1000 steps 15933 / 105; N = 256, 1000 steps 115.7 ms /
+// 191 us; N = 1024, 8 steps 15.0 / 2.1 ms; 4096 instances of N = 9, 200 steps 626 / 199 us.
+bool power_shape(int N, int n_inst, int64_t nsteps, int n_obs, bool have_out, int64_t save_every, Shape* s) {
+  if (nsteps < (N <= 16 ? 32 : N < 64 ? 8 : 4)) return false;
+  if (have_out && save_every != 1) return false;
+  const bool traj = have_out || n_obs > 0;
+  s->seg = 0;
+  if (traj && !have_out)
+    s->seg = std::max<int64_t>(1, std::min<int64_t>(nsteps, kScratchBytes / ((int64_t)n_inst * N * 16)));
+  const int64_t span = traj ? (have_out ? nsteps : s->seg) : nsteps;  // rows, or steps, a power may cover
+  s->levels = 1;
+  while ((int64_t(1) << s->levels) <= std::min<int64_t>(span, kCap)) ++s->levels;
+  const int64_t rows = traj ? (int64_t)n_inst * s->seg : n_inst;
+  s->bytes = 16 * ((int64_t)(3 + s->levels) * N * N + rows * N);
+  // rows of a launch and its grid in 32 bits
+  return (int64_t)n_inst * kCap * ((N + 15) / 16) < INT32_MAX / 2;
+}
+
+template <int R, int SPLIT>
+int launch_form(PwParams p, int64_t row_tiles, int64_t mat_tiles, hipStream_t st) {
+  constexpr int per = SPLIT == 4 ? 1 : 4;  // tiles of a workgroup
+  p.row_blocks = (int)((row_tiles + per - 1) / per);
+  hipLaunchKernelGGL((liouville_power_kernel<R, SPLIT>), dim3((unsigned)(p.row_blocks + (mat_tiles + per - 1) / per)), dim3(kThreads),
+                     0, st, p);
+  PQA_HIP(hipGetLastError());
+  return PYQED_OK;
+}
+
+int launch_power(const PwParams& p, bool rows, bool mat, hipStream_t st) {
+  const int64_t nrow = rows ? (int64_t)p.cnt * p.n_inst : 0, nm = mat ? p.N : 0;
+  const int64_t c16 = (p.N + 15) / 16, c32 = (p.N + 31) / 32;
+  const int64_t r16 = (nrow + 15) / 16 * c16, m16 = (nm + 15) / 16 * c16;
+  const int64_t r32 = (nrow + 31) / 32 * c32, m32 = (nm + 31) / 32 * c32;
+  if (p.N > 16 && r32 + m32 >= kTilesFull) return launch_form<2, 1>(p, r32, m32, st);
+  if (p.N <= 32 && r16 + m16 >= kTilesFull) return launch_form<1, 1>(p, r16, m16, st);
+  return launch_form<1, 4>(p, r16, m16, st);
+}
+
+int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps, double dt, int n_obs, const double2* obs,
+              double2* obs_out, double2* rho_out, const Shape& sh, double2* work, hipStream_t st) {
+  const int64_t NN = (int64_t)N * N;
+  double2* zt = work;
+  double2* z2 = zt + NN;
+  double2* w = z2 + NN;
+  double2* G = w + NN;  // [levels][N][N]
+  double2* V = G + sh.levels * NN;
+  int rc;
+  PwParams p;
+  std::memset(&p, 0, sizeof(p));
+  p.N = N;
+  p.n_inst = n_inst;
+  p.cnt = 1;
+  p.v0 = rho;
+  const int nt = (N + 15) / 16;
+  hipLaunchKernelGGL(liouville_step_kernel, dim3(nt * nt), dim3(kThreads), 0, st, N, A, dt, zt);
+  PQA_HIP(hipGetLastError());
+  p.X = p.B = zt;
+  p.out = z2;
+  p.w = w;
+  if ((rc = launch_power(p, false, true, st))) return rc;
+  // G_0 = z + z^2 (1/2 + z/6 + z^2/24)
+  p.X = z2;
+  p.B = w;
+  p.w = nullptr;
+  p.add = zt;
+  p.addc = 1.0;
+  p.out = G;
+  if ((rc = launch_power(p, false, true, st))) return rc;
+  p.addc = 2.0;
+  // the launch that squares power j into power j + 1 also advances rows by power j
+  auto level = [&](int j, bool rows, bool square) {
+    p.G = G + j * NN;
+    p.X = p.B = p.add = p.G;
+    p.out = G + (j + 1) * NN;
+    return launch_power(p, rows, square, st);
+  };
+  if (!rho_out && n_obs == 0) {
+    // final states only: nsteps = top * (most significant power) + remaining bits
+    const int top = sh.levels - 1;
+    double2* bufs[2] = {rho, V};
+    int cur = 0;
+    p.s_in = 0;
+    p.shift = 1;
+    p.strideI = N;
+    auto step = [&](int j, bool rows, bool square) {
+      p.v0 = bufs[cur];
+      p.V = bufs[cur ^ 1];
+      if (rows) cur ^= 1;
+      return level(j, rows, square);
+    };
+    for (int j = 0; j < top; ++j)
+      if ((rc = step(j, (nsteps >> j) & 1, true))) return rc;
+    for (int64_t k = nsteps >> top; k > 0; --k)
+      if ((rc = step(top, true, false))) return rc;
+    if (cur) {
+      p.v0 = V;
+      hipLaunchKernelGGL(liouville_row_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)n_inst * N + kThreads - 1) / kThreads, 2048)),
+                         dim3(kThreads), 0, st, p, 0, rho);
+      PQA_HIP(hipGetLastError());
+    }
+    return PYQED_OK;
+  }
+  const int64_t seg = rho_out ? nsteps : sh.seg;
+  int gsz = 1;
+  while (gsz < N && gsz < 64) gsz *= 2;
+  int have_pow = 1;  // powers formed so far
+  for (int64_t t0 = 0; t0 < nsteps; t0 += seg) {
+    const int64_t S = std::min(seg, nsteps - t0);
+    p.V = rho_out ? rho_out : V;
+    p.strideI = (rho_out ? nsteps : seg) * N;
+    int64_t have = 1;  // rows 0 .. have - 1 are in place
+    for (int j = 0; have < S + 1;) {
+      const int64_t step = int64_t(1) << j;  // have = step while doubling; then the last step rows advance
+      const int64_t cnt = std::min(step, S + 1 - have);
+      p.cnt = (int)cnt;
+      p.s_in = have - step;
+      p.shift = step;
+      const bool up = j + 1 < sh.levels && have + cnt < S + 1;
+      const bool square = up && j + 1 >= have_pow;
+      if ((rc = level(j, true, square))) return rc;
+      if (square) have_pow = j + 2;
+      if (up) ++j;
+      have += cnt;
+    }
+    p.s_in = t0 == 0 ? 0 : 1;
+    if (n_obs) {
+      p.cnt = (int)(S + 1 - p.s_in);
+      const int64_t per = kThreads / gsz, nr = (int64_t)p.cnt * n_inst;
+      hipLaunchKernelGGL(liouville_observe_kernel, dim3((unsigned)((nr + per - 1) / per)), dim3(kThreads), 0, st, p, gsz, n_obs, obs,
+                         obs_out, nsteps + 1, t0);
+      PQA_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(liouville_row_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)n_inst * N + kThreads - 1) / kThreads, 2048)),
+                       dim3(kThreads), 0, st, p, S, rho);
+    PQA_HIP(hipGetLastError());
+  }
+  return PYQED_OK;
+}
+
+}  // namespace
+
+extern "C" int pyqed_liouville_work_bytes(int32_t N, int32_t nterm, int32_t n_inst, int64_t nsteps, int32_t n_obs, int32_t keep_states,
+                                          int64_t save_every, int64_t* bytes) {
+  if (!bytes || N < 1 || N > 1024 || nterm < 1 || n_inst < 1 || nsteps < 0 || n_obs < 0)
+    return fail(PYQED_EINVAL, "liouville_work_bytes: need 1 <= N <= 1024, nterm >= 1, n_inst >= 1, nsteps >= 0, n_obs >= 0");
+  Shape s;
+  *bytes = nterm == 1 && power_shape(N, n_inst, nsteps, n_obs, keep_states != 0, save_every > 0 ? save_every : 1, &s) ? s.bytes : 0;
+  return PYQED_OK;
+}
+
+extern "C" int pyqed_liouville_run_work(int32_t N, int32_t nterm, const void* A, int32_t n_inst, void* rho, const double* field,
+                                        int64_t nsteps, double dt, int32_t n_obs, const void* obs, void* obs_out, void* rho_out,
+                                        int64_t save_every, void* work, int64_t work_bytes, void* stream) {
+  Shape s;
+  if (save_every <= 0) save_every = 1;
+  const bool ok = N >= 1 && N <= 1024 && nterm == 1 && n_inst >= 1 && A && rho && n_obs >= 0 && (n_obs == 0 || (obs && obs_out)) &&
+                  nsteps >= 0;
+  if (!ok || !work || !power_shape(N, n_inst, nsteps, n_obs, rho_out != nullptr, save_every, &s))
+    return pyqed_liouville_run(N, nterm, A, n_inst, rho, field, nsteps, dt, n_obs, obs, obs_out, rho_out, save_every, stream);
+  if (work_bytes < s.bytes)
+    return fail(PYQED_EINVAL, "liouville_run_work: workspace of " + std::to_string(work_bytes) + " bytes < " + std::to_string(s.bytes));
+  return run_power(N, (const double2*)A, n_inst, (double2*)rho, nsteps, dt, n_obs, (const double2*)obs, (double2*)obs_out, (double2*)rho_out,
+                   s, (double2*)work, (hipStream_t)stream);
+}

@@ -35,6 +35,20 @@ def lindblad_generator(H, c_ops):
     return L
 
 
+def run_workspace(torch, N, nterm, n_inst, nsteps, n_obs, keep_states, save_every, dev):
+    """Workspace of pyqed_liouville_run_work, or None where it needs none or the device has no room for it
+    (the run then steps without one)."""
+    wb = _lib.C.c_int64()
+    _lib.check(_lib.lib().pyqed_liouville_work_bytes(N, nterm, n_inst, nsteps, n_obs, int(keep_states), save_every,
+                                                     _lib.C.byref(wb)))
+    if wb.value == 0:
+        return None
+    try:
+        return torch.empty(wb.value, dtype=torch.uint8, device=dev)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 def propagate(gens, rho0s, dt, nsteps, field=None, e_ops=(), save_every=1, keep_states=True):
     """Run pyqed_liouville_run.  gens: [nterm, N, N]; rho0s: [n_inst, d, d]; field: [n_inst, nsteps,
     nterm-1] or None.  Returns (observables [n_inst, nsteps+1, n_obs], states [n_inst, nsave, d, d],
@@ -60,9 +74,10 @@ def propagate(gens, rho0s, dt, nsteps, field=None, e_ops=(), save_every=1, keep_
         obs_out = torch.empty((n_inst, nsteps + 1, n_obs), dtype=torch.complex128, device=dev)
     nsave = nsteps // save_every if keep_states else 0
     rho_out = torch.empty((n_inst, max(nsave, 1), N), dtype=torch.complex128, device=dev) if nsave else None
-    _lib.check(L.pyqed_liouville_run(N, nterm, A.data_ptr(), n_inst, rho.data_ptr(), _lib.ptr(f), nsteps, float(dt),
-                                     n_obs, _lib.ptr(obs), _lib.ptr(obs_out), _lib.ptr(rho_out), save_every,
-                                     _lib.stream_ptr(torch)))
+    work = run_workspace(torch, N, nterm, n_inst, nsteps, n_obs, rho_out is not None, save_every, dev)
+    _lib.check(L.pyqed_liouville_run_work(N, nterm, A.data_ptr(), n_inst, rho.data_ptr(), _lib.ptr(f), nsteps, float(dt),
+                                          n_obs, _lib.ptr(obs), _lib.ptr(obs_out), _lib.ptr(rho_out), save_every,
+                                          _lib.ptr(work), 0 if work is None else work.numel(), _lib.stream_ptr(torch)))
     torch.cuda.synchronize()
     o = obs_out.cpu().numpy() if n_obs else np.zeros((n_inst, nsteps + 1, 0), complex)
     st = rho_out.cpu().numpy().reshape(n_inst, -1, d, d)[:, :nsave] if nsave else np.zeros((n_inst, 0, d, d), complex)
