@@ -749,7 +749,9 @@ def bench_lindblad_matrix(args, torch):
     obs_out = torch.empty((n, nsteps + 1, 2), dtype=torch.complex128, device=dev)
     wb = _lib.C.c_int64()
     _lib.check(L.pyqed_lindblad_work_bytes(d, 2, 0, n, _lib.C.byref(wb)))
-    work = torch.empty(wb.value, dtype=torch.uint8, device=dev)
+    tb = _lib.C.c_int64()
+    _lib.check(L.pyqed_lindblad_table_bytes(d, 2, _lib.C.byref(tb)))
+    work = torch.empty(wb.value + tb.value, dtype=torch.uint8, device=dev)
     st = torch.cuda.current_stream()
     ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
 

@@ -274,8 +274,11 @@ int pyqed_liouville_run_work(int32_t N, int32_t nterm, const void* A, int32_t n_
  *   obs          device [n_obs][d][d], O^T flattened (Tr(O rho) = sum_e obs[e] rho[e]); obs_out
  *                device [n_inst][nsteps+1][n_obs] (row 0 = the initial state)
  *   rho_out      device [n_inst][nsteps/save_every][d][d] or NULL
- *   work         device, >= pyqed_lindblad_work_bytes(d, nc, ndrive, n_inst) bytes */
+ *   work         device, >= pyqed_lindblad_work_bytes(d, nc, ndrive, n_inst) bytes; with
+ *                pyqed_lindblad_table_bytes(d, nc) more, 16 x 16 blocks of the operators that are exactly
+ *                zero are found once per call and skipped (same results) */
 int pyqed_lindblad_work_bytes(int32_t d, int32_t nc, int32_t ndrive, int32_t n_inst, int64_t* bytes);
+int pyqed_lindblad_table_bytes(int32_t d, int32_t nc, int64_t* bytes);
 int pyqed_lindblad_run(int32_t d, int32_t nc, const void* Heff, const void* HeffD, const void* C, const void* CD,
                        int32_t ndrive, const void* Hd, const void* HdD, int32_t n_inst, void* rho,
                        const double* field, int64_t nsteps, double dt, int32_t n_obs, const void* obs,

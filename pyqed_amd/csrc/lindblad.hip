@@ -63,7 +63,7 @@ struct LbParams {
   double2* ws;           // per instance (ws_stride elements): X0, X1, acc, T[nc], Hs, HsD
   // Nonzero blocks, (real, imaginary) bits: operators that multiply from the left, tab[op][row tile][word]
   // with a bit per column block, op = 0..nc-1 for C_k, nc for H; then operators that multiply from the
-  // right, tab[nc + 1 + op][column tile][word] with a bit per row block.
+  // right, tab[nc + 1 + op][column tile][word] with a bit per row block.  NULL: every block counts.
   uint2* tab;
   int* flags;            // [kScanBlocks]: a workgroup of the scan met a non-finite value
   int gemm_blocks;       // workgroups that hold output tiles; the rest observe and form Hs (phase 1, stage 0)
@@ -246,7 +246,10 @@ struct Walk {
     for (int u = 0; u < R; ++u) {
       const int t = (pr.left ? tr : tc) + u;
       uint2 v = make_uint2(0, 0);
-      if (t < p.nt) v = pr.tab[(int64_t)t * p.nw + w];
+      if (t < p.nt) {
+        const uint32_t all = p.nt - 32 * w < 32 ? (1u << (p.nt - 32 * w)) - 1u : ~0u;
+        v = p.tab ? pr.tab[(int64_t)t * p.nw + w] : make_uint2(all, all);
+      }
       const uint32_t x = __builtin_amdgcn_readfirstlane(v.x), z = __builtin_amdgcn_readfirstlane(v.y);
       wre[u] = pr.scale ? z : x;  // +-i times the operator: the parts change places
       wim[u] = pr.scale ? x : z;
@@ -475,16 +478,226 @@ __global__ __launch_bounds__(kLThreads, R == 2 ? 2 : 4) void lindblad_product_ke
   }
 }
 
+// ------------------------------------------------------------------ resident form, d <= 64
+// One workgroup per instance and one launch for the whole run: NT x NT wavefronts (NT = tiles per
+// dimension) hold a 16 x 16 tile of rho, of the RK4 sum and of every product in registers, and the two
+// matrices a product reads across tiles, the stage input X and one T_k = X c_k^dag, stand in LDS (133 KB at
+// NT = 4).  Only the operators come from memory, and every workgroup reads the same ones (L2).  It wins
+// where the instances give the CUs work or where eight launches per step cost more than the products:
+// 256 dense d = 64 instances reach 44 TFLOP/s (FP64 matrix products reach 71 on this card), against 27 by
+// launches; what bounds it there is four wavefronts per SIMD waiting on operator fragments between barriers.
+template <int NT, bool DRIVEN>
+__global__ __launch_bounds__(64 * NT * NT) void lindblad_resident_kernel(LbParams p) {
+  constexpr int LD = 16 * NT + 1;  // row stride: the column reads of the left operand fall on different banks
+  extern __shared__ __align__(16) char smem[];
+  double2* X = (double2*)smem;
+  double2* T = X + 16 * NT * LD;
+  double2* red = T + 16 * NT * LD;     // [NT * NT]
+  uint2* stab = (uint2*)(red + NT * NT);  // block table: [2 (nc + 1)][NT]
+  const int tid = threadIdx.x, lane = tid & 63, gi = lane & 15, gk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int d = p.d, nc = p.nc, ti = wv / NT, tj = wv % NT;
+  const int64_t d2 = (int64_t)d * d, inst = blockIdx.x;
+  double2* rho = p.rho + inst * d2;
+  const double dt = p.dt, dt2 = dt / 2.0;
+  const int j = 16 * tj + gi, i0 = 16 * ti + gk;  // this lane's elements: (i0 + 4 r, j), r = 0..3
+  for (int e = tid; e < 2 * (nc + 1) * NT; e += 64 * NT * NT)
+    stab[e] = p.tab ? p.tab[e] : make_uint2((1u << NT) - 1u, (1u << NT) - 1u);
+  double2 y[4], a[4];
+  auto valid = [&](int r) { return i0 + 4 * r < d && j < d; };
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    y[r] = valid(r) ? rho[(i0 + 4 * r) * d + j] : make_double2(0.0, 0.0);
+    X[(i0 + 4 * r) * LD + j] = y[r];
+  }
+  // acc += (operator) M (left) or M (operator): operator element fetch(e), rows of the operator from
+  // memory, M from LDS, zero blocks skipped
+  doublex4 sr, si, tr, tm;
+  auto product = [&](doublex4& re, doublex4& im, bool left, int scale, const double2* M, int row, auto fetch)
+                     __attribute__((always_inline)) {
+    const uint2 m = stab[row * NT + (left ? ti : tj)];
+    const uint32_t mx = __builtin_amdgcn_readfirstlane(m.x), my = __builtin_amdgcn_readfirstlane(m.y);
+    const uint32_t br = scale ? my : mx, bi = scale ? mx : my;
+    uint32_t bits = mx | my;
+    auto load = [&](int kb, double2 (&f)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int k = 16 * kb + 4 * c + gk, o = 16 * (left ? ti : tj) + gi;
+        f[c] = k < d && o < d ? fetch(left ? o * d + k : k * d + o) : make_double2(0.0, 0.0);
+      }
+    };
+    auto multiply = [&](int kb, double2 (&f)[4]) __attribute__((always_inline)) {
+      double2 x[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int k = 16 * kb + 4 * c + gk;
+        x[c] = left ? M[k * LD + j] : M[(16 * ti + gi) * LD + k];
+        if (scale) f[c] = scale == 1 ? make_double2(f[c].y, -f[c].x) : make_double2(-f[c].y, f[c].x);
+      }
+      if ((br >> kb) & 1u) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          re = left ? __builtin_amdgcn_mfma_f64_16x16x4f64(f[c].x, x[c].x, re, 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f64_16x16x4f64(x[c].x, f[c].x, re, 0, 0, 0);
+          im = left ? __builtin_amdgcn_mfma_f64_16x16x4f64(f[c].x, x[c].y, im, 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f64_16x16x4f64(x[c].y, f[c].x, im, 0, 0, 0);
+        }
+      }
+      if ((bi >> kb) & 1u) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          re = left ? __builtin_amdgcn_mfma_f64_16x16x4f64(-f[c].y, x[c].y, re, 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f64_16x16x4f64(x[c].y, -f[c].y, re, 0, 0, 0);
+          im = left ? __builtin_amdgcn_mfma_f64_16x16x4f64(f[c].y, x[c].x, im, 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f64_16x16x4f64(x[c].x, f[c].y, im, 0, 0, 0);
+        }
+      }
+    };
+    double2 f0[4], f1[4];
+    auto take = [&]() __attribute__((always_inline)) {
+      const int b = __ffs(bits) - 1;
+      bits &= bits - 1;
+      return b;
+    };
+    if constexpr (NT == 4) {  // four wavefronts per SIMD cover the loads; the registers of a second block spill
+#pragma unroll 1
+      while (bits) {
+        const int kb = take();
+        load(kb, f0);
+        multiply(kb, f0);
+      }
+      return;
+    }
+    if (bits == 0) return;
+    int k0 = take(), k1;
+    load(k0, f0);
+#pragma unroll 1
+    for (;;) {
+      if (bits == 0) {
+        multiply(k0, f0);
+        break;
+      }
+      k1 = take();
+      load(k1, f1);
+      multiply(k0, f0);
+      if (bits == 0) {
+        multiply(k1, f1);
+        break;
+      }
+      k0 = take();
+      load(k0, f0);
+      multiply(k1, f1);
+    }
+  };
+  auto observe = [&](int64_t row) {
+    for (int o = 0; o < p.n_obs; ++o) {
+      double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (valid(r)) {
+          const double2 v = cmul2(p.obs[o * d2 + (i0 + 4 * r) * d + j], y[r]);
+          s.x += v.x;
+          s.y += v.y;
+        }
+      for (int w = 32; w > 0; w >>= 1) {
+        s.x += __shfl_xor(s.x, w, 64);
+        s.y += __shfl_xor(s.y, w, 64);
+      }
+      if (lane == 0) red[wv] = s;
+      __syncthreads();
+      if (tid == 0) {
+        for (int w = 1; w < NT * NT; ++w) {
+          s.x += red[w].x;
+          s.y += red[w].y;
+        }
+        p.obs_out[(inst * (p.nsteps + 1) + row) * p.n_obs + o] = s;
+      }
+      __syncthreads();
+    }
+  };
+  __syncthreads();
+  if (p.n_obs) observe(0);
+  for (int64_t s = 0; s < p.nsteps; ++s) {
+    const double* f = p.field + (inst * p.nsteps + s) * p.ndrive;
+    auto driven = [&](const double2* H, const double2* D) {
+      return [=](int e) {
+        double2 h = H[e];
+        for (int q = 0; DRIVEN && q < p.ndrive; ++q) {
+          const double2 v = D[q * d2 + e];
+          h.x -= f[q] * v.x;
+          h.y -= f[q] * v.y;
+        }
+        return h;
+      };
+    };
+#pragma unroll 1
+    for (int stage = 0; stage < 4; ++stage) {
+      const doublex4 zero = {0.0, 0.0, 0.0, 0.0};
+      sr = si = zero;
+      product(sr, si, true, 1, X, nc, driven(p.Heff, p.Hd));
+      product(sr, si, false, 2, X, 2 * nc + 1, driven(p.HeffD, p.HdD));
+#pragma unroll 1
+      for (int k = 0; k < nc; ++k) {
+        const double2* C = p.C + k * d2;
+        const double2* D = p.CD + k * d2;
+        tr = tm = zero;
+        product(tr, tm, false, 0, X, nc + 1 + k, [=](int e) { return D[e]; });
+        if (k) __syncthreads();  // T_{k-1} is no longer read
+#pragma unroll
+        for (int r = 0; r < 4; ++r) T[(i0 + 4 * r) * LD + j] = valid(r) ? make_double2(tr[r], tm[r]) : make_double2(0.0, 0.0);
+        __syncthreads();
+        product(sr, si, true, 0, T, k, [=](int e) { return C[e]; });
+      }
+      __syncthreads();  // every read of X (and T) is done
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double2 v = make_double2(sr[r], si[r]);
+        double2 x;
+        if (stage == 3) {
+          x = y[r] = make_double2(y[r].x + (a[r].x + v.x) / 6.0 * dt, y[r].y + (a[r].y + v.y) / 6.0 * dt);
+        } else {
+          const double h = stage == 2 ? dt : dt2;
+          a[r] = stage == 0 ? v : make_double2(a[r].x + 2.0 * v.x, a[r].y + 2.0 * v.y);
+          x = make_double2(y[r].x + v.x * h, y[r].y + v.y * h);
+        }
+        X[(i0 + 4 * r) * LD + j] = valid(r) ? x : make_double2(0.0, 0.0);
+      }
+      __syncthreads();
+    }
+    if (p.n_obs) observe(s + 1);
+    if (p.rho_out && (s + 1) % p.save_every == 0) {
+      double2* dst = p.rho_out + (inst * (p.nsteps / p.save_every) + (s + 1) / p.save_every - 1) * d2;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (valid(r)) dst[(i0 + 4 * r) * d + j] = y[r];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (valid(r)) rho[(i0 + 4 * r) * d + j] = y[r];
+}
+
 int lb_tiles(int d) { return (d + 15) / 16; }
 int lb_words(int d) { return (lb_tiles(d) + 31) / 32; }
 
-// bytes of the block tables and scan flags, before the instances' buffers
+// bytes of the block tables and scan flags, after the instances' buffers
 int64_t lb_table_bytes(int d, int nc) {
-  const int64_t t = 2 * (int64_t)(nc + 1) * lb_tiles(d) * lb_words(d) * (int64_t)sizeof(uint2) + kScanBlocks * (int64_t)sizeof(int);
-  return (t + 255) / 256 * 256;
+  return 2 * (int64_t)(nc + 1) * lb_tiles(d) * lb_words(d) * (int64_t)sizeof(uint2) + kScanBlocks * (int64_t)sizeof(int);
 }
 
 int64_t lb_inst_elems(int d, int nc, int ndrive) { return (int64_t)(3 + nc + (ndrive > 0 ? 2 : 0)) * d * d; }
+
+template <int NT, bool DRIVEN>
+int lb_resident(const LbParams& p, hipStream_t st) {
+  constexpr size_t mats = 2 * (size_t)(16 * NT) * (16 * NT + 1) * sizeof(double2) + NT * NT * sizeof(double2);
+  const size_t lds = mats + 2 * (size_t)(p.nc + 1) * NT * sizeof(uint2);
+  if (lds > 65536)
+    PQA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&lindblad_resident_kernel<NT, DRIVEN>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL((lindblad_resident_kernel<NT, DRIVEN>), dim3((unsigned)p.n_inst), dim3(64 * NT * NT), lds, st, p);
+  PQA_HIP(hipGetLastError());
+  return PYQED_OK;
+}
 
 template <int R>
 int lb_stage(const LbParams& base, int64_t blocks1, int64_t blocks2, hipStream_t st) {
@@ -508,7 +721,13 @@ using namespace pqa;
 extern "C" int pyqed_lindblad_work_bytes(int32_t d, int32_t nc, int32_t ndrive, int32_t n_inst, int64_t* bytes) {
   if (!bytes || d < 1 || nc < 0 || ndrive < 0 || n_inst < 1)
     return fail(PYQED_EINVAL, "lindblad_work_bytes: need d >= 1, nc >= 0, ndrive >= 0, n_inst >= 1");
-  *bytes = lb_table_bytes(d, nc) + (int64_t)n_inst * lb_inst_elems(d, nc, ndrive) * (int64_t)sizeof(double2);
+  *bytes = (int64_t)n_inst * lb_inst_elems(d, nc, ndrive) * (int64_t)sizeof(double2);
+  return PYQED_OK;
+}
+
+extern "C" int pyqed_lindblad_table_bytes(int32_t d, int32_t nc, int64_t* bytes) {
+  if (!bytes || d < 1 || nc < 0) return fail(PYQED_EINVAL, "lindblad_table_bytes: need d >= 1, nc >= 0");
+  *bytes = lb_table_bytes(d, nc);
   return PYQED_OK;
 }
 
@@ -554,14 +773,31 @@ extern "C" int pyqed_lindblad_run(int32_t d, int32_t nc, const void* Heff, const
   p.obs = (const double2*)obs;
   p.obs_out = (double2*)obs_out;
   p.rho_out = (double2*)rho_out;
-  p.tab = (uint2*)work;
-  p.flags = (int*)(p.tab + 2 * (int64_t)(nc + 1) * p.nt * p.nw);
-  p.ws = (double2*)((char*)work + lb_table_bytes(d, nc));
+  p.ws = (double2*)work;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(lindblad_scan_kernel, dim3(kScanBlocks), dim3(kLThreads), 0, st, p);
-  PQA_HIP(hipGetLastError());
-  hipLaunchKernelGGL(lindblad_table_kernel, dim3((unsigned)(2 * (nc + 1) * (int64_t)p.nt)), dim3(kLThreads), 2 * p.nw * sizeof(uint32_t), st, p);
-  PQA_HIP(hipGetLastError());
+  if (work_bytes - need >= lb_table_bytes(d, nc)) {
+    p.tab = (uint2*)((char*)work + need);
+    p.flags = (int*)(p.tab + 2 * (int64_t)(nc + 1) * p.nt * p.nw);
+    hipLaunchKernelGGL(lindblad_scan_kernel, dim3(kScanBlocks), dim3(kLThreads), 0, st, p);
+    PQA_HIP(hipGetLastError());
+    hipLaunchKernelGGL(lindblad_table_kernel, dim3((unsigned)(2 * (nc + 1) * (int64_t)p.nt)), dim3(kLThreads),
+                       2 * p.nw * sizeof(uint32_t), st, p);
+    PQA_HIP(hipGetLastError());
+  }
+  // d <= 64: the resident form from the number of instances where it is the faster one, by tiles per
+  // dimension.  us per step with two collapse operators, launches against resident, dense / banded operators:
+  // d = 16: 30-39 / 23, 29-38 / 19; d = 32: 39 / 48, 36 / 31 for one instance, 96 / 48, 78 / 32 for 256;
+  // d = 48: 98 / 138, 71 / 54 for 64, 137 / 138, 97 / 55 for 128; d = 64: 129 / 231, 82 / 75 for 64,
+  // 224 / 233, 131 / 75 for 128, 368 / 233, 181 / 75 for 256.
+  constexpr int kResFrom[5] = {0, 1, 16, 96, 96};
+  if (p.nt <= 4 && n_inst >= kResFrom[p.nt] && nc <= 256) {
+    switch (p.nt) {
+      case 1: return ndrive ? lb_resident<1, true>(p, st) : lb_resident<1, false>(p, st);
+      case 2: return ndrive ? lb_resident<2, true>(p, st) : lb_resident<2, false>(p, st);
+      case 3: return ndrive ? lb_resident<3, true>(p, st) : lb_resident<3, false>(p, st);
+      default: return ndrive ? lb_resident<4, true>(p, st) : lb_resident<4, false>(p, st);
+    }
+  }
   // 32 x 32 wavefront tiles once they give every CU a workgroup, 16 x 16 tiles split four ways below
   const int64_t t16 = (int64_t)p.nt * p.nt, t32 = (int64_t)((p.nt + 1) / 2) * ((p.nt + 1) / 2);
   const bool big = p.nt > 1 && t32 * n_inst >= 4 * kFullChip;

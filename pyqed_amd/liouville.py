@@ -154,9 +154,10 @@ def run_matrix(Heff, lefts, rights, drives, rho0s, dt, nsteps, field=None, e_ops
         obs_out = torch.empty((n_inst, nsteps + 1, n_obs), dtype=torch.complex128, device=dev)
     nsave = nsteps // save_every if keep_states else 0
     rho_out = torch.empty((n_inst, max(nsave, 1), d * d), dtype=torch.complex128, device=dev) if nsave else None
-    wb = _lib.C.c_int64()
+    wb, tb = _lib.C.c_int64(), _lib.C.c_int64()
     _lib.check(L.pyqed_lindblad_work_bytes(d, len(ls), len(hs), n_inst, _lib.C.byref(wb)))
-    work = torch.empty(max(wb.value, 16), dtype=torch.uint8, device=dev)
+    _lib.check(L.pyqed_lindblad_table_bytes(d, len(ls), _lib.C.byref(tb)))
+    work = torch.empty(wb.value + tb.value, dtype=torch.uint8, device=dev)
     _lib.check(L.pyqed_lindblad_run(d, len(ls), He.data_ptr(), HeD.data_ptr(), _lib.ptr(Lm), _lib.ptr(Rm), len(hs),
                                     _lib.ptr(Hd), _lib.ptr(HdD), n_inst, rho.data_ptr(), _lib.ptr(f), nsteps, float(dt),
                                     n_obs, _lib.ptr(obs), _lib.ptr(obs_out), _lib.ptr(rho_out), save_every,

@@ -66,3 +66,25 @@ def test_non_finite_input_spreads():
     rhos[0, 3, 50] = np.nan
     final = LindbladSolver(H, c, form="matrix").run_batch(rhos, 0.02, 1)
     assert np.isnan(final).all()
+
+
+def test_without_block_tables():
+    """A workspace of pyqed_lindblad_work_bytes alone (no room for the tables): the full products, equal to
+    the run that skips zero blocks up to rounding."""
+    import torch
+    from pyqed_amd import _lib
+    from pyqed_amd.oqs import LindbladSolver
+    L = _lib.lib()
+    for d, n in ((20, 3), (40, 2), (64, 128), (100, 1)):
+        H, c, rhos = _problem(d, n, "ladder", 6)
+        want = LindbladSolver(H, c, form="matrix").run_batch(rhos, 0.02, 3)
+        t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+        Heff = H - 0.5j * sum(x.conj().T @ x for x in c)
+        ops = [t(Heff), t(Heff.conj().T), t(np.array(c)), t(np.array([x.conj().T for x in c]))]
+        rho = t(rhos)
+        wb = _lib.C.c_int64()
+        _lib.check(L.pyqed_lindblad_work_bytes(d, len(c), 0, n, _lib.C.byref(wb)))
+        work = torch.empty(wb.value, dtype=torch.uint8, device="cuda")
+        _lib.check(L.pyqed_lindblad_run(d, len(c), *(o.data_ptr() for o in ops), 0, None, None, n, rho.data_ptr(), None, 3, 0.02, 0, None,
+                                        None, None, 1, work.data_ptr(), wb.value, torch.cuda.current_stream().cuda_stream))
+        assert np.abs(rho.cpu().numpy() - want).max() < 1e-13
