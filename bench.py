@@ -291,11 +291,11 @@ def kernel_name(stage, cls, precision, eng):
     pack = "true" if eng.packed else "false"
     if cls == 0:
         return f"heom_stage_kernel<{T}, {TI}, {T}, {stage}, {pack}>"
-    mfma = "true" if (cls >= 2 and precision == "mixed") else "false"
+    mfma = "true" if cls >= 2 else "false"
     herm = "true" if eng.hermitian else "false"
-    nt = 2 if (cls == 3 and precision == "mixed") else 1
-    # single-instance form: FP32 packed classes 1 and 3 when the class's streamed work is one instance
-    one = precision == "mixed" and eng.packed and cls in (1, 3) and eng.class_single()[cls] >= 0
+    nt = 2 if cls == 3 else 1
+    # single-instance form: packed classes 1 (FP32) and 3 when the class's streamed work is one instance
+    one = eng.packed and (cls == 3 or (cls == 1 and precision == "mixed")) and eng.class_single()[cls] >= 0
     return f"heom_proj_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {herm}, {pack}, {nt}, {'true' if one else 'false'}>"
 
 

@@ -195,7 +195,7 @@ int pyqed_heom_plan_set_variant(pyqed_heom_plan* plan, int32_t variant);
  * (host arrays [4], either may be NULL). */
 int pyqed_heom_plan_classes(const pyqed_heom_plan* plan, int64_t* items, int64_t* elems);
 /* Per kernel class (host array [4]): for classes 1 and 3 of a packed plan whose streamed work is a
- * single instance, that instance's index (their FP32 forms then run the single-instance kernel:
+ * single instance, that instance's index (class 1 in FP32 and class 3 then run the single-instance kernel:
  * instance record from the kernel arguments, neighbour lists at a fixed stride); -1 otherwise, and
  * always for classes 0 and 2.
  * No counterpart in the reference; used to name the kernels a benchmark's launches run. */

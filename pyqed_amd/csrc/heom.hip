@@ -617,9 +617,38 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(StageParams p) {
 //      (for non-Hermitian ADOs column s as well).
 // The neighbour list is sorted by site in LDS (ballot counting sort), so element (i, j) reads only
 // its two groups from the row buffer: sum_{site(t)=i} cL_t R_t(j) + sum_{site(t)=j} cR_t R_t(i)^*
-// (Hermitian ADOs: X'(i, s) = conj(X'(s, i))).  The commutator -i[H, X] runs on FP32 MFMA 16x16x4
-// for PQA_MFMA_DMIN <= d <= 16 and on VALU otherwise, while the round-trip-2 loads are in flight.
+// (Hermitian ADOs: X'(i, s) = conj(X'(s, i))).  The commutator -i[H, X] runs on MFMA 16x16x4, FP32 or FP64,
+// for PQA_MFMA_DMIN <= d <= 16 (one tile) and 17 <= d <= 32 (2 x 2 tiles) and on VALU below, while the
+// round-trip-2 loads are in flight.  In FP64 the VALU form was bound by its LDS reads (four 16-byte reads per
+// complex multiply-add) and, with a tile of its own, by 91 KB of LDS per block at d = 16; on MFMA a chunk of
+// four k reads two values per lane and the tile shares the own-matrix buffer.  Measured per step, FP64 VALU
+// against FP64 MFMA: 16 sites at depth 3 355 -> 157 us, 12 sites at depth 3 84 -> 49; 24 sites at depth 3,
+// whose VALU form did not fit LDS and ran on the generic kernel, 9193 -> 1409 us (145 KB per block, one
+// wavefront per SIMD: the latency of one ADO at a time bounds it).
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// 16 x 16 x 4 MFMA of the right-hand side's precision.  Operands: A[lane % 16][lane / 16] and
+// B[lane / 16][lane % 16] in both; result register r of lane (gk = lane / 16, gi = lane % 16) is element
+// (4 gk + r, gi) in FP32 and (4 r + gk, gi) in FP64.
+template <typename T>
+struct Mfma;
+template <>
+struct Mfma<float> {
+  typedef floatx4 acc;
+  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int gk, int r) { return 4 * gk + r; }
+};
+template <>
+struct Mfma<double> {
+  typedef doublex4 acc;
+  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int gk, int r) { return 4 * r + gk; }
+};
 
 constexpr int kMaxEnt = 64;  // neighbour entries per ADO handled by the projector path
 #ifndef PQA_PROJ_WAVES
@@ -792,7 +821,8 @@ __device__ __forceinline__ void proj_header(const StageParams& p, const InstDev&
 
 // Minimum waves per SIMD each form of the projector kernel is compiled for.
 constexpr int proj_waves(bool mfma, bool f32, bool pack, int stage, int nt) {
-  return (mfma && nt == 2) ? PQA_WIDE_WAVES
+  return (mfma && nt == 2) ? (f32 ? PQA_WIDE_WAVES : 1)
+         : mfma && !f32 ? PQA_PROJ_WAVES
          : mfma ? (pack ? (stage == 3 ? PQA_PACK_WAVES_LAST : PQA_PACK_WAVES) : PQA_PROJ_WAVES)
                 : (f32 ? PQA_VALU_WAVES : PQA_PROJ_WAVES);
 }
@@ -1026,7 +1056,7 @@ void heom_proj_kernel(StageParams p) {
       };
       if constexpr (kDMA) dma_rows();
       else issue(0, 0);
-      cpx<T> acc[4 * NT * NT];  // MFMA layout: element (16 ti + 4 gk + r, 16 tj + gi) at (ti NT + tj) 4 + r
+      cpx<T> acc[4 * NT * NT];  // MFMA layout: element (16 ti + Mfma::row(gk, r), 16 tj + gi) at (ti NT + tj) 4 + r
       Pre<kDelta> pr[NT == 1 ? 4 : kQP];
       PreM pm[NT == 1 ? 4 : kQP];
       // packed mode: the RK4 operands of this lane's upper elements (packed indices lane + 64q, at most
@@ -1046,19 +1076,16 @@ void heom_proj_kernel(StageParams p) {
       if (MFMA && NT == 1 && !PACK && PQA_RK4_HOIST == 2) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (4 * gk + r < d && gi < d) pr[r] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, 4 * gk + r, gi));
+          if (Mfma<T>::row(gk, r) < d && gi < d) pr[r] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, Mfma<T>::row(gk, r), gi));
       }
       if (a + kThreads / 64 < aend) prefetch(a + kThreads / 64);
       // ---- commutator and damping (while the neighbour loads are in flight)
       if (MFMA) {
-        floatx4 aR[NT][NT], aI[NT][NT];
+        typename Mfma<T>::acc aR[NT][NT], aI[NT][NT];
 #pragma unroll
         for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
-          for (int tj = 0; tj < NT; ++tj) {
-            aR[ti][tj] = floatx4{0.f, 0.f, 0.f, 0.f};
-            aI[ti][tj] = floatx4{0.f, 0.f, 0.f, 0.f};
-          }
+          for (int tj = 0; tj < NT; ++tj) aR[ti][tj] = aI[ti][tj] = typename Mfma<T>::acc{0, 0, 0, 0};
         // H is read from LDS for every ADO rather than kept in registers across the item's ADOs
         // (an opaque zero offset stops the compiler from hoisting the loads out of the ADO loop)
         int hz = 0;
@@ -1075,7 +1102,7 @@ void heom_proj_kernel(StageParams p) {
 #pragma unroll kUnrollKC
           for (int kc = 0; kc < nkc; ++kc) {
             const int kk = 4 * kc + gk;
-            float xar[NT], xai[NT], har[NT], hai[NT], xbr[NT], xbi[NT], hbr[NT], hbi[NT];
+            T xar[NT], xai[NT], har[NT], hai[NT], xbr[NT], xbi[NT], hbr[NT], hbi[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
               const int g = 16 * t + gi;
@@ -1087,26 +1114,26 @@ void heom_proj_kernel(StageParams p) {
               // kHalf: P is formed from the Hermitian part of X, whose diagonal is real.  The stored
               // diagonal carries rounding-level imaginary parts, which H X - X H cancels exactly and
               // H X alone would turn into a trace drift of 2 Im(H_ii X_ii)
-              xbr[t] = (float)xb.x, xbi[t] = (kHalf && kk == g) ? 0.f : (float)xb.y;
-              xar[t] = (float)xa.x, xai[t] = (float)xa.y;
-              har[t] = (float)ha.x, hai[t] = (float)ha.y, hbr[t] = (float)hb.x, hbi[t] = (float)hb.y;
+              xbr[t] = xb.x, xbi[t] = (kHalf && kk == g) ? (T)0 : xb.y;
+              xar[t] = xa.x, xai[t] = xa.y;
+              har[t] = ha.x, hai[t] = ha.y, hbr[t] = hb.x, hbi[t] = hb.y;
             }
 #pragma unroll
             for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
               for (int tj = 0; tj < NT; ++tj) {
-                floatx4 r = aR[ti][tj], m = aI[ti][tj];
+                typename Mfma<T>::acc r = aR[ti][tj], m = aI[ti][tj];
                 // + H X: rows of tile ti from H, columns of tile tj from X
-                r = __builtin_amdgcn_mfma_f32_16x16x4f32(har[ti], xbr[tj], r, 0, 0, 0);
-                if constexpr (!kRealH) r = __builtin_amdgcn_mfma_f32_16x16x4f32(-hai[ti], xbi[tj], r, 0, 0, 0);
-                m = __builtin_amdgcn_mfma_f32_16x16x4f32(har[ti], xbi[tj], m, 0, 0, 0);
-                if constexpr (!kRealH) m = __builtin_amdgcn_mfma_f32_16x16x4f32(hai[ti], xbr[tj], m, 0, 0, 0);
+                r = Mfma<T>::mul(har[ti], xbr[tj], r);
+                if constexpr (!kRealH) r = Mfma<T>::mul(-hai[ti], xbi[tj], r);
+                m = Mfma<T>::mul(har[ti], xbi[tj], m);
+                if constexpr (!kRealH) m = Mfma<T>::mul(hai[ti], xbr[tj], m);
                 // - X H
                 if constexpr (!kHalf) {
-                  r = __builtin_amdgcn_mfma_f32_16x16x4f32(xar[ti], -hbr[tj], r, 0, 0, 0);
-                  if constexpr (!kRealH) r = __builtin_amdgcn_mfma_f32_16x16x4f32(xai[ti], hbi[tj], r, 0, 0, 0);
-                  if constexpr (!kRealH) m = __builtin_amdgcn_mfma_f32_16x16x4f32(xar[ti], -hbi[tj], m, 0, 0, 0);
-                  m = __builtin_amdgcn_mfma_f32_16x16x4f32(xai[ti], -hbr[tj], m, 0, 0, 0);
+                  r = Mfma<T>::mul(xar[ti], -hbr[tj], r);
+                  if constexpr (!kRealH) r = Mfma<T>::mul(xai[ti], hbi[tj], r);
+                  if constexpr (!kRealH) m = Mfma<T>::mul(xar[ti], -hbi[tj], m);
+                  m = Mfma<T>::mul(xai[ti], -hbr[tj], m);
                 }
                 aR[ti][tj] = r;
                 aI[ti][tj] = m;
@@ -1123,7 +1150,7 @@ void heom_proj_kernel(StageParams p) {
           for (int tj = 0; tj < NT; ++tj)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const int i = 16 * ti + 4 * gk + r, j = 16 * tj + gi;
+              const int i = 16 * ti + Mfma<T>::row(gk, r), j = 16 * tj + gi;
               cpx<T>& a2 = acc[(ti * NT + tj) * 4 + r];
               a2 = mul_mi(mk<T>((T)aR[ti][tj][r], (T)aI[ti][tj][r]));
               // kHalf: -i P - (damp / 2) X here; the reader adds the conjugate of the (j, i) entry
@@ -1148,7 +1175,7 @@ void heom_proj_kernel(StageParams p) {
       } else if (MFMA && NT == 1 && PQA_RK4_HOIST == 1) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (4 * gk + r < d && gi < d) pr[r] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, 4 * gk + r, gi));
+          if (Mfma<T>::row(gk, r) < d && gi < d) pr[r] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, Mfma<T>::row(gk, r), gi));
       }
       wave_sync();
       // ---- gather the neighbour terms from the row buffer, RK4 update
@@ -1194,7 +1221,7 @@ void heom_proj_kernel(StageParams p) {
             for (int tj = 0; tj < NT; ++tj)
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                const int i = 16 * ti + 4 * gk + r, j = 16 * tj + gi;
+                const int i = 16 * ti + Mfma<T>::row(gk, r), j = 16 * tj + gi;
                 if (i < d && j < d) w.Tt[i * rs + j] = acc[(ti * NT + tj) * 4 + r];
               }
           wave_sync();
@@ -1284,39 +1311,41 @@ void heom_proj_kernel(StageParams p) {
           st(xout + I.off + base + e, mk<TO>((TO)u.x, (TO)u.y));
         }
       } else if (MFMA) {
-        // tile by tile (one for d <= 16): lane (gk, gi) holds elements (16 ti + 4 gk + r, 16 tj + gi)
+        // tile by tile (one for d <= 16): register r of lane (gk, gi) holds element
+        // (16 ti + Mfma::row(gk, r), 16 tj + gi)
 #pragma unroll
         for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
           for (int tj = 0; tj < NT; ++tj) {
-            const int j = 16 * tj + gi, i0 = 16 * ti + 4 * gk;
+            const int j = 16 * tj + gi;
+            auto row_of = [&](int r) { return 16 * ti + Mfma<T>::row(gk, r); };
             cpx<T>* at = acc + (ti * NT + tj) * 4;
             if (j < d) {
               if (NT == 2) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                  if (i0 + r < d) pr[r] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, i0 + r, j));
+                  if (row_of(r) < d) pr[r] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, row_of(r), j));
               }
-              // column term, site j: element (i0+r, j) <- cR_t * conj(R_t[i0+r])
+              // column term, site j: element (i, j) <- cR_t * conj(R_t[i])
               for (int t = w.gs[j]; t < w.gs[j + 1]; ++t) {
                 const cpx<T> c = w.cr[t];
-                const cpx<T>* row = (HERM ? w.R : w.Cc) + t * rs + i0;
+                const cpx<T>* row = (HERM ? w.R : w.Cc) + t * rs;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                   // the diagonal element keeps X'(s, s) itself, so that (cL + cR) X'(s, s) is formed exactly
                   // as without the Hermitian shortcut (cL = -cR for the n + e_k terms: no trace drift)
-                  if (i0 + r < d) cmac(at[r], c, (HERM && i0 + r != j) ? conjg(row[r]) : row[r]);
+                  if (row_of(r) < d) cmac(at[r], c, (HERM && row_of(r) != j) ? conjg(row[row_of(r)]) : row[row_of(r)]);
               }
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                const int i = i0 + r;
+                const int i = row_of(r);
                 // row term, site i: element (i, j) <- cL_t * R_t[j]
                 if (i < d)
                   for (int t = w.gs[i]; t < w.gs[i + 1]; ++t) cmac(at[r], w.cl[t], w.R[t * rs + j]);
               }
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                const int i = i0 + r;
+                const int i = row_of(r);
                 if (i < d) {
                   const int e = i * d + j;
                   const StateRef sr = state_ref<PACK>(I, a, i, j);
@@ -2402,7 +2431,7 @@ size_t stream_lds_bytes(const pyqed_heom_plan* P, size_t tsize) {
 
 size_t proj_lds_bytes(const pyqed_heom_plan* P, int c, size_t tsize) {
   const auto& q = P->pd[c];
-  const bool mfma = c >= 2 && tsize == sizeof(float);  // the MFMA forms keep their tile in the own-matrix buffer
+  const bool mfma = c >= 2;  // the MFMA forms keep their tile in the own-matrix buffer
   return proj_block_bytes(q.d2pad, q.Kmax, q.Lmax, tsize, P->packed) +
          (kThreads / 64) * proj_wave_bytes(q.d2pad, q.rowbuf, q.colbuf, tsize, P->packed && !mfma);
 }
@@ -3109,7 +3138,7 @@ int stream_grid(const pyqed_heom_plan* P, int n_items, int c) {
 }
 
 // One RK4 stage over every streamed item class: generic kernel, projector kernel with VALU
-// commutator, projector kernel with MFMA commutator (FP32 only; FP64 uses VALU).
+// commutator, projector kernel with MFMA commutator.
 // Event pair around one class launch when the plan records per-launch timing (never while the
 // stream is being captured into a graph).
 struct LaunchTimer {
@@ -3177,14 +3206,14 @@ int launch_stage_ti(pyqed_heom_plan* P, const StageParams& p0, hipStream_t st, i
       const size_t wlds = c == 3 ? proj_block_bytes(P->pd[3].d2pad, P->pd[3].Kmax, P->pd[3].Lmax, sizeof(float), true) +
                                        wide_ado_bytes(P->pd[3].d2pad, P->pd[3].rowbuf)
                                  : 0;
-      if (c == 2 && F32)
-        rc = launch(heom_proj_kernel<T, TI, T, S, F32, true, true, 1>, grid, plds, st, p);
+      if (c == 2)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 1>, grid, plds, st, p);
       else if (c == 3 && F32 && (P->variant & 2) && wlds <= (size_t)P->max_lds)
         rc = launch(heom_wide_kernel<S>, grid, wlds, st, p);
-      else if (c == 3 && F32 && one)
-        rc = launch(heom_proj_kernel<T, TI, T, S, F32, true, true, F32 ? 2 : 1, F32>, grid, plds, st, p);
-      else if (c == 3 && F32)
-        rc = launch(heom_proj_kernel<T, TI, T, S, F32, true, true, F32 ? 2 : 1>, grid, plds, st, p);
+      else if (c == 3 && one)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 2, true>, grid, plds, st, p);
+      else if (c == 3)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 2>, grid, plds, st, p);
       else if (F32 && one)
         rc = launch(heom_proj_kernel<T, TI, T, S, false, true, true, 1, F32>, grid, plds, st, p);
       else
@@ -3192,17 +3221,17 @@ int launch_stage_ti(pyqed_heom_plan* P, const StageParams& p0, hipStream_t st, i
     } else if (P->hermitian && c == 2 && F32 && (P->variant & 1) && pipe_lds_bytes(P, c) <= (size_t)P->max_lds) {
       rc = launch(heom_pipe_kernel<S>, grid, pipe_lds_bytes(P, c), st, p);
     } else if (P->hermitian) {
-      if (c == 2 && F32)
-        rc = launch(heom_proj_kernel<T, TI, T, S, F32, true, false, 1>, grid, plds, st, p);
-      else if (c == 3 && F32)
-        rc = launch(heom_proj_kernel<T, TI, T, S, F32, true, false, F32 ? 2 : 1>, grid, plds, st, p);
+      if (c == 2)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, false, 1>, grid, plds, st, p);
+      else if (c == 3)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, false, 2>, grid, plds, st, p);
       else
         rc = launch(heom_proj_kernel<T, TI, T, S, false, true, false, 1>, grid, plds, st, p);
     } else {
-      if (c == 2 && F32)
-        rc = launch(heom_proj_kernel<T, TI, T, S, F32, false, false, 1>, grid, plds, st, p);
-      else if (c == 3 && F32)
-        rc = launch(heom_proj_kernel<T, TI, T, S, F32, false, false, F32 ? 2 : 1>, grid, plds, st, p);
+      if (c == 2)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, false, false, 1>, grid, plds, st, p);
+      else if (c == 3)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, false, false, 2>, grid, plds, st, p);
       else
         rc = launch(heom_proj_kernel<T, TI, T, S, false, false, false, 1>, grid, plds, st, p);
     }

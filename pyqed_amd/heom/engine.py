@@ -272,7 +272,7 @@ class HeomEngine:
 
     def class_single(self):
         """Per kernel class: for classes 1 and 3 of a packed plan whose streamed work is one instance, its
-        index (their FP32 forms then run the single-instance kernel), else -1."""
+        index (class 1 in FP32 and class 3 then run the single-instance kernel), else -1."""
         out = np.zeros(NCLASSES, np.int32)
         _lib.check(self.L.pyqed_heom_plan_class_single(self.plan, out.ctypes.data))
         return out.tolist()
