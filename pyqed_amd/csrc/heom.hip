@@ -2510,7 +2510,12 @@ std::complex<double> cz(const double* p, int i) { return std::complex<double>(p[
 
 // Cut every instance into work items of about `target` complex elements (0: automatic), streamed
 // classes first (generic, projector/VALU, projector/MFMA), resident instances last, and split each
-// class into eight contiguous ranges of equal element count (one per XCD).  `blocks_per_cu` sets the
+// class into eight contiguous ranges of equal cost (one per XCD): elements plus neighbour-row values.  Ranks
+// follow the tiers of a hierarchy, and an ADO below the last tier has K + n neighbours where one of the last
+// has at most L, so by element count alone the first XCD of a single hierarchy got all the long ADOs (24-site
+// chain at depth 3: 1.7 times the average work; step 623 -> 562 us mixed, 1415 -> 1204 us FP64; 14 sites at
+// depth 4 in FP64 685 -> 523 us).  Up to 4 items per CU all items are resident at once and the ranges are of
+// equal length: a longer range would only queue (7 sites at depth 4 in FP64: 36 us, 49 us by cost).  `blocks_per_cu` sets the
 // persistent grid of the streamed kernels.
 void build_items(pyqed_heom_plan* P);
 
@@ -2555,7 +2560,13 @@ void build_items(pyqed_heom_plan* P) {
   for (int c = 0; c < kClasses; ++c) {
     const int b0 = P->cls_begin[c], n = P->cls_begin[c + 1] - b0;
     std::vector<int64_t> pre(n + 1, 0);
-    for (int k = 0; k < n; ++k) pre[k + 1] = pre[k] + (int64_t)P->items[b0 + k].nado * P->inst[P->items[b0 + k].inst].d2;
+    const bool by_cost = n > 4 * P->num_cu;
+    for (int k = 0; k < n; ++k) {
+      const WorkItem& w = P->items[b0 + k];
+      const InstDev& I = P->inst[w.inst];
+      const auto& rp = P->tabs.at({I.K, I.L})->rowptr;
+      pre[k + 1] = pre[k] + (by_cost ? (int64_t)w.nado * I.d2 + (int64_t)(rp[w.ado0 + w.nado] - rp[w.ado0]) * I.d : 1);
+    }
     P->xr[c][0] = 0;
     for (int x = 1; x < 8; ++x) {
       const int64_t goal = pre.back() * x / 8;
@@ -3131,10 +3142,12 @@ int launch(Kern k, int grid, size_t lds, hipStream_t s, const StageParams& p, in
   return PYQED_OK;
 }
 
-int stream_grid(const pyqed_heom_plan* P, int n_items, int c) {
-  int g = std::min(n_items, P->num_cu * P->cls_bpc[c]);
-  g = ((g + 7) / 8) * 8;
-  return std::max(g, 8);
+// Blocks of a class launch: as many on every XCD as the XCD with the most items has items, at most
+// blocks_per_cu on every CU (the XCDs' ranges are of equal cost, not of equal length).
+int stream_grid(const pyqed_heom_plan* P, int c) {
+  int most = 1;
+  for (int x = 0; x < 8; ++x) most = std::max(most, P->xr[c][x + 1] - P->xr[c][x]);
+  return 8 * std::min(most, std::max(1, (P->num_cu * P->cls_bpc[c] + 7) / 8));
 }
 
 // One RK4 stage over every streamed item class: generic kernel, projector kernel with VALU
@@ -3193,7 +3206,7 @@ int launch_stage_ti(pyqed_heom_plan* P, const StageParams& p0, hipStream_t st, i
     p.item_end = P->cls_begin[c + 1];
     p.use_xcd = 1;
     std::memcpy(p.xr, P->xr[c], sizeof(p.xr));
-    const int grid = stream_grid(P, n, c);
+    const int grid = stream_grid(P, c);
     int rc;
     // the projector kernel keeps neighbour rows (and columns) in LDS; when they do not fit, the
     // generic kernel (which any instance can use) takes the class
