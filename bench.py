@@ -606,7 +606,7 @@ def bench_c4(args, torch):
         "config": {"workload": f"3-level Lambda system, Lindblad dephasing and decay, 200 segments x 20 steps "
                                f"(dt 0.05), checkpoint every {ce}; {n} gradient problems per launch; a step "
                                "is one batch", "instances": n},
-        "roofline": {"bound": "mfma", "kernel": "liouville_adjoint_kernel", "launch_ms": launch_ms,
+        "roofline": {"bound": "mfma", "kernel": "small_adjoint_kernel (+ small_checkpoint_kernel)", "launch_ms": launch_ms,
                      "flops_per_launch": flops, "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None},
         "check_vs_single_instance": check,
@@ -689,7 +689,7 @@ def bench_lindblad(args, torch):
         "config": {"workload": f"3-level Lambda system, Lindblad dephasing and decay, 200 field segments x 20 "
                                f"steps (dt 0.05), populations every step; {n} instances per launch; a step is one "
                                "launch of 4000 RK4 steps", "instances": n},
-        "roofline": {"bound": "mfma", "kernel": "liouville_forward_kernel", "launch_ms": launch_ms,
+        "roofline": {"bound": "mfma", "kernel": "small_forward_kernel", "launch_ms": launch_ms,
                      "flops_per_launch": flops, "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None},
         "trace_deviation": float((pops - 1.0).abs().max()),

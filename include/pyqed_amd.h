@@ -248,7 +248,8 @@ int pyqed_liouville_run(int32_t N, int32_t nterm, const void* A, int32_t n_inst,
  * use for one; keep_states says whether rho_out is given).  With a workspace and a constant generator
  * (nterm == 1) the states of many steps are formed at once by powers of the RK4 step matrix I + D,
  * D = z + z^2/2 + z^3/6 + z^4/24, z = A dt -- the polynomial that the four stages of phys.py:1051-1063
- * evaluate; other runs, and work == NULL, are pyqed_liouville_run. */
+ * evaluate.  With a workspace, a driven run of N <= 16 and few instances is cut along time (segment
+ * propagators, then all segments at once).  Other runs, and work == NULL, are pyqed_liouville_run. */
 int pyqed_liouville_work_bytes(int32_t N, int32_t nterm, int32_t n_inst, int64_t nsteps, int32_t n_obs,
                                int32_t keep_states, int64_t save_every, int64_t* bytes);
 int pyqed_liouville_run_work(int32_t N, int32_t nterm, const void* A, int32_t n_inst, void* rho,
@@ -301,6 +302,17 @@ int pyqed_liouville_adjoint(int32_t N, int32_t nterm, const void* A, int32_t n_i
                             const double* field, int64_t nsteps, double dt, int32_t ckpt_every,
                             const void* rhoT_bar, double* grad_field, void* grad_A, void* rho0_bar,
                             void* ckpt, int64_t ckpt_bytes, void* stream);
+
+/* pyqed_liouville_adjoint with a workspace of pyqed_liouville_adjoint_work_bytes (at least the checkpoints that
+ * pyqed_liouville_adjoint takes; work replaces ckpt).  For N <= 16 and few instances the sweep is cut along
+ * time: the segments' propagators give every segment's first state and last adjoint state, then all segments
+ * are swept at once. */
+int pyqed_liouville_adjoint_work_bytes(int32_t N, int32_t nterm, int32_t n_inst, int64_t nsteps, int32_t ckpt_every,
+                                       int64_t* bytes);
+int pyqed_liouville_adjoint_work(int32_t N, int32_t nterm, const void* A, int32_t n_inst, const void* rho0,
+                                 const double* field, int64_t nsteps, double dt, int32_t ckpt_every,
+                                 const void* rhoT_bar, double* grad_field, void* grad_A, void* rho0_bar, void* work,
+                                 int64_t work_bytes, void* stream);
 
 /* Legacy single-exponential HEOM of oqs.HEOMSolver (modes 0, 1: forward Euler
  * with the reference's in-place sweep over the hierarchy, ADO n seeing ADO n-1

@@ -28,7 +28,8 @@ SYMBOLS = [
     "pyqed_heom_plan_classes", "pyqed_heom_plan_class_single", "pyqed_heom_plan_set_tiling", "pyqed_heom_plan_get_tiling", "pyqed_heom_plan_set_variant",
     "pyqed_heom_plan_class_state", "pyqed_heom_plan_set_timing", "pyqed_heom_plan_read_timing",
     "pyqed_heom_adjoint_work_bytes", "pyqed_heom_adjoint_contract",
-    "pyqed_liouville_run", "pyqed_liouville_work_bytes", "pyqed_liouville_run_work", "pyqed_liouville_adjoint", "pyqed_legacy_heom_run",
+    "pyqed_liouville_run", "pyqed_liouville_work_bytes", "pyqed_liouville_run_work", "pyqed_liouville_adjoint", "pyqed_liouville_adjoint_work_bytes",
+    "pyqed_liouville_adjoint_work", "pyqed_legacy_heom_run",
     "pyqed_spectral_work_bytes", "pyqed_spectral_sum", "pyqed_spectral_sum_static",
 ]
 SPECTRAL_STATIC_MAX = 1 << 20  # complex weights the static scratch of pyqed_spectral_sum_static holds
@@ -98,6 +99,8 @@ def lib():
     L.pyqed_liouville_work_bytes.argtypes = [i32, i32, i32, i64, i32, i32, i64, C.POINTER(i64)]
     L.pyqed_liouville_run_work.argtypes = [i32, i32, vp, i32, vp, vp, i64, dbl, i32, vp, vp, vp, i64, vp, i64, vp]
     L.pyqed_liouville_adjoint.argtypes = [i32, i32, vp, i32, vp, vp, i64, dbl, i32, vp, vp, vp, vp, vp, i64, vp]
+    L.pyqed_liouville_adjoint_work_bytes.argtypes = [i32, i32, i32, i64, i32, C.POINTER(i64)]
+    L.pyqed_liouville_adjoint_work.argtypes = [i32, i32, vp, i32, vp, vp, i64, dbl, i32, vp, vp, vp, vp, vp, i64, vp]
     L.pyqed_legacy_heom_run.argtypes = [i32, i32, i32, i32, vp, vp, vp, vp, vp, i64, dbl, i32, vp, vp, vp]
     L.pyqed_spectral_work_bytes.argtypes = [i32, i32]
     L.pyqed_spectral_sum.argtypes = [i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, i64, i64, i64, vp, i64, vp]

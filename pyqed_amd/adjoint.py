@@ -14,7 +14,7 @@ every `ckpt_every` steps and recomputed per segment).
 import numpy as np
 
 from . import _lib
-from .liouville import lindblad_generator, op2sop
+from .liouville import lindblad_generator, op2sop, run_workspace
 
 
 class LindbladAdjoint:
@@ -50,8 +50,10 @@ class LindbladAdjoint:
         A = torch.as_tensor(self._gens(theta), device=dev)
         rho = torch.as_tensor(np.asarray(rho0, np.complex128).reshape(1, -1).copy(), device=dev)
         f = torch.as_tensor(self._field(amps)[None], device=dev) if len(self.B) else None
-        _lib.check(L.pyqed_liouville_run(self.N, 1 + len(self.B), A.data_ptr(), 1, rho.data_ptr(), _lib.ptr(f),
-                                         self.nsteps, self.dt, 0, None, None, None, 1, _lib.stream_ptr(torch)))
+        work = run_workspace(torch, self.N, 1 + len(self.B), 1, self.nsteps, 0, False, 1, dev)
+        _lib.check(L.pyqed_liouville_run_work(self.N, 1 + len(self.B), A.data_ptr(), 1, rho.data_ptr(), _lib.ptr(f),
+                                              self.nsteps, self.dt, 0, None, None, None, 1, _lib.ptr(work),
+                                              0 if work is None else work.numel(), _lib.stream_ptr(torch)))
         torch.cuda.synchronize()
         return rho.cpu().numpy().reshape(self.shape)
 
@@ -68,13 +70,13 @@ class LindbladAdjoint:
         gf = torch.zeros((1, self.nsteps, max(nterm - 1, 1)), dtype=torch.float64, device=dev)
         gA = torch.zeros((1, nterm, self.N, self.N), dtype=torch.complex128, device=dev)
         r0b = torch.zeros((1, self.N), dtype=torch.complex128, device=dev)
-        nck = (self.nsteps + self.ckpt_every - 1) // self.ckpt_every + 1
-        ck_bytes = (nck + self.ckpt_every) * self.N * 16
-        ck = torch.empty(ck_bytes, dtype=torch.uint8, device=dev)
-        _lib.check(L.pyqed_liouville_adjoint(self.N, nterm, A.data_ptr(), 1, rho.data_ptr(), _lib.ptr(f), self.nsteps,
-                                             self.dt, self.ckpt_every, bar.data_ptr(),
-                                             gf.data_ptr() if nterm > 1 else None, gA.data_ptr(), r0b.data_ptr(),
-                                             ck.data_ptr(), ck_bytes, _lib.stream_ptr(torch)))
+        wb = _lib.C.c_int64()
+        _lib.check(L.pyqed_liouville_adjoint_work_bytes(self.N, nterm, 1, self.nsteps, self.ckpt_every, _lib.C.byref(wb)))
+        work = torch.empty(wb.value, dtype=torch.uint8, device=dev)
+        _lib.check(L.pyqed_liouville_adjoint_work(self.N, nterm, A.data_ptr(), 1, rho.data_ptr(), _lib.ptr(f), self.nsteps,
+                                                  self.dt, self.ckpt_every, bar.data_ptr(),
+                                                  gf.data_ptr() if nterm > 1 else None, gA.data_ptr(), r0b.data_ptr(),
+                                                  work.data_ptr(), wb.value, _lib.stream_ptr(torch)))
         torch.cuda.synchronize()
         gA0 = gA[0, 0].cpu().numpy()
         g_theta = np.array([np.real(np.sum(np.conj(gA0) * Gj)) for Gj in self.G])

@@ -19,10 +19,11 @@
 // recomputed from its checkpoint into a segment buffer and swept backwards.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 
-#include "common.h"
+#include "liouville.h"
 
 using namespace pqa;
 
@@ -117,9 +118,9 @@ __device__ void gf_move(const LvParams& p, const Grp& q, Win& g, int64_t s) {
 __device__ __forceinline__ double coeff(const double* cf, int i) { return i == 0 ? 1.0 : cf[i - 1]; }
 
 // generator element A_i[r][c]: from the workgroup's LDS copy (ALDS) or global memory
-template <bool ALDS, int NT>
+template <bool ALDS>
 __device__ __forceinline__ cpx<double> gen(const LvParams& p, const cpx<double>* sA, int i, int r, int c) {
-  const int N = NT > 0 ? NT : p.N;
+  const int N = p.N;
   const int64_t e = ((int64_t)i * N + r) * N + c;
   if (ALDS) return sA[e];
   const double2 a = p.A[e];
@@ -129,103 +130,57 @@ __device__ __forceinline__ cpx<double> gen(const LvParams& p, const cpx<double>*
 // sum_k A_i[r][k] x[k] (HT = false) or sum_k conj(A_i[k][r]) x[k] (HT = true), with four
 // independent partial sums: a single wave per SIMD is common here, and one accumulator would make
 // every complex multiply-add wait for the previous one
-template <bool ALDS, bool HT, int NT>
+template <bool ALDS, bool HT>
 __device__ __forceinline__ cpx<double> row_dot(const LvParams& p, const cpx<double>* sA, int i, int r,
                                                const cpx<double>* x) {
-  const int N = NT > 0 ? NT : p.N;
+  const int N = p.N;
   cpx<double> a0 = mk(0.0, 0.0), a1 = a0, a2 = a0, a3 = a0;
   int k = 0;
   for (; k + 3 < N; k += 4) {
-    cmac(a0, HT ? conjg(gen<ALDS, NT>(p, sA, i, k, r)) : gen<ALDS, NT>(p, sA, i, r, k), x[k]);
-    cmac(a1, HT ? conjg(gen<ALDS, NT>(p, sA, i, k + 1, r)) : gen<ALDS, NT>(p, sA, i, r, k + 1), x[k + 1]);
-    cmac(a2, HT ? conjg(gen<ALDS, NT>(p, sA, i, k + 2, r)) : gen<ALDS, NT>(p, sA, i, r, k + 2), x[k + 2]);
-    cmac(a3, HT ? conjg(gen<ALDS, NT>(p, sA, i, k + 3, r)) : gen<ALDS, NT>(p, sA, i, r, k + 3), x[k + 3]);
+    cmac(a0, HT ? conjg(gen<ALDS>(p, sA, i, k, r)) : gen<ALDS>(p, sA, i, r, k), x[k]);
+    cmac(a1, HT ? conjg(gen<ALDS>(p, sA, i, k + 1, r)) : gen<ALDS>(p, sA, i, r, k + 1), x[k + 1]);
+    cmac(a2, HT ? conjg(gen<ALDS>(p, sA, i, k + 2, r)) : gen<ALDS>(p, sA, i, r, k + 2), x[k + 2]);
+    cmac(a3, HT ? conjg(gen<ALDS>(p, sA, i, k + 3, r)) : gen<ALDS>(p, sA, i, r, k + 3), x[k + 3]);
   }
-  for (; k < N; ++k) cmac(a0, HT ? conjg(gen<ALDS, NT>(p, sA, i, k, r)) : gen<ALDS, NT>(p, sA, i, r, k), x[k]);
-  return (a0 + a1) + (a2 + a3);
-}
-
-// Compile-time N (with at most two generators, which the host guarantees for those instantiations):
-// the lane's row r = li of A_0 and A_1 lives in registers, so a product reads only x from LDS.
-template <int NT>
-struct Rows {
-  cpx<double> a[2][NT > 0 ? NT : 1];
-};
-
-template <bool ALDS, int NT>
-__device__ void load_rows(const LvParams& p, const Grp& q, const cpx<double>* sA, Rows<NT>& R) {
-  if constexpr (NT > 0) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int k = 0; k < NT; ++k)
-        R.a[i][k] = (q.live && q.li < NT && i < p.nterm) ? gen<ALDS, NT>(p, sA, i, q.li, k) : mk(0.0, 0.0);
-  }
-}
-
-template <int NT>
-__device__ __forceinline__ cpx<double> reg_dot(const cpx<double> (&row)[NT > 0 ? NT : 1], const cpx<double>* x) {
-  cpx<double> a0 = mk(0.0, 0.0), a1 = a0, a2 = a0, a3 = a0;
-#pragma unroll
-  for (int k = 0; k < NT; ++k) {
-    if (k % 4 == 0) cmac(a0, row[k], x[k]);
-    if (k % 4 == 1) cmac(a1, row[k], x[k]);
-    if (k % 4 == 2) cmac(a2, row[k], x[k]);
-    if (k % 4 == 3) cmac(a3, row[k], x[k]);
-  }
+  for (; k < N; ++k) cmac(a0, HT ? conjg(gen<ALDS>(p, sA, i, k, r)) : gen<ALDS>(p, sA, i, r, k), x[k]);
   return (a0 + a1) + (a2 + a3);
 }
 
 // out = A(step) x   (row r by lane r of the group, r += gsz)
-template <bool ALDS, int NT>
+template <bool ALDS>
 __device__ void matvec(const LvParams& p, const Grp& q, const cpx<double>* sA, const double* cf,
-                       const cpx<double>* x, cpx<double>* out, const Rows<NT>& R) {
-  const int N = NT > 0 ? NT : p.N;
-  if constexpr (NT > 0) {
-    if (q.live && q.li < NT) {
-      cpx<double> s = reg_dot<NT>(R.a[0], x);
-      if (p.nterm > 1) {
-        const double c = coeff(cf, 1);
-        if (c != 0.0) s = s + reg_dot<NT>(R.a[1], x) * c;
-      }
-      out[q.li] = s;
-    }
-    return;
-  }
+                       const cpx<double>* x, cpx<double>* out) {
+  const int N = p.N;
   for (int r = q.li; q.live && r < N; r += q.gsz) {
     cpx<double> s = mk(0.0, 0.0);
     for (int i = 0; i < p.nterm; ++i) {
       const double c = coeff(cf, i);
       if (c == 0.0) continue;
-      s = s + row_dot<ALDS, false, NT>(p, sA, i, r, x) * c;
+      s = s + row_dot<ALDS, false>(p, sA, i, r, x) * c;
     }
     out[r] = s;
   }
 }
 
 // out = A_i x for one generator
-template <bool ALDS, int NT>
+template <bool ALDS>
 __device__ void matvec_term(const LvParams& p, const Grp& q, const cpx<double>* sA, int i, const cpx<double>* x,
-                            cpx<double>* out, const Rows<NT>& R) {
-  const int N = NT > 0 ? NT : p.N;
-  if constexpr (NT > 0) {
-    if (q.live && q.li < NT) out[q.li] = i == 0 ? reg_dot<NT>(R.a[0], x) : reg_dot<NT>(R.a[1], x);
-    return;
-  }
-  for (int r = q.li; q.live && r < N; r += q.gsz) out[r] = row_dot<ALDS, false, NT>(p, sA, i, r, x);
+                            cpx<double>* out) {
+  const int N = p.N;
+  for (int r = q.li; q.live && r < N; r += q.gsz) out[r] = row_dot<ALDS, false>(p, sA, i, r, x);
 }
 
 // out = A(step)^H v
-template <bool ALDS, int NT>
+template <bool ALDS>
 __device__ void matvec_h(const LvParams& p, const Grp& q, const cpx<double>* sA, const double* cf,
                          const cpx<double>* v, cpx<double>* out) {
-  const int N = NT > 0 ? NT : p.N;
+  const int N = p.N;
   for (int c = q.li; q.live && c < N; c += q.gsz) {
     cpx<double> s = mk(0.0, 0.0);
     for (int i = 0; i < p.nterm; ++i) {
       const double f = coeff(cf, i);
       if (f == 0.0) continue;
-      s = s + row_dot<ALDS, true, NT>(p, sA, i, c, v) * f;
+      s = s + row_dot<ALDS, true>(p, sA, i, c, v) * f;
     }
     out[c] = s;
   }
@@ -250,9 +205,9 @@ __device__ double group_sum(const Grp& q, double v, double* red) {
   return r;
 }
 
-template <bool ALDS, int NT>
+template <bool ALDS>
 __device__ void observe(const LvParams& p, const Grp& q, const cpx<double>* v, int64_t row, double* red) {
-  const int N = NT > 0 ? NT : p.N;
+  const int N = p.N;
   for (int o = 0; o < p.n_obs; ++o) {
     cpx<double> s = mk(0.0, 0.0);
     for (int e = q.li; q.live && e < N; e += q.gsz) {
@@ -266,33 +221,33 @@ __device__ void observe(const LvParams& p, const Grp& q, const cpx<double>* v, i
 }
 
 // One RK4 step in place on v (LDS), field row cf.  Scratch: X, k, acc (each N).
-template <bool ALDS, int NT>
+template <bool ALDS>
 __device__ void rk4_step(const LvParams& p, const Grp& q, const cpx<double>* sA, const double* cf, cpx<double>* v,
-                         cpx<double>* X, cpx<double>* k, cpx<double>* acc, const Rows<NT>& R) {
-  const int N = NT > 0 ? NT : p.N;
+                         cpx<double>* X, cpx<double>* k, cpx<double>* acc) {
+  const int N = p.N;
   const double dt = p.dt, dt2 = p.dt / 2.0;
-  matvec<ALDS, NT>(p, q, sA, cf, v, k, R);  // k1
+  matvec<ALDS>(p, q, sA, cf, v, k);  // k1
   __syncthreads();
   for (int e = q.li; q.live && e < N; e += q.gsz) {
     acc[e] = k[e];
     X[e] = v[e] + k[e] * dt2;
   }
   __syncthreads();
-  matvec<ALDS, NT>(p, q, sA, cf, X, k, R);  // k2
+  matvec<ALDS>(p, q, sA, cf, X, k);  // k2
   __syncthreads();
   for (int e = q.li; q.live && e < N; e += q.gsz) {
     acc[e] = acc[e] + k[e] * 2.0;
     X[e] = v[e] + k[e] * dt2;
   }
   __syncthreads();
-  matvec<ALDS, NT>(p, q, sA, cf, X, k, R);  // k3
+  matvec<ALDS>(p, q, sA, cf, X, k);  // k3
   __syncthreads();
   for (int e = q.li; q.live && e < N; e += q.gsz) {
     acc[e] = acc[e] + k[e] * 2.0;
     X[e] = v[e] + k[e] * dt;
   }
   __syncthreads();
-  matvec<ALDS, NT>(p, q, sA, cf, X, k, R);  // k4
+  matvec<ALDS>(p, q, sA, cf, X, k);  // k4
   __syncthreads();
   for (int e = q.li; q.live && e < N; e += q.gsz) {
     const cpx<double> a = acc[e] + k[e];
@@ -302,20 +257,20 @@ __device__ void rk4_step(const LvParams& p, const Grp& q, const cpx<double>* sA,
 }
 
 // LDS copy of the generators (shared by every instance of the workgroup)
-template <bool ALDS, int NT>
+template <bool ALDS>
 __device__ void stage_generators(const LvParams& p, cpx<double>* sA) {
   if (!ALDS) return;
-  const int N = NT > 0 ? NT : p.N;
+  const int N = p.N;
   const int64_t n = (int64_t)p.nterm * N * N;
   for (int64_t e = threadIdx.x; e < n; e += blockDim.x) sA[e] = mk(p.A[e].x, p.A[e].y);
 }
 
 // LDS layout: [generators (ALDS)] [per group: 4 N state] [red: blockDim doubles]
 // [per group: field window, ch (nterm - 1) doubles]
-template <bool ALDS, int NT>
+template <bool ALDS>
 __global__ __launch_bounds__(kT) void liouville_forward_kernel(LvParams p) {
   extern __shared__ __align__(16) char smem[];
-  const int N = NT > 0 ? NT : p.N;
+  const int N = p.N;
   const Grp q = group_of(p);
   const int groups = blockDim.x / p.gsz;
   const int g = q.tid / p.gsz, nt1 = p.nterm - 1;
@@ -327,17 +282,15 @@ __global__ __launch_bounds__(kT) void liouville_forward_kernel(LvParams p) {
   cpx<double>* acc = k + N;
   double* red = (double*)(base + (int64_t)groups * 4 * N);
   Win cw{red + blockDim.x + (int64_t)g * p.ch * nt1, 0, 0};
-  stage_generators<ALDS, NT>(p, sA);
+  stage_generators<ALDS>(p, sA);
   double2* rho = p.rho + q.b * N;
   for (int e = q.li; q.live && e < N; e += q.gsz) v[e] = mk(rho[e].x, rho[e].y);
   __syncthreads();
-  Rows<NT> R;
-  load_rows<ALDS, NT>(p, q, sA, R);
-  if (p.n_obs) observe<ALDS, NT>(p, q, v, 0, red);
+  if (p.n_obs) observe<ALDS>(p, q, v, 0, red);
   for (int64_t s = 0; s < p.nsteps; ++s) {
     if (nt1) cf_ensure(p, q, cw, s, false);
-    rk4_step<ALDS, NT>(p, q, sA, nt1 ? cw.w + (s - cw.lo) * nt1 : nullptr, v, X, k, acc, R);
-    if (p.n_obs) observe<ALDS, NT>(p, q, v, s + 1, red);
+    rk4_step<ALDS>(p, q, sA, nt1 ? cw.w + (s - cw.lo) * nt1 : nullptr, v, X, k, acc);
+    if (p.n_obs) observe<ALDS>(p, q, v, s + 1, red);
     if (p.rho_out && ((s + 1) % p.save_every) == 0) {
       const int64_t slot = (s + 1) / p.save_every - 1;
       const int64_t nslot = p.nsteps / p.save_every;
@@ -357,10 +310,10 @@ __device__ double redot(const Grp& q, const cpx<double>* a, const cpx<double>* b
 
 // LDS layout: [generators (ALDS)] [per group: 11 N state, then nterm N^2 gradient accumulators (GALDS)]
 // [red: blockDim doubles] [per group: field window and field-gradient window, ch (nterm - 1) doubles each]
-template <bool ALDS, bool GALDS, int NT>
+template <bool ALDS, bool GALDS>
 __global__ __launch_bounds__(kT) void liouville_adjoint_kernel(LvParams p) {
   extern __shared__ __align__(16) char smem[];
-  const int N = NT > 0 ? NT : p.N;
+  const int N = p.N;
   const Grp q = group_of(p);
   const int groups = blockDim.x / p.gsz;
   const int64_t NN = (int64_t)N * N;
@@ -383,7 +336,7 @@ __global__ __launch_bounds__(kT) void liouville_adjoint_kernel(LvParams p) {
   const int g = q.tid / p.gsz, nt1 = p.nterm - 1;
   Win cw{red + blockDim.x + (int64_t)g * 2 * p.ch * nt1, 0, 0};
   Win gw{cw.w + (int64_t)p.ch * nt1, p.nsteps, p.nsteps};
-  stage_generators<ALDS, NT>(p, sA);
+  stage_generators<ALDS>(p, sA);
   const int64_t b = q.b;
   const double dt = p.dt;
   const int ce = p.ckpt_every;
@@ -396,11 +349,9 @@ __global__ __launch_bounds__(kT) void liouville_adjoint_kernel(LvParams p) {
     ck[e] = r;
   }
   __syncthreads();
-  Rows<NT> R;
-  load_rows<ALDS, NT>(p, q, sA, R);
   for (int64_t s = 0; s < p.nsteps; ++s) {
     if (nt1) cf_ensure(p, q, cw, s, false);
-    rk4_step<ALDS, NT>(p, q, sA, nt1 ? cw.w + (s - cw.lo) * nt1 : nullptr, v, X1, k, acc, R);
+    rk4_step<ALDS>(p, q, sA, nt1 ? cw.w + (s - cw.lo) * nt1 : nullptr, v, X1, k, acc);
     if ((s + 1) % ce == 0 && (s + 1) / ce < p.nck)
       for (int e = q.li; q.live && e < N; e += q.gsz) ck[((s + 1) / ce) * N + e] = make_double2(v[e].x, v[e].y);
   }
@@ -431,7 +382,7 @@ __global__ __launch_bounds__(kT) void liouville_adjoint_kernel(LvParams p) {
       __syncthreads();
       if (s + 1 < s1) {
         if (nt1) cf_ensure(p, q, cw, s, false);
-        rk4_step<ALDS, NT>(p, q, sA, nt1 ? cw.w + (s - cw.lo) * nt1 : nullptr, v, X1, k, acc, R);
+        rk4_step<ALDS>(p, q, sA, nt1 ? cw.w + (s - cw.lo) * nt1 : nullptr, v, X1, k, acc);
       }
     }
     __syncthreads();
@@ -448,15 +399,15 @@ __global__ __launch_bounds__(kT) void liouville_adjoint_kernel(LvParams p) {
         X1[e] = mk(r.x, r.y);
       }
       __syncthreads();
-      matvec<ALDS, NT>(p, q, sA, cf, X1, k, R);
+      matvec<ALDS>(p, q, sA, cf, X1, k);
       __syncthreads();
       for (int e = q.li; q.live && e < N; e += q.gsz) X2[e] = X1[e] + k[e] * (dt / 2.0);
       __syncthreads();
-      matvec<ALDS, NT>(p, q, sA, cf, X2, k, R);
+      matvec<ALDS>(p, q, sA, cf, X2, k);
       __syncthreads();
       for (int e = q.li; q.live && e < N; e += q.gsz) X3[e] = X1[e] + k[e] * (dt / 2.0);
       __syncthreads();
-      matvec<ALDS, NT>(p, q, sA, cf, X3, k, R);
+      matvec<ALDS>(p, q, sA, cf, X3, k);
       __syncthreads();
       for (int e = q.li; q.live && e < N; e += q.gsz) {
         X4[e] = X1[e] + k[e] * dt;
@@ -471,7 +422,7 @@ __global__ __launch_bounds__(kT) void liouville_adjoint_kernel(LvParams p) {
         cpx<double>* Xst = Xs[st];
         // field gradients: Re <kbar_s, A_i X_s>
         for (int i = 1; i < p.nterm; ++i) {
-          matvec_term<ALDS, NT>(p, q, sA, i, Xst, k, R);
+          matvec_term<ALDS>(p, q, sA, i, Xst, k);
           __syncthreads();
           const double gi = redot(q, kb, k, N, red);
           if (q.live && q.li == 0) gw.w[(s - gw.lo) * nt1 + (i - 1)] += gi;
@@ -492,7 +443,7 @@ __global__ __launch_bounds__(kT) void liouville_adjoint_kernel(LvParams p) {
             }
           }
         }
-        matvec_h<ALDS, NT>(p, q, sA, cf, kb, Xb);
+        matvec_h<ALDS>(p, q, sA, cf, kb, Xb);
         __syncthreads();
         for (int e = q.li; q.live && e < N; e += q.gsz) {
           ub[e] = ub[e] + Xb[e];
@@ -546,6 +497,43 @@ int launch_lv(K kernel, int blocks, int nth, size_t lds, hipStream_t st, const L
 
 }  // namespace
 
+namespace pqa {
+
+LiouvilleRun forward_run(int N, int nterm, const void* A, int n_inst, void* rho, const double* field, int64_t nsteps, double dt,
+                         int n_obs, const void* obs, void* obs_out, void* rho_out, int64_t save_every) {
+  LiouvilleRun r;
+  std::memset(&r, 0, sizeof(r));
+  r.N = N;
+  r.nterm = nterm;
+  r.n_inst = n_inst;
+  r.n_obs = n_obs;
+  r.nsteps = nsteps;
+  r.save_every = save_every > 0 ? save_every : 1;
+  r.dt = dt;
+  r.A = (const double2*)A;
+  r.field = field;
+  r.rho = (double2*)rho;
+  r.obs = (const double2*)obs;
+  r.obs_out = (double2*)obs_out;
+  r.rho_out = (double2*)rho_out;
+  return r;
+}
+
+LiouvilleRun adjoint_run(int N, int nterm, const void* A, int n_inst, const void* rho0, const double* field, int64_t nsteps,
+                         double dt, int64_t seg, const void* rhoT_bar, double* grad_field, void* grad_A, void* rho0_bar,
+                         void* ckpt) {
+  LiouvilleRun r = forward_run(N, nterm, A, n_inst, const_cast<void*>(rho0), field, nsteps, dt, 0, nullptr, nullptr, nullptr, 1);
+  r.rhoT_bar = (const double2*)rhoT_bar;
+  r.grad_field = grad_field;
+  r.grad_A = (double2*)grad_A;
+  r.rho0_bar = (double2*)rho0_bar;
+  r.ckpt = (double2*)ckpt;
+  r.seg = seg;
+  return r;
+}
+
+}  // namespace pqa
+
 extern "C" int pyqed_liouville_run(int32_t N, int32_t nterm, const void* A, int32_t n_inst, void* rho,
                                    const double* field, int64_t nsteps, double dt, int32_t n_obs, const void* obs,
                                    void* obs_out, void* rho_out, int64_t save_every, void* stream) {
@@ -554,6 +542,9 @@ extern "C" int pyqed_liouville_run(int32_t N, int32_t nterm, const void* A, int3
   if (nterm > 1 && !field) return fail(PYQED_EINVAL, "liouville_run: nterm > 1 needs a field table");
   if (n_obs < 0 || (n_obs > 0 && (!obs || !obs_out))) return fail(PYQED_EINVAL, "liouville_run: bad observables");
   if (nsteps < 0) return fail(PYQED_EINVAL, "liouville_run: negative step count");
+  if (small_fits(N, nterm, false))
+    return small_forward(forward_run(N, nterm, A, n_inst, rho, field, nsteps, dt, n_obs, obs, obs_out, rho_out, save_every),
+                         (hipStream_t)stream);
   LvParams p;
   std::memset(&p, 0, sizeof(p));
   p.N = N;
@@ -583,12 +574,8 @@ extern "C" int pyqed_liouville_run(int32_t N, int32_t nterm, const void* A, int3
   const size_t lds = (alds ? a_bytes : 0) + st_bytes;
   if (lds > maxl) return fail(PYQED_EINVAL, "liouville_run: the state does not fit one workgroup's LDS");
   hipStream_t st = (hipStream_t)stream;
-  // N = 4 (a qubit) and N = 9 (three levels) at compile time, at most two generators: the lane's
-  // generator rows in registers, the row products unrolled
-  if (alds && nterm <= 2 && N == 4) return launch_lv(liouville_forward_kernel<true, 4>, blocks, nth, lds, st, p);
-  if (alds && nterm <= 2 && N == 9) return launch_lv(liouville_forward_kernel<true, 9>, blocks, nth, lds, st, p);
-  return alds ? launch_lv(liouville_forward_kernel<true, 0>, blocks, nth, lds, st, p)
-              : launch_lv(liouville_forward_kernel<false, 0>, blocks, nth, lds, st, p);
+  return alds ? launch_lv(liouville_forward_kernel<true>, blocks, nth, lds, st, p)
+              : launch_lv(liouville_forward_kernel<false>, blocks, nth, lds, st, p);
 }
 
 extern "C" int pyqed_liouville_adjoint(int32_t N, int32_t nterm, const void* A, int32_t n_inst, const void* rho0,
@@ -605,6 +592,10 @@ extern "C" int pyqed_liouville_adjoint(int32_t N, int32_t nterm, const void* A, 
   if (ckpt_bytes < need)
     return fail(PYQED_EINVAL, "liouville_adjoint: checkpoint workspace too small (" + std::to_string(ckpt_bytes) +
                                   " < " + std::to_string(need) + ")");
+  if (small_fits(N, nterm, grad_A != nullptr))
+    return small_adjoint(adjoint_run(N, nterm, A, n_inst, rho0, field, nsteps, dt, ckpt_every, rhoT_bar, grad_field, grad_A,
+                                     rho0_bar, ckpt),
+                         (hipStream_t)stream);
   LvParams p;
   std::memset(&p, 0, sizeof(p));
   p.N = N;
@@ -641,12 +632,34 @@ extern "C" int pyqed_liouville_adjoint(int32_t N, int32_t nterm, const void* A, 
   const size_t lds = (alds ? a_bytes : 0) + st2;
   if (lds > maxl) return fail(PYQED_EINVAL, "liouville_adjoint: the state does not fit one workgroup's LDS");
   hipStream_t st = (hipStream_t)stream;
-  if (alds && galds && nterm <= 2 && N == 4)
-    return launch_lv(liouville_adjoint_kernel<true, true, 4>, blocks, nth, lds, st, p);
-  if (alds && galds && nterm <= 2 && N == 9)
-    return launch_lv(liouville_adjoint_kernel<true, true, 9>, blocks, nth, lds, st, p);
-  if (alds && galds) return launch_lv(liouville_adjoint_kernel<true, true, 0>, blocks, nth, lds, st, p);
-  if (alds) return launch_lv(liouville_adjoint_kernel<true, false, 0>, blocks, nth, lds, st, p);
-  if (galds) return launch_lv(liouville_adjoint_kernel<false, true, 0>, blocks, nth, lds, st, p);
-  return launch_lv(liouville_adjoint_kernel<false, false, 0>, blocks, nth, lds, st, p);
+  if (alds && galds) return launch_lv(liouville_adjoint_kernel<true, true>, blocks, nth, lds, st, p);
+  if (alds) return launch_lv(liouville_adjoint_kernel<true, false>, blocks, nth, lds, st, p);
+  if (galds) return launch_lv(liouville_adjoint_kernel<false, true>, blocks, nth, lds, st, p);
+  return launch_lv(liouville_adjoint_kernel<false, false>, blocks, nth, lds, st, p);
+}
+
+extern "C" int pyqed_liouville_adjoint_work_bytes(int32_t N, int32_t nterm, int32_t n_inst, int64_t nsteps, int32_t ckpt_every,
+                                                  int64_t* bytes) {
+  if (!bytes || N < 1 || N > 512 || nterm < 1 || n_inst < 1 || nsteps < 1 || ckpt_every < 1)
+    return fail(PYQED_EINVAL, "liouville_adjoint_work_bytes: need 1 <= N <= 512 and positive sizes");
+  const int64_t nck = (nsteps + ckpt_every - 1) / ckpt_every + 1;
+  const int64_t ckpt = ((int64_t)n_inst * nck * N + (int64_t)n_inst * ckpt_every * N) * 16;
+  const int64_t seg = small_fits(N, nterm, true) ? small_split(N, nterm, n_inst, nsteps, true) : 0;
+  *bytes = std::max(ckpt, seg ? small_split_bytes(N, nterm, n_inst, nsteps, seg, true) : 0);
+  return PYQED_OK;
+}
+
+extern "C" int pyqed_liouville_adjoint_work(int32_t N, int32_t nterm, const void* A, int32_t n_inst, const void* rho0,
+                                            const double* field, int64_t nsteps, double dt, int32_t ckpt_every,
+                                            const void* rhoT_bar, double* grad_field, void* grad_A, void* rho0_bar, void* work,
+                                            int64_t work_bytes, void* stream) {
+  const bool ok = N >= 1 && nterm >= 1 && n_inst >= 1 && A && rho0 && rhoT_bar && work && nsteps >= 1 && ckpt_every >= 1 &&
+                  (nterm == 1 || (field && grad_field));
+  const int64_t seg = ok && small_fits(N, nterm, true) ? small_split(N, nterm, n_inst, nsteps, true) : 0;
+  if (seg && work_bytes >= small_split_bytes(N, nterm, n_inst, nsteps, seg, true))
+    return small_adjoint_split(adjoint_run(N, nterm, A, n_inst, rho0, field, nsteps, dt, seg, rhoT_bar, grad_field, grad_A, rho0_bar,
+                                           nullptr),
+                               work, (hipStream_t)stream);
+  return pyqed_liouville_adjoint(N, nterm, A, n_inst, rho0, field, nsteps, dt, ckpt_every, rhoT_bar, grad_field, grad_A, rho0_bar, work,
+                                 work_bytes, stream);
 }

@@ -24,7 +24,7 @@
 #include <cstring>
 #include <string>
 
-#include "common.h"
+#include "liouville.h"
 
 using namespace pqa;
 
@@ -229,13 +229,13 @@ struct Shape {
 };
 
 // Is a run served here, and what does it need?  The power path pays for forming and squaring N x N matrices
-// (about 8 products of N^3) and for a dozen launches, 45-60 us in all up to N = 64; the stepping kernel takes
-// 2 us a step up to N = 9, 5 us at 16, 16 us at 64, 115 us at 256 and 1.9 ms at 1024 (one workgroup per
-// instance streaming A from L2 four times).  Measured, stepping against powers: N = 9, 32 steps 110 / 58 us;
-// N = 25, 8 steps 63 / 49; N = 64, 8 steps 149 / 47, 1000 steps 15933 / 105; N = 256, 1000 steps 115.7 ms /
-// 191 us; N = 1024, 8 steps 15.0 / 2.1 ms; 4096 instances of N = 9, 200 steps 626 / 199 us.
+// (about 8 products of N^3) and for a dozen launches, 45-60 us in all up to N = 64; the stepping kernels take
+// 0.7 us a step at N = 4, 1.0 at 9, 1.5 at 16, 8 at 25, 16 at 64, 115 at 256 and 1900 at 1024 (one workgroup
+// per instance streaming A from L2 four times).  Measured, stepping against powers: N = 25, 8 steps 63 / 49 us;
+// N = 64, 8 steps 149 / 47, 1000 steps 15933 / 105; N = 256, 1000 steps 115.7 ms / 191 us; N = 1024, 8 steps
+// 15.0 / 2.1 ms; 4096 instances of N = 9, 200 steps with observables 450 / 199 us.
 bool power_shape(int N, int n_inst, int64_t nsteps, int n_obs, bool have_out, int64_t save_every, Shape* s) {
-  if (nsteps < (N <= 16 ? 32 : N < 64 ? 8 : 4)) return false;
+  if (nsteps < (N <= 4 ? 80 : N <= 9 ? 50 : N <= 16 ? 32 : N < 64 ? 8 : 4)) return false;
   if (have_out && save_every != 1) return false;
   const bool traj = have_out || n_obs > 0;
   s->seg = 0;
@@ -378,7 +378,12 @@ extern "C" int pyqed_liouville_work_bytes(int32_t N, int32_t nterm, int32_t n_in
   if (!bytes || N < 1 || N > 1024 || nterm < 1 || n_inst < 1 || nsteps < 0 || n_obs < 0)
     return fail(PYQED_EINVAL, "liouville_work_bytes: need 1 <= N <= 1024, nterm >= 1, n_inst >= 1, nsteps >= 0, n_obs >= 0");
   Shape s;
-  *bytes = nterm == 1 && power_shape(N, n_inst, nsteps, n_obs, keep_states != 0, save_every > 0 ? save_every : 1, &s) ? s.bytes : 0;
+  if (nterm == 1 && power_shape(N, n_inst, nsteps, n_obs, keep_states != 0, save_every > 0 ? save_every : 1, &s)) {
+    *bytes = s.bytes;
+    return PYQED_OK;
+  }
+  const int64_t seg = small_fits(N, nterm, false) ? small_split(N, nterm, n_inst, nsteps, false) : 0;
+  *bytes = seg ? small_split_bytes(N, nterm, n_inst, nsteps, seg, false) : 0;
   return PYQED_OK;
 }
 
@@ -387,10 +392,17 @@ extern "C" int pyqed_liouville_run_work(int32_t N, int32_t nterm, const void* A,
                                         int64_t save_every, void* work, int64_t work_bytes, void* stream) {
   Shape s;
   if (save_every <= 0) save_every = 1;
-  const bool ok = N >= 1 && N <= 1024 && nterm == 1 && n_inst >= 1 && A && rho && n_obs >= 0 && (n_obs == 0 || (obs && obs_out)) &&
-                  nsteps >= 0;
-  if (!ok || !work || !power_shape(N, n_inst, nsteps, n_obs, rho_out != nullptr, save_every, &s))
+  const bool ok = N >= 1 && N <= 1024 && nterm >= 1 && n_inst >= 1 && A && rho && n_obs >= 0 &&
+                  (n_obs == 0 || (obs && obs_out)) && nsteps >= 0 && (nterm == 1 || field) && work;
+  if (!ok || nterm > 1 || !power_shape(N, n_inst, nsteps, n_obs, rho_out != nullptr, save_every, &s)) {
+    const int64_t seg = ok && small_fits(N, nterm, false) ? small_split(N, nterm, n_inst, nsteps, false) : 0;
+    if (seg && work_bytes >= small_split_bytes(N, nterm, n_inst, nsteps, seg, false)) {
+      LiouvilleRun r = forward_run(N, nterm, A, n_inst, rho, field, nsteps, dt, n_obs, obs, obs_out, rho_out, save_every);
+      r.seg = seg;
+      return small_forward_split(r, work, (hipStream_t)stream);
+    }
     return pyqed_liouville_run(N, nterm, A, n_inst, rho, field, nsteps, dt, n_obs, obs, obs_out, rho_out, save_every, stream);
+  }
   if (work_bytes < s.bytes)
     return fail(PYQED_EINVAL, "liouville_run_work: workspace of " + std::to_string(work_bytes) + " bytes < " + std::to_string(s.bytes));
   return run_power(N, (const double2*)A, n_inst, (double2*)rho, nsteps, dt, n_obs, (const double2*)obs, (double2*)obs_out, (double2*)rho_out,

@@ -35,7 +35,7 @@ def _run(A, r0, nt, mode, power, dt=0.01, obs=None):
 
 
 @pytest.mark.parametrize("mode", ["final", "obs", "traj", "both"])
-@pytest.mark.parametrize("N,n,nt", [(1, 3, 40), (4, 1, 32), (9, 5, 63), (15, 2, 64), (16, 1, 65), (17, 3, 127), (33, 1, 128), (49, 2, 129),
+@pytest.mark.parametrize("N,n,nt", [(1, 3, 100), (4, 1, 80), (9, 5, 63), (15, 2, 64), (16, 1, 65), (17, 3, 127), (33, 1, 128), (49, 2, 129),
                                     (64, 1, 4), (64, 40, 200), (9, 4096, 100), (33, 600, 70), (25, 4096, 180)])
 def test_powers_equal_stepping(N, n, nt, mode):
     if mode in ("traj", "both") and n > 1000:
