@@ -222,6 +222,19 @@ __global__ __launch_bounds__(kThreads) void liouville_row_kernel(PwParams p, int
   }
 }
 
+// the first n elements of the rows after every `every` steps, to out + slot stride (one instance)
+struct Pick {
+  double2* out;
+  int n;
+  int64_t stride, every;
+};
+
+__global__ __launch_bounds__(64) void liouville_pick_kernel(PwParams p, Pick k, int64_t t0, int64_t slot0) {
+  const int64_t slot = slot0 + blockIdx.x, s = (slot + 1) * k.every - t0;  // row of the slot's step
+  const double2* v = row_ptr(p, 0, s);
+  for (int e = threadIdx.x; e < k.n; e += 64) k.out[slot * k.stride + e] = v[e];
+}
+
 struct Shape {
   int levels;       // powers kept: 1, 2, .. 2^(levels - 1) steps
   int64_t seg;      // states kept at a time (rows 1..seg) in the workspace; 0: in the caller's rho_out
@@ -271,7 +284,7 @@ int launch_power(const PwParams& p, bool rows, bool mat, hipStream_t st) {
 }
 
 int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps, double dt, int n_obs, const double2* obs,
-              double2* obs_out, double2* rho_out, const Shape& sh, double2* work, hipStream_t st) {
+              double2* obs_out, double2* rho_out, const Shape& sh, double2* work, hipStream_t st, const Pick* pick = nullptr) {
   const int64_t NN = (int64_t)N * N;
   double2* zt = work;
   double2* z2 = zt + NN;
@@ -308,7 +321,7 @@ int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps,
     p.out = G + (j + 1) * NN;
     return launch_power(p, rows, square, st);
   };
-  if (!rho_out && n_obs == 0) {
+  if (!rho_out && n_obs == 0 && !pick) {
     // final states only: nsteps = top * (most significant power) + remaining bits
     const int top = sh.levels - 1;
     double2* bufs[2] = {rho, V};
@@ -364,6 +377,11 @@ int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps,
                          obs_out, nsteps + 1, t0);
       PQA_HIP(hipGetLastError());
     }
+    if (pick && (t0 + S) / pick->every > t0 / pick->every) {
+      const int64_t slot0 = t0 / pick->every;
+      hipLaunchKernelGGL(liouville_pick_kernel, dim3((unsigned)((t0 + S) / pick->every - slot0)), dim3(64), 0, st, p, *pick, t0, slot0);
+      PQA_HIP(hipGetLastError());
+    }
     hipLaunchKernelGGL(liouville_row_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)n_inst * N + kThreads - 1) / kThreads, 2048)),
                        dim3(kThreads), 0, st, p, S, rho);
     PQA_HIP(hipGetLastError());
@@ -371,7 +389,27 @@ int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps,
   return PYQED_OK;
 }
 
+// One vector of N <= 1024 elements by powers of its step matrix, kRowSeg rows at a time.
+constexpr int64_t kRowSeg = 1024;
+
 }  // namespace
+
+namespace pqa {
+
+int64_t power_vector_bytes(int N) { return 16 * ((int64_t)(3 + 7) * N * N + kRowSeg * N); }
+
+int power_vector(int N, const double2* A, double2* v, int64_t nsteps, double dt, double2* out, int n_out, int64_t out_stride,
+                 int64_t every, void* work, hipStream_t st) {
+  Shape s;
+  s.seg = std::min(nsteps, kRowSeg);
+  s.levels = 1;
+  while ((int64_t(1) << s.levels) <= std::min<int64_t>(out ? s.seg : nsteps, kCap)) ++s.levels;
+  s.bytes = 0;
+  const Pick k{out, n_out, out_stride, every};
+  return run_power(N, A, 1, v, nsteps, dt, 0, nullptr, nullptr, nullptr, s, (double2*)work, st, out ? &k : nullptr);
+}
+
+}  // namespace pqa
 
 extern "C" int pyqed_liouville_work_bytes(int32_t N, int32_t nterm, int32_t n_inst, int64_t nsteps, int32_t n_obs, int32_t keep_states,
                                           int64_t save_every, int64_t* bytes) {
