@@ -294,9 +294,13 @@ def kernel_name(stage, cls, precision, eng):
     mfma = "true" if cls >= 2 else "false"
     herm = "true" if eng.hermitian else "false"
     nt = 2 if cls == 3 else 1
-    # single-instance form: packed classes 1 (FP32) and 3 when the class's streamed work is one instance
-    one = eng.packed and (cls == 3 or (cls == 1 and precision == "mixed")) and eng.class_single()[cls] >= 0
-    return f"heom_proj_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {herm}, {pack}, {nt}, {'true' if one else 'false'}>"
+    # single-instance form: packed classes 1 to 3 when the class's streamed work is one instance; launches
+    # with more items than resident blocks (at most 8 on each of 256 CUs) loop over them
+    if eng.packed and eng.class_single()[cls] >= 0:
+        if eng.classes()["items"][cls] > 8 * 256:
+            return f"heom_proj_loop_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {nt}>"
+        return f"heom_proj_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {herm}, {pack}, {nt}, true>"
+    return f"heom_proj_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {herm}, {pack}, {nt}, false>"
 
 
 def measured_traffic(name, key, workload, packed, tiling):

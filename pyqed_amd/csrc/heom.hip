@@ -718,14 +718,46 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The value a lane exchanges with in step o of a butterfly sum over the wavefront (o = 32, 16, .. 1, in that
+// order), by permute instructions of the vector ALU instead of LDS lane exchanges.  row_ror:4 reads lane
+// (i + 4) mod 16 of the row, which holds the value of lane i ^ 4 since the step before made lanes i and i ^ 8
+// equal.  Lane layouts: permlane32_swap with both operands v gives (v[i & 31], v[i | 32]), permlane16_swap
+// (v[i & ~16], v[i | 16]), whose sum is the step's sum in every lane.
+template <int O>
+__device__ __forceinline__ uint32_t dpp_word(uint32_t v) {
+  constexpr int ctrl = O == 8 ? 0x128 : O == 4 ? 0x124 : O == 2 ? 0x4E : 0xB1;
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, true);
+}
+template <int O, typename T>
+__device__ __forceinline__ T butterfly(T v) {
+  constexpr int W = sizeof(T) / 4;
+  uint32_t a[W], b[W];
+  __builtin_memcpy(a, &v, sizeof(T));
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    if constexpr (O >= 16) {
+      const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap(a[w], a[w], false, false)
+                             : __builtin_amdgcn_permlane16_swap(a[w], a[w], false, false);
+      a[w] = r[0];
+      b[w] = r[1];
+    } else {
+      b[w] = dpp_word<O>(a[w]);
+    }
+  }
+  T x, y;
+  __builtin_memcpy(&x, a, sizeof(T));
+  __builtin_memcpy(&y, b, sizeof(T));
+  return x + y;
+}
+
+// Sum over the wavefront, the same in every lane: the butterfly of lane exchanges by 32, 16, 8, 4, 2, 1.
+template <typename T>
+__device__ __forceinline__ T wave_sum(T v) {
+  return butterfly<1>(butterfly<2>(butterfly<4>(butterfly<8>(butterfly<16>(butterfly<32>(v))))));
+}
 template <typename T>
 __device__ __forceinline__ cpx<T> wave_sum(cpx<T> v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    v.x += __shfl_xor(v.x, o, 64);
-    v.y += __shfl_xor(v.y, o, 64);
-  }
-  return v;
+  return mk(wave_sum(v.x), wave_sum(v.y));
 }
 
 // Site order of a wave's neighbour list (one entry per lane, my_site = INT_MAX past the end):
@@ -829,10 +861,14 @@ constexpr int proj_waves(bool mfma, bool f32, bool pack, int stage, int nt) {
 
 // NT: MFMA tiles per dimension, 1 for d <= 16 (one 16 x 16 tile) or 2 for d <= 32 (2 x 2 tiles of 16).
 // ONE: the class holds a single instance (StageParams::one_per, inst0, ent_fix); a compile-time form so
-// that the table-driven forms keep their registers.
-template <typename T, typename TI, typename TO, int STAGE, bool MFMA, bool HERM, bool PACK, int NT, bool ONE = false>
-__global__ __launch_bounds__(kThreads, proj_waves(MFMA, std::is_same<T, float>::value, PACK, STAGE, NT))
-void heom_proj_kernel(StageParams p) {
+// that the table-driven forms keep their registers.  1: a block has one item, as in launches whose blocks are
+// all resident at once; 2: a block runs through several items, loads the instance once and keeps its prefetch
+// going from item to item.  Measured per step, 16 sites at depth 3: FP64 120 us with form 1 and 110 with
+// form 2 (138 with a header per item of four ADOs per wavefront and all blocks launched), mixed 76 and 75 (86);
+// 7 sites at depth 4, one item per block: mixed 30.1 and 32.1 us (the second prefetch is code that every
+// launch fetches).
+template <typename T, typename TI, typename TO, int STAGE, bool MFMA, bool HERM, bool PACK, int NT, int ONE>
+__device__ __forceinline__ void proj_body(const StageParams& p) {
   constexpr bool kDelta = std::is_same<TO, float>::value;  // mixed precision: FP32 RK4 increment
   constexpr bool kPM = kDelta && PACK;  // packed mixed run: two FP32 registers (rk4_upper_m)
   static_assert(NT == 1 || (NT == 2 && MFMA), "2 x 2 tiles are an MFMA form");
@@ -878,6 +914,13 @@ void heom_proj_kernel(StageParams p) {
   constexpr bool kHalf = PQA_HALF_COMMUTATOR && MFMA && PACK && HERM;
   int it0, itstep, itend;
   item_range(p, it0, itend, itstep);
+  // Software pipeline over this wave's ADOs: the neighbour list (and, on the MFMA path, the own
+  // matrix) of the next ADO are loaded while the current one is processed; they are issued after
+  // the current ADO's neighbour loads, so waiting for those does not wait for the prefetch.  With a
+  // single instance the pipeline runs on across work items.
+  int nent_n = 0;
+  int2 en_n = make_int2(0, 0);
+  cpx_store<TI> xt_n[kPF];
   for (int it = it0; it < itend; it += itstep) {
     const WorkItem wi = ONE ? one_item(p, it) : ro_load(p.items + it);
     const InstDev I = ONE ? p.inst0 : ro_load(p.insts + wi.inst);
@@ -888,13 +931,7 @@ void heom_proj_kernel(StageParams p) {
     // the A operand (stride rs) and the rows of the row buffer fall on different banks
     const int rs = d + 1;
     const cpx_store<TI>* xi = xin + I.off;
-    // Software pipeline over this wave's ADOs: the neighbour list (and, on the MFMA path, the own
-    // matrix) of the next ADO are loaded while the current one is processed; they are issued after
-    // the current ADO's neighbour loads, so waiting for those does not wait for the prefetch.
     const int aend = wi.ado0 + wi.nado;
-    int nent_n = 0;
-    int2 en_n = make_int2(0, 0);
-    cpx_store<TI> xt_n[kPF];
     auto prefetch = [&](int an) {
       if constexpr (ONE) {
         // the list's address does not depend on the row pointers, which only give its length
@@ -914,11 +951,13 @@ void heom_proj_kernel(StageParams p) {
       }
     };
     // the first ADO's list and matrix are requested before the instance header, so the two round
-    // trips overlap (the prefetch touches registers only)
-    if (wi.ado0 + wv < aend) prefetch(wi.ado0 + wv);
-    __syncthreads();
-    proj_header<T>(p, I, col, dmag, sH, sC, sSite, sS, PACK ? sIJ : nullptr);
-    __syncthreads();
+    // trips overlap (the prefetch touches registers only).  A single instance's header serves every item.
+    if (ONE != 2 || it == it0) {
+      if (wi.ado0 + wv < aend) prefetch(wi.ado0 + wv);
+      __syncthreads();
+      proj_header<T>(p, I, col, dmag, sH, sC, sSite, sS, PACK ? sIJ : nullptr);
+      __syncthreads();
+    }
     // MFMA lane coordinates: lane = (gk, gi), gk = lane / 16, gi = lane % 16
     const int gi = lane & 15, gk = lane >> 4;
     for (int a = wi.ado0 + wv; a < aend; a += kThreads / 64) {
@@ -1078,7 +1117,12 @@ void heom_proj_kernel(StageParams p) {
         for (int r = 0; r < 4; ++r)
           if (Mfma<T>::row(gk, r) < d && gi < d) pr[r] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, Mfma<T>::row(gk, r), gi));
       }
-      if (a + kThreads / 64 < aend) prefetch(a + kThreads / 64);
+      if (a + kThreads / 64 < aend) {
+        prefetch(a + kThreads / 64);
+      } else if (ONE == 2 && it + itstep < itend) {
+        const WorkItem wn = one_item(p, it + itstep);
+        if (wv < wn.nado) prefetch(wn.ado0 + wv);
+      }
       // ---- commutator and damping (while the neighbour loads are in flight)
       if (MFMA) {
         typename Mfma<T>::acc aR[NT][NT], aI[NT][NT];
@@ -1389,6 +1433,19 @@ void heom_proj_kernel(StageParams p) {
       wave_sync();
     }
   }
+}
+
+template <typename T, typename TI, typename TO, int STAGE, bool MFMA, bool HERM, bool PACK, int NT, bool ONE = false>
+__global__ __launch_bounds__(kThreads, proj_waves(MFMA, std::is_same<T, float>::value, PACK, STAGE, NT))
+void heom_proj_kernel(StageParams p) {
+  proj_body<T, TI, TO, STAGE, MFMA, HERM, PACK, NT, ONE ? 1 : 0>(p);
+}
+
+// a single instance's class, a block running through several items
+template <typename T, typename TI, typename TO, int STAGE, bool MFMA, int NT>
+__global__ __launch_bounds__(kThreads, proj_waves(MFMA, std::is_same<T, float>::value, true, STAGE, NT))
+void heom_proj_loop_kernel(StageParams p) {
+  proj_body<T, TI, TO, STAGE, MFMA, true, true, NT, 2>(p);
 }
 
 // ------------------------------------------------------------------ block-cooperative wide kernel
@@ -2530,12 +2587,17 @@ std::complex<double> cz(const double* p, int i) { return std::complex<double>(p[
 void build_items(pyqed_heom_plan* P);
 
 void retile(pyqed_heom_plan* P, int64_t target, int blocks_per_cu) {
-  if (target <= 0)
+  const bool automatic = target <= 0;
+  if (automatic)
     target = std::min<int64_t>(8192, std::max<int64_t>(64, P->stream_elems / std::max<int64_t>(1, (int64_t)P->num_cu * 8)));
   P->tile_target = target;
   P->blocks_per_cu = std::max(1, std::min(blocks_per_cu, 32));
   for (int c = 0; c < kClasses; ++c) {
-    P->cls_target[c] = P->tile_target;
+    // the single-instance kernels pay nothing per item, so their items are as small as they get (one ADO per
+    // wavefront) and the tail of a launch is short.  Step in us with 1, 2, 4 and 8 ADOs per wavefront and item:
+    // 24 sites at depth 3 mixed 521, 566, 591, 806, FP64 1093, 1165, 1187, 1667; 14 sites at depth 4 mixed 229,
+    // 229, 255, 346; 16 sites at depth 3 mixed 75, 87, 138, 244
+    P->cls_target[c] = automatic && P->one_inst[c] >= 0 ? 1 : P->tile_target;
     P->cls_bpc[c] = P->blocks_per_cu;
   }
   build_items(P);
@@ -2876,17 +2938,16 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
   P->is_res = is_res;
   for (int i = 0; i < n_inst; ++i)
     if (is_res[i]) P->resident.push_back(i);
-  retile(P, 0, 8);
   for (int i = 0; i < n_inst; ++i)
     if (!is_res[i]) P->cls_state[P->inst[i].path] += (int64_t)P->inst[i].nmax * P->inst[i].dp;
   if (stream_lds_bytes(P, sizeof(double)) > (size_t)P->max_lds) {
     destroy_plan(P);
     return fail(PYQED_EUNSUPPORTED, "instance too large for the streamed kernel's LDS budget");
   }
-  // ---- projector classes with a single streamed instance: neighbour lists at a fixed stride, for the
-  // classes whose packed forms have a single-instance kernel (the VALU class and the wide class)
+  // ---- projector classes of a packed plan with a single streamed instance: neighbour lists at a fixed
+  // stride for the single-instance kernel
   std::vector<std::vector<int2>> entfix(kClasses);
-  for (int c = 1; c < kClasses && P->packed; c += 2) {
+  for (int c = 1; c < kClasses && P->packed; ++c) {
     int only = -1, count = 0;
     for (int i = 0; i < n_inst; ++i)
       if (!is_res[i] && P->inst[i].path == c) only = i, ++count;
@@ -2909,6 +2970,7 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
     P->one_inst[c] = only;
     P->fix_stride[c] = S;
   }
+  retile(P, 0, 8);
   // ---- upload
   int rc = 0;
   for (int c = 1; c < kClasses && rc == 0; ++c)
@@ -3133,19 +3195,26 @@ StageParams base_params(const pyqed_heom_plan* P) {
   return p;
 }
 
+// Raise the kernel's dynamic-LDS limit, only when a larger size is first needed, so launches that are being
+// captured into a graph make no attribute calls.
 template <typename Kern>
-int launch(Kern k, int grid, size_t lds, hipStream_t s, const StageParams& p, int threads = kThreads) {
-  // raise the kernel's dynamic-LDS limit only when a larger size is first needed, so launches that
-  // are being captured into a graph make no attribute calls
+int allow_lds(Kern k, size_t lds) {
   static std::mutex mu;
   static std::map<void*, size_t> limit;
+  std::lock_guard<std::mutex> g(mu);
+  size_t& cur = limit[kernel_ptr(k)];
+  if (lds > cur) {
+    PQA_HIP(hipFuncSetAttribute(kernel_ptr(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    cur = lds;
+  }
+  return PYQED_OK;
+}
+
+template <typename Kern>
+int launch(Kern k, int grid, size_t lds, hipStream_t s, const StageParams& p, int threads = kThreads) {
   if (lds > 65536) {
-    std::lock_guard<std::mutex> g(mu);
-    size_t& cur = limit[kernel_ptr(k)];
-    if (lds > cur) {
-      PQA_HIP(hipFuncSetAttribute(kernel_ptr(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      cur = lds;
-    }
+    const int rc = allow_lds(k, lds);
+    if (rc) return rc;
   }
   hipLaunchKernelGGL(k, dim3(grid), dim3(threads), lds, s, p);
   PQA_HIP(hipGetLastError());
@@ -3158,6 +3227,33 @@ int stream_grid(const pyqed_heom_plan* P, int c) {
   int most = 1;
   for (int x = 0; x < 8; ++x) most = std::max(most, P->xr[c][x + 1] - P->xr[c][x]);
   return 8 * std::min(most, std::max(1, (P->num_cu * P->cls_bpc[c] + 7) / 8));
+}
+
+// Blocks of 256 threads of a kernel that fit a CU at this much dynamic LDS.
+template <typename Kern>
+int resident_blocks(Kern k, size_t lds) {
+  static std::mutex mu;
+  static std::map<std::pair<void*, size_t>, int> known;
+  std::lock_guard<std::mutex> g(mu);
+  auto it = known.find({kernel_ptr(k), lds});
+  if (it != known.end()) return it->second;
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel_ptr(k), kThreads, lds) != hipSuccess || n < 1) n = 1;
+  return known[{kernel_ptr(k), lds}] = n;
+}
+
+// A single-instance launch: a block per item where all of them are resident at once (form 1), else as many
+// blocks as are resident, each running through items (form 2).
+template <typename K1, typename K2>
+int launch_single(K1 one_shot, K2 looping, const pyqed_heom_plan* P, int c, size_t lds, hipStream_t st, const StageParams& p) {
+  int most = 1;
+  for (int x = 0; x < 8; ++x) most = std::max(most, P->xr[c][x + 1] - P->xr[c][x]);
+  if (lds > 65536) {
+    const int rc = allow_lds(looping, lds);
+    if (rc) return rc;
+  }
+  const int room = std::max(1, P->num_cu * std::min(P->cls_bpc[c], resident_blocks(looping, lds)) / 8);
+  return most <= room ? launch(one_shot, 8 * most, lds, st, p) : launch(looping, 8 * room, lds, st, p);
 }
 
 // One RK4 stage over every streamed item class: generic kernel, projector kernel with VALU
@@ -3229,18 +3325,21 @@ int launch_stage_ti(pyqed_heom_plan* P, const StageParams& p0, hipStream_t st, i
       const size_t wlds = c == 3 ? proj_block_bytes(P->pd[3].d2pad, P->pd[3].Kmax, P->pd[3].Lmax, sizeof(float), true) +
                                        wide_ado_bytes(P->pd[3].d2pad, P->pd[3].rowbuf)
                                  : 0;
-      if (c == 2)
-        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 1>, grid, plds, st, p);
-      else if (c == 3 && F32 && (P->variant & 2) && wlds <= (size_t)P->max_lds)
+      if (c == 3 && F32 && (P->variant & 2) && wlds <= (size_t)P->max_lds)
         rc = launch(heom_wide_kernel<S>, grid, wlds, st, p);
-      else if (c == 3 && one)
-        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 2, true>, grid, plds, st, p);
-      else if (c == 3)
-        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 2>, grid, plds, st, p);
-      else if (F32 && one)
-        rc = launch(heom_proj_kernel<T, TI, T, S, false, true, true, 1, F32>, grid, plds, st, p);
-      else
+      else if (one)
+        rc = c == 1   ? launch_single(heom_proj_kernel<T, TI, T, S, false, true, true, 1, true>,
+                                      heom_proj_loop_kernel<T, TI, T, S, false, 1>, P, c, plds, st, p)
+             : c == 2 ? launch_single(heom_proj_kernel<T, TI, T, S, true, true, true, 1, true>,
+                                      heom_proj_loop_kernel<T, TI, T, S, true, 1>, P, c, plds, st, p)
+                      : launch_single(heom_proj_kernel<T, TI, T, S, true, true, true, 2, true>,
+                                      heom_proj_loop_kernel<T, TI, T, S, true, 2>, P, c, plds, st, p);
+      else if (c == 1)
         rc = launch(heom_proj_kernel<T, TI, T, S, false, true, true, 1>, grid, plds, st, p);
+      else if (c == 2)
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 1>, grid, plds, st, p);
+      else
+        rc = launch(heom_proj_kernel<T, TI, T, S, true, true, true, 2>, grid, plds, st, p);
     } else if (P->hermitian && c == 2 && F32 && (P->variant & 1) && pipe_lds_bytes(P, c) <= (size_t)P->max_lds) {
       rc = launch(heom_pipe_kernel<S>, grid, pipe_lds_bytes(P, c), st, p);
     } else if (P->hermitian) {

@@ -271,8 +271,8 @@ class HeomEngine:
         return dict(items=it.tolist(), elems=el.tolist())
 
     def class_single(self):
-        """Per kernel class: for classes 1 and 3 of a packed plan whose streamed work is one instance, its
-        index (class 1 in FP32 and class 3 then run the single-instance kernel), else -1."""
+        """Per kernel class: for classes 1 to 3 of a packed plan whose streamed work is one instance, its
+        index (the class then runs the single-instance kernel), else -1."""
         out = np.zeros(NCLASSES, np.int32)
         _lib.check(self.L.pyqed_heom_plan_class_single(self.plan, out.ctypes.data))
         return out.tolist()
