@@ -143,11 +143,11 @@ struct StageParams {
   int32_t d2max, qmax, Kmax, Lmax;
   int32_t d2pad;  // projector path: max d*(d+1), matrices in LDS with row stride d+1
   // right-hand-side evaluation (STAGE 4) with combinations, r = L x: xout = cbase + calpha r when
-  // cbase is set (else xout = r, when xout is set); cacc = (cinit ? 0 : cacc) + cbeta r when cacc is set
+  // cbase is set (else xout = r, when xout is set); cacc = (caccin or 0) + cbeta r when cacc is set
   const double2* cbase;
+  const double2* caccin;
   double2* cacc;
   double calpha, cbeta;
-  int32_t cinit;
   // projector classes with a single streamed instance (one_per > 0): its record is inst0 and item k of
   // the class holds ADOs [k one_per, min((k + 1) one_per, nmax)), so neither table is read; its
   // neighbour lists are read from ent_fix at fix_stride entries per ADO (the row pointers give only
@@ -373,6 +373,12 @@ __device__ __forceinline__ float2 ld_delta(const double2* q, const StateRef& s) 
 template <int STAGE, bool DELTA>
 __device__ __forceinline__ Pre<DELTA> rk4_prefetch(const StageParams& p, const StateRef& s) {
   Pre<DELTA> v;
+  if constexpr (STAGE == 4) {  // the combination's operands (full matrices: s.g is the element's index)
+    v.y = p.cbase ? p.cbase[s.g] : make_double2(0, 0);
+    const double2 a = p.caccin ? p.caccin[s.g] : make_double2(0, 0);
+    v.an.x = a.x, v.an.y = a.y;
+    return v;
+  }
   v.y = (STAGE <= 2 || (DELTA && STAGE == 3)) ? ld_state(p.y, s) : make_double2(0, 0);
   if constexpr (DELTA) {
     v.an = (STAGE >= 1 && STAGE <= 3) ? ld_delta(p.ynew, s) : make_float2(0.f, 0.f);
@@ -460,12 +466,13 @@ __device__ __forceinline__ void rk4_store(const StageParams& p, int64_t gx, int6
                                           int64_t tposT) {
   const double dt = p.dt;
   if (STAGE == 4) {
+    double2 b = v.y;
     if (p.cacc) {
-      const double2 a = p.cinit ? make_double2(0, 0) : p.cacc[gx];
-      p.cacc[gx] = make_double2(a.x + p.cbeta * rx, a.y + p.cbeta * ry);
+      const double2 a = make_double2((double)v.an.x + p.cbeta * rx, (double)v.an.y + p.cbeta * ry);
+      p.cacc[gx] = a;
+      if (p.cacc == p.cbase) b = a;  // one buffer for both: the base is the new accumulator
     }
     if (p.cbase) {
-      const double2 b = p.cbase[gx];
       ((double2*)p.xout)[gx] = make_double2(b.x + p.calpha * rx, b.y + p.calpha * ry);
     } else if (p.xout) {
       ((double2*)p.xout)[gx] = make_double2(rx, ry);
@@ -872,11 +879,13 @@ __device__ __forceinline__ void proj_body(const StageParams& p) {
   constexpr bool kDelta = std::is_same<TO, float>::value;  // mixed precision: FP32 RK4 increment
   constexpr bool kPM = kDelta && PACK;  // packed mixed run: two FP32 registers (rk4_upper_m)
   static_assert(NT == 1 || (NT == 2 && MFMA), "2 x 2 tiles are an MFMA form");
+  static_assert((PQA_MFMA_DMIN - 1) * (PQA_MFMA_DMIN - 1) <= 128, "VALU classes: two elements per lane");
 #ifndef PQA_WIDE_PF
 #define PQA_WIDE_PF 9  // own-matrix elements per lane the wide wave form prefetches (the rest load in place)
 #endif
   constexpr int kPF = NT == 1 ? 4 : PQA_WIDE_PF;  // own-matrix elements per lane prefetched (64 kPF)
-  constexpr int kQP = NT == 1 ? 3 : 9;  // packed upper elements per lane, d(d+1)/2 <= 64 kQP
+  // packed upper elements per lane, d(d+1)/2 <= 64 kQP (VALU classes have d <= 11: 2, also for full matrices)
+  constexpr int kQP = !MFMA ? 2 : NT == 1 ? 3 : 9;
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: ADO indices stay scalar
@@ -1111,7 +1120,14 @@ __device__ __forceinline__ void proj_body(const StageParams& p) {
           }
         }
       };
-      if (MFMA && PACK && !(kPM && STAGE == 0) && (PQA_PACK_HOIST == 1 || kDMA)) request_packed();
+      // VALU classes: behind the rows, so that they cost no round trip of their own (us per step before and after,
+      // FP64: 7 sites depth 4 35.0, 34.0; mixed: 9 sites depth 4 54.9, 53.0)
+      if (PACK && !(kPM && STAGE == 0) && (!MFMA || PQA_PACK_HOIST == 1 || kDMA)) request_packed();
+      if (!MFMA && !PACK) {
+#pragma unroll
+        for (int q = 0; q < kQP; ++q)
+          if (lane + 64 * q < d2) pr[q] = rk4_prefetch<STAGE, kDelta>(p, StateRef{I.off + base + lane + 64 * q, false});
+      }
       if (MFMA && NT == 1 && !PACK && PQA_RK4_HOIST == 2) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -1301,49 +1317,36 @@ __device__ __forceinline__ void proj_body(const StageParams& p) {
             }
           }
         } else {
-          for (int p0 = 0; p0 < np; p0 += 256) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int pk = p0 + lane + 64 * q;
-              if (pk < np) {
-                if constexpr (kPM) {
-                  pm[q] = rk4_prefetch_m<STAGE>(p, I.poff + (int64_t)a * I.dp + pk);
-                } else {
-                  pr[q] = rk4_prefetch<STAGE, kDelta>(p, StateRef{I.poff + (int64_t)a * I.dp + pk, false});
+          for (int q = 0; q < kQP; ++q) {
+            const int pk = lane + 64 * q;
+            if (pk < np) {
+              const int ij = sIJ[pk], i = ij >> 8, j = ij & 255;
+              cpx<T> c = mk<T>(0, 0);
+              // real H (H(t) too): the products with Im H are zeros, two FMAs instead of four (not in
+              // stage 0, whose form the second loop would take from 5 to 4 waves per SIMD)
+              if (STAGE >= 1 && (I.flags & F_REALH)) {
+                for (int kk = 0; kk < d; ++kk) {
+                  const T hik = sH[i * rs + kk].x, hkj = sH[kk * rs + j].x;
+                  const cpx<T> xkj = w.X[kk * rs + j], xik = w.X[i * rs + kk];
+                  c.x += hik * xkj.x - xik.x * hkj;
+                  c.y += hik * xkj.y - xik.y * hkj;
+                }
+              } else {
+                for (int kk = 0; kk < d; ++kk) {
+                  cmac(c, sH[i * rs + kk], w.X[kk * rs + j]);
+                  cmsub(c, w.X[i * rs + kk], sH[kk * rs + j]);
                 }
               }
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int pk = p0 + lane + 64 * q;
-              if (pk < np) {
-                const int ij = sIJ[pk], i = ij >> 8, j = ij & 255;
-                cpx<T> c = mk<T>(0, 0);
-                // real H (H(t) too): the products with Im H are zeros, two FMAs instead of four (not in
-                // stage 0, whose form the second loop would take from 5 to 4 waves per SIMD)
-                if (STAGE >= 1 && (I.flags & F_REALH)) {
-                  for (int kk = 0; kk < d; ++kk) {
-                    const T hik = sH[i * rs + kk].x, hkj = sH[kk * rs + j].x;
-                    const cpx<T> xkj = w.X[kk * rs + j], xik = w.X[i * rs + kk];
-                    c.x += hik * xkj.x - xik.x * hkj;
-                    c.y += hik * xkj.y - xik.y * hkj;
-                  }
-                } else {
-                  for (int kk = 0; kk < d; ++kk) {
-                    cmac(c, sH[i * rs + kk], w.X[kk * rs + j]);
-                    cmsub(c, w.X[i * rs + kk], sH[kk * rs + j]);
-                  }
-                }
-                cpx<T> o = mul_mi(c);
-                cmsub(o, damp, w.X[i * rs + j]);
-                neighbours(o, i, j);
-                const int64_t g = I.poff + (int64_t)a * I.dp + pk;
-                if constexpr (kPM) {
-                  if (STAGE <= 2) pm[q].y = y_from_input_m<STAGE>(w.X[i * rs + j], pm[q]);
-                  output(i, j, rk4_upper_m<STAGE>(p, g, (double)o.x, (double)o.y, pm[q]));
-                } else {
-                  output(i, j, rk4_upper<STAGE, kDelta>(p, g, (double)o.x, (double)o.y, pr[q]));
-                }
+              cpx<T> o = mul_mi(c);
+              cmsub(o, damp, w.X[i * rs + j]);
+              neighbours(o, i, j);
+              const int64_t g = I.poff + (int64_t)a * I.dp + pk;
+              if constexpr (kPM) {
+                if (STAGE <= 2) pm[q].y = y_from_input_m<STAGE>(w.X[i * rs + j], pm[q]);
+                output(i, j, rk4_upper_m<STAGE>(p, g, (double)o.x, (double)o.y, pm[q]));
+              } else {
+                output(i, j, rk4_upper<STAGE, kDelta>(p, g, (double)o.x, (double)o.y, pr[q]));
               }
             }
           }
@@ -1401,32 +1404,23 @@ __device__ __forceinline__ void proj_body(const StageParams& p) {
             }
           }
       } else {
-        // four elements per lane at a time: their RK4 operands are requested together
-        for (int e0 = 0; e0 < d2; e0 += 256) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int e = e0 + lane + 64 * q;
-            const int i = (int)(((uint32_t)e * dmag) >> 20);
-            if (e < d2) pr[q] = rk4_prefetch<STAGE, kDelta>(p, state_ref<PACK>(I, a, i, e - i * d));
-          }
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int e = e0 + lane + 64 * q;
-            if (e < d2) {
-              const int i = (int)(((uint32_t)e * dmag) >> 20), j = e - i * d;
-              cpx<T> c = mk<T>(0, 0);
-              for (int kk = 0; kk < d; ++kk) {
-                cmac(c, sH[i * rs + kk], w.X[kk * rs + j]);
-                cmsub(c, w.X[i * rs + kk], sH[kk * rs + j]);
-              }
-              cpx<T> o = mul_mi(c);
-              cmsub(o, damp, w.X[i * rs + j]);
-              for (int t = w.gs[i]; t < w.gs[i + 1]; ++t) cmac(o, w.cl[t], w.R[t * rs + j]);
-              for (int t = w.gs[j]; t < w.gs[j + 1]; ++t)
-                cmac(o, w.cr[t], HERM ? (i != j ? conjg(w.R[t * rs + i]) : w.R[t * rs + i]) : w.Cc[t * rs + i]);
-              rk4_store<TO, STAGE, PACK, kDelta>(p, I.off + base + e, I.off + base + j * d + i, state_ref<PACK>(I, a, i, j),
-                                         (double)o.x, (double)o.y, pr[q], xout, save_ado, tbase + e, tbase + j * d + i);
+        for (int q = 0; q < kQP; ++q) {
+          const int e = lane + 64 * q;
+          if (e < d2) {
+            const int i = (int)(((uint32_t)e * dmag) >> 20), j = e - i * d;
+            cpx<T> c = mk<T>(0, 0);
+            for (int kk = 0; kk < d; ++kk) {
+              cmac(c, sH[i * rs + kk], w.X[kk * rs + j]);
+              cmsub(c, w.X[i * rs + kk], sH[kk * rs + j]);
             }
+            cpx<T> o = mul_mi(c);
+            cmsub(o, damp, w.X[i * rs + j]);
+            for (int t = w.gs[i]; t < w.gs[i + 1]; ++t) cmac(o, w.cl[t], w.R[t * rs + j]);
+            for (int t = w.gs[j]; t < w.gs[j + 1]; ++t)
+              cmac(o, w.cr[t], HERM ? (i != j ? conjg(w.R[t * rs + i]) : w.R[t * rs + i]) : w.Cc[t * rs + i]);
+            rk4_store<TO, STAGE, PACK, kDelta>(p, I.off + base + e, I.off + base + j * d + i, state_ref<PACK>(I, a, i, j),
+                                       (double)o.x, (double)o.y, pr[q], xout, save_ado, tbase + e, tbase + j * d + i);
           }
         }
       }
@@ -3835,6 +3829,6 @@ extern "C" int pyqed_heom_rhs_combine(pyqed_heom_plan* P, const void* x, void* o
   p.calpha = alpha;
   p.cacc = (double2*)acc;
   p.cbeta = beta;
-  p.cinit = acc_init ? 1 : 0;
+  p.caccin = acc_init ? nullptr : p.cacc;
   return rhs_launch(P, p, col, stream);
 }
