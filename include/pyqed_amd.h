@@ -224,6 +224,18 @@ int pyqed_heom_plan_read_timing(pyqed_heom_plan* plan, double* ms, int64_t* laun
 int pyqed_heom_adjoint_work_bytes(const pyqed_heom_plan* plan, int64_t* bytes);
 int pyqed_heom_adjoint_contract(pyqed_heom_plan* plan, const void* const* x, const void* const* u, const double* w,
                                 void* G, void* work, int64_t work_bytes, void* stream);
+/* FP64 RK4 steps that keep their stage inputs (no counterpart in the reference; pyqed_heom_rhs's layout, n
+ * elements a state): X is device [4 nsteps + 1][n], X[0] the state on entry; states 4 s .. 4 s + 3 become the
+ * stage inputs of step s, and state 4 nsteps is the result.  The field is taken at steps step0, step0 + 1, ...,
+ * or, with reverse, at step0, step0 - 1, ... and with the times of a step reversed (the adjoint's order).
+ * acc: device scratch [n]. */
+int pyqed_heom_stage_run(pyqed_heom_plan* plan, void* X, void* acc, const double* field, int64_t step0, int64_t nsteps,
+                         double dt, int32_t reverse, void* stream);
+/* pyqed_heom_adjoint_contract for nsteps consecutive steps: X as pyqed_heom_stage_run leaves it on the forward
+ * plan, U as its reverse form leaves it on the adjoint plan over the same steps (the last step first); G is
+ * device complex double [nsteps][3][traj_stride], work >= nsteps * pyqed_heom_adjoint_work_bytes. */
+int pyqed_heom_adjoint_contract_steps(pyqed_heom_plan* plan, const void* X, const void* U, const double* w,
+                                      int64_t nsteps, void* G, void* work, int64_t work_bytes, void* stream);
 
 /* ------------------------------------------------------------------ Liouville-space RK4
  * Batched propagation of vec(rho) (row-major, length N = d*d) under

@@ -193,7 +193,7 @@ __host__ __device__ inline size_t lds_header_bytes(int d2max, int qmax, int Kmax
   return (o + 15) & ~size_t(15);
 }
 
-__device__ __forceinline__ int stage_col(int stage) { return stage == 0 ? 0 : (stage == 3 ? 2 : 1); }
+__host__ __device__ __forceinline__ int stage_col(int stage) { return stage == 0 ? 0 : (stage == 3 ? 2 : 1); }
 
 // Load H(t), Q(t) diagonals, per-mode coefficients and sqrt table of one instance into LDS.
 template <typename T>
@@ -3600,6 +3600,7 @@ struct AdjParams {
   double2* G;     // [3][traj_stride]
   int nitems, d2max;
   int64_t traj_stride;
+  int64_t x_step, u_step;  // several steps (grid y, and z of the reduction): elements from one to the next
 };
 
 constexpr int kAdjMaxEl = 4;  // elements per lane: I.grp >= d2 lanes per ADO for d2 <= 64, else 256 lanes
@@ -3607,6 +3608,8 @@ constexpr int kAdjMaxEl = 4;  // elements per lane: I.grp >= d2 lanes per ADO fo
 __global__ __launch_bounds__(kThreads) void heom_adjoint_contract_kernel(AdjParams q) {
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x;
+  const int64_t xo = blockIdx.y * q.x_step, uo = blockIdx.y * q.u_step;
+  q.part += (int64_t)blockIdx.y * q.nitems * 3 * q.d2max;
   for (int it = blockIdx.x; it < q.nitems; it += gridDim.x) {
     const WorkItem wi = q.items[it];
     const InstDev I = q.insts[wi.inst];
@@ -3630,8 +3633,8 @@ __global__ __launch_bounds__(kThreads) void heom_adjoint_contract_kernel(AdjPara
         if (act) {
           const int64_t base = I.off + (int64_t)a * d2;
           for (int e = le; e < d2; e += G) {
-            sx[e] = q.x[st][base + e];
-            su[e] = q.u[st][base + e];
+            sx[e] = q.x[st][xo + base + e];
+            su[e] = q.u[st][uo + base + e];
           }
         }
         __syncthreads();
@@ -3687,6 +3690,8 @@ constexpr int kRedVals = 4, kRedLanes = kThreads / kRedVals;
 __global__ __launch_bounds__(kThreads) void heom_adjoint_reduce_kernel(AdjParams q) {
   __shared__ double2 red[kRedLanes][kRedVals];
   const int i = blockIdx.y;
+  q.part += (int64_t)blockIdx.z * q.nitems * 3 * q.d2max;
+  q.G += (int64_t)blockIdx.z * 3 * q.traj_stride;
   const InstDev I = q.insts[i];
   const int2 r = q.inst_items[i];
   const int v = threadIdx.x % kRedVals, ln = threadIdx.x / kRedVals;
@@ -3739,25 +3744,20 @@ extern "C" int pyqed_heom_adjoint_work_bytes(const pyqed_heom_plan* P, int64_t* 
   return PYQED_OK;
 }
 
-extern "C" int pyqed_heom_adjoint_contract(pyqed_heom_plan* P, const void* const* x, const void* const* u,
-                                           const double* w, void* G, void* work, int64_t work_bytes, void* stream) {
-  if (!P || !x || !u || !w || !G || !work) return fail(PYQED_EINVAL, "heom_adjoint_contract: null argument");
+namespace {
+// Contraction of nsteps steps: q.x and q.u are the pointers of the first, x_step and u_step apart.
+int contract(pyqed_heom_plan* P, const char* who, AdjParams& q, const double* w, int64_t nsteps, void* G, void* work,
+             int64_t work_bytes, void* stream) {
   int64_t need = 0;
   pyqed_heom_adjoint_work_bytes(P, &need);
-  if (work_bytes < need)
-    return fail(PYQED_EINVAL, "heom_adjoint_contract: workspace of " + std::to_string(work_bytes) + " bytes < " +
-                                  std::to_string(need) + " needed");
+  if (work_bytes < need * nsteps)
+    return fail(PYQED_EINVAL, std::string(who) + ": workspace of " + std::to_string(work_bytes) + " bytes < " +
+                                  std::to_string(need * nsteps) + " needed");
   if (P->items.empty()) return PYQED_OK;
-  AdjParams q;
-  std::memset(&q, 0, sizeof(q));
   q.insts = P->d_inst;
   q.items = P->d_items;
   q.inst_items = P->d_inst_items;
-  for (int s = 0; s < 4; ++s) {
-    q.x[s] = (const double2*)x[s];
-    q.u[s] = (const double2*)u[s];
-    q.w[s] = w[s];
-  }
+  for (int s = 0; s < 4; ++s) q.w[s] = w[s];
   q.part = (double2*)work;
   q.G = (double2*)G;
   q.nitems = (int)P->items.size();
@@ -3765,13 +3765,43 @@ extern "C" int pyqed_heom_adjoint_contract(pyqed_heom_plan* P, const void* const
   q.traj_stride = P->traj_stride;
   const hipStream_t st = (hipStream_t)stream;
   const int grid = std::max(1, std::min(q.nitems, P->num_cu * 8));
-  hipLaunchKernelGGL(heom_adjoint_contract_kernel, dim3(grid), dim3(kThreads), adjoint_lds_bytes(P), st, q);
+  hipLaunchKernelGGL(heom_adjoint_contract_kernel, dim3(grid, (unsigned)nsteps), dim3(kThreads), adjoint_lds_bytes(P), st, q);
   PQA_HIP(hipGetLastError());
-  if (P->n_inst > 65535) return fail(PYQED_EINVAL, "heom_adjoint_contract: at most 65535 instances per plan");
+  if (P->n_inst > 65535) return fail(PYQED_EINVAL, std::string(who) + ": at most 65535 instances per plan");
   const unsigned nx = (unsigned)((3 * P->d2max + kRedVals - 1) / kRedVals);
-  hipLaunchKernelGGL(heom_adjoint_reduce_kernel, dim3(nx, P->n_inst), dim3(kThreads), 0, st, q);
+  hipLaunchKernelGGL(heom_adjoint_reduce_kernel, dim3(nx, P->n_inst, (unsigned)nsteps), dim3(kThreads), 0, st, q);
   PQA_HIP(hipGetLastError());
   return PYQED_OK;
+}
+}  // namespace
+
+extern "C" int pyqed_heom_adjoint_contract(pyqed_heom_plan* P, const void* const* x, const void* const* u,
+                                           const double* w, void* G, void* work, int64_t work_bytes, void* stream) {
+  if (!P || !x || !u || !w || !G || !work) return fail(PYQED_EINVAL, "heom_adjoint_contract: null argument");
+  AdjParams q;
+  std::memset(&q, 0, sizeof(q));
+  for (int s = 0; s < 4; ++s) {
+    q.x[s] = (const double2*)x[s];
+    q.u[s] = (const double2*)u[s];
+  }
+  return contract(P, "heom_adjoint_contract", q, w, 1, G, work, work_bytes, stream);
+}
+
+extern "C" int pyqed_heom_adjoint_contract_steps(pyqed_heom_plan* P, const void* X, const void* U, const double* w,
+                                                 int64_t nsteps, void* G, void* work, int64_t work_bytes, void* stream) {
+  if (!P || !X || !U || !w || !G || !work) return fail(PYQED_EINVAL, "heom_adjoint_contract_steps: null argument");
+  if (nsteps < 0 || nsteps > 65535) return fail(PYQED_EINVAL, "heom_adjoint_contract_steps: 0 to 65535 steps");
+  if (nsteps == 0) return PYQED_OK;
+  AdjParams q;
+  std::memset(&q, 0, sizeof(q));
+  const int64_t n = P->n_elems;
+  for (int s = 0; s < 4; ++s) {  // forward stage s pairs with adjoint stage 3 - s, which ran backwards in time
+    q.x[s] = (const double2*)X + s * n;
+    q.u[s] = (const double2*)U + (4 * (nsteps - 1) + 3 - s) * n;
+  }
+  q.x_step = 4 * n;
+  q.u_step = -4 * n;
+  return contract(P, "heom_adjoint_contract_steps", q, w, nsteps, G, work, work_bytes, stream);
 }
 
 namespace {
@@ -3831,4 +3861,35 @@ extern "C" int pyqed_heom_rhs_combine(pyqed_heom_plan* P, const void* x, void* o
   p.cbeta = beta;
   p.caccin = acc_init ? nullptr : p.cacc;
   return rhs_launch(P, p, col, stream);
+}
+
+// RK4 steps that keep their stage inputs: four launches per step, each forming its right-hand side, the next
+// stage input and the running sum of the step.  For the adjoint, whose stages and the contraction need them;
+// on small hierarchies, where a launch costs what it takes to start (about 7 us), a step was 19 launches with
+// copies, a recomputed forward step and the sum apart: a gradient over 60 steps of 680 ADOs of 7 x 7 took 9.1 ms
+// and takes 4.9, plans included.
+extern "C" int pyqed_heom_stage_run(pyqed_heom_plan* P, void* X, void* acc, const double* field, int64_t step0,
+                                    int64_t nsteps, double dt, int32_t reverse, void* stream) {
+  if (!P || !X || !acc) return fail(PYQED_EINVAL, "heom_stage_run: null argument");
+  if (step0 < 0 || nsteps < 0 || (reverse && nsteps > step0 + 1))
+    return fail(PYQED_EINVAL, "heom_stage_run: steps out of range");
+  StageParams p = base_params(P);
+  p.field = field;
+  double2* x = (double2*)X;
+  const int64_t n = P->n_elems;
+  for (int64_t s = 0; s < nsteps; ++s, x += 4 * n) {
+    p.step = reverse ? step0 - s : step0 + s;
+    for (int k = 0; k < 4; ++k) {
+      p.xin = x + k * n;
+      p.xout = x + (k + 1) * n;
+      p.cbase = k < 3 ? x : (const double2*)acc;
+      p.calpha = k < 2 ? dt / 2 : k == 2 ? dt : dt / 6;
+      p.caccin = k == 0 ? x : (const double2*)acc;
+      p.cacc = k < 3 ? (double2*)acc : nullptr;
+      p.cbeta = k == 0 ? dt / 6 : dt / 3;
+      const int rc = rhs_launch(P, p, reverse ? 2 - stage_col(k) : stage_col(k), stream);
+      if (rc) return rc;
+    }
+  }
+  return PYQED_OK;
 }

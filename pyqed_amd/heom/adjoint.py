@@ -21,8 +21,11 @@ accumulated per step and field column by pyqed_heom_adjoint_contract.  J is real
 dJ = Re sum conj(rhoT_bar) d rho(T) (rhoT_bar = dJ/dRe rho + i dJ/dIm rho; for J = Re Tr(O rho(T)),
 rhoT_bar = O^H).
 
-Checkpoints: the forward run keeps the state every `ckpt_every` steps; the backward sweep recomputes one
-segment of states at a time, so memory is (nt / ckpt_every + ckpt_every) states.
+Memory: where the stage inputs of all steps (4 nt states) fit `HeomAdjoint.keep_bytes`, the forward run keeps
+them and nothing is recomputed.  Beyond that the forward run keeps the state every `ckpt_every` steps and the
+backward sweep recomputes one segment at a time, the last one excepted: its stage inputs where 4 ckpt_every
+states fit (nt / ckpt_every + 4 ckpt_every states in all), else its states, with the stage inputs formed again
+step by step (nt / ckpt_every + ckpt_every states).
 """
 import ctypes as C
 
@@ -33,6 +36,11 @@ from .. import _lib
 
 class HeomAdjoint:
     """Forward run and streamed adjoint of one or more HEOM instances (HeomEngine instance dicts)."""
+
+    # Stage inputs kept for the backward sweep, 1.4% of a GPU's 288 GB.  A step costs 8 launches with all of them
+    # kept, 12 with a segment's, 16 and a copy with none: on 680 ADOs of 7 x 7, where a launch takes about 7 us
+    # whatever it does, and on large hierarchies, where it takes its bytes, the fewer the faster.
+    keep_bytes = 4 << 30
 
     def __init__(self, instances, dt, nt, *, ckpt_every=50):
         from .engine import HeomEngine
@@ -116,12 +124,41 @@ class HeomAdjoint:
         dev = fwd.device
         n = fwd.n_elems
         z = lambda: torch.zeros(n, dtype=torch.complex128, device=dev)  # noqa: E731
+        G = torch.zeros((max(nt, 1), 3, fwd.traj_stride), dtype=torch.complex128, device=dev)
+        w = (C.c_double * 4)(dt / 6, dt / 3, dt / 3, dt / 6)
+        stream = _lib.stream_ptr(torch)
+        fp = None if f is None else f.data_ptr()
+        # steps whose stage inputs are kept at a time (X), and of those the steps of an adjoint sweep (U)
+        state = 16 * n
+        seg = nt if 4 * nt * state <= self.keep_bytes else ck
+        X = None
+        if nt and 4 * seg * state <= self.keep_bytes:
+            try:
+                cb = min(seg, 32)
+                X = torch.empty((4 * min(seg, nt) + 1, n), dtype=torch.complex128, device=dev)
+                U = torch.empty((4 * cb + 1, n), dtype=torch.complex128, device=dev)
+                acc = torch.empty(n, dtype=torch.complex128, device=dev)
+                work = torch.empty(max(cb * self._wb, 16), dtype=torch.uint8, device=dev)
+            except torch.OutOfMemoryError:
+                X = U = acc = work = None
+                seg = ck
+
+        def stages(eng, buf, step, m, reverse):
+            _lib.check(self.L.pyqed_heom_stage_run(eng.plan, buf.data_ptr(), acc.data_ptr(), fp, step, m, dt, reverse, stream))
+
         # forward with checkpoints
         fwd.reset()
         ckpts = []
-        for c0 in range(0, nt, ck):
-            ckpts.append(fwd.y.clone())
-            fwd.advance(min(ck, nt - c0), dt, "fp64", field=f)
+        for c0 in range(0, nt, seg or 1):
+            m = min(seg, nt - c0)
+            if X is not None and c0 + m == nt:  # the segment that the backward sweep starts with
+                X[0].copy_(fwd.y)
+                stages(fwd, X, c0, m, 0)
+                ckpts.append(None)
+                fwd.y.copy_(X[4 * m])
+            else:
+                ckpts.append(fwd.y.clone())
+                fwd.advance(m, dt, "fp64", field=f)
         torch.cuda.synchronize()
         rhoT = fwd.reduced_states()
         # terminal cotangent: ADO 0 of every instance
@@ -133,14 +170,53 @@ class HeomAdjoint:
             o = int(fwd.state_offset[k])
             d = fwd.prep[k]["d"]
             lam[o:o + d * d] = torch.as_tensor(self._to_work(k, bar).reshape(-1), device=dev)
-        G = torch.zeros((max(nt, 1), 3, fwd.traj_stride), dtype=torch.complex128, device=dev)
-        Ys = torch.zeros((min(ck, max(nt, 1)), n), dtype=torch.complex128, device=dev)
+        if X is not None:
+            for i in reversed(range(len(ckpts))):
+                c0 = i * seg
+                m = min(seg, nt - c0)
+                if ckpts[i] is not None:
+                    X[0].copy_(ckpts[i])
+                    stages(fwd, X, c0, m, 0)
+                for j1 in range(m, 0, -cb):
+                    b = min(cb, j1)
+                    U[0].copy_(lam)
+                    stages(adj, U, c0 + j1 - 1, b, 1)
+                    lam = U[4 * b].clone()
+                    _lib.check(self.L.pyqed_heom_adjoint_contract_steps(
+                        adj.plan, X[4 * (j1 - b)].data_ptr(), U.data_ptr(), w, b, G[c0 + j1 - b].data_ptr(),
+                        work.data_ptr(), cb * self._wb, stream))
+        else:
+            self._sweep(ckpts, f, G, lam, w, stream)
+        torch.cuda.synchronize()
+        Gh = G.cpu().numpy()
+        lam_h = lam.cpu().numpy()
+        out = dict(rho=rhoT, J=J, gH=[], grho0=[], G=[], gfield=[])
+        for k in range(self.n):
+            p = fwd.prep[k]
+            d = p["d"]
+            to = int(fwd.traj_offset[k])
+            Gk = Gh[:nt, :, to:to + d * d].reshape(nt, 3, d, d)
+            Gtot = self._from_work(k, Gk.sum(axis=(0, 1)))
+            out["gH"].append(1j * Gtot.conj().T)
+            o = int(fwd.state_offset[k])
+            out["grho0"].append(self._from_work(k, lam_h[o:o + d * d].reshape(d, d)))
+            out["G"].append(Gk)
+            mu = p["sdip"]
+            out["gfield"].append(None if mu is None else np.real(-1j * np.einsum("ab,tcba->tc", mu, Gk)))
+        return out
+
+    def _sweep(self, ckpts, f, G, lam, w, stream):
+        """Backward sweep with one segment of states kept: lam is updated in place, G filled."""
+        torch = self.torch
+        fwd, adj = self.fwd, self.adj
+        dt, nt, ck = self.dt, self.nt, self.ckpt_every
+        n = fwd.n_elems
+        z = lambda: torch.zeros(n, dtype=torch.complex128, device=fwd.device)  # noqa: E731
+        Ys = torch.zeros((min(ck, max(nt, 1)), n), dtype=torch.complex128, device=fwd.device)
         x2, x3, x4 = z(), z(), z()
         X2, X3, X4, acc = z(), z(), z(), z()
-        w = (C.c_double * 4)(dt / 6, dt / 3, dt / 3, dt / 6)
         xp = (C.c_void_p * 4)()
         up = (C.c_void_p * 4)()
-        stream = _lib.stream_ptr(torch)
         for seg in reversed(range(len(ckpts))):
             c0 = seg * ck
             m = min(ck, nt - c0)
@@ -170,23 +246,6 @@ class HeomAdjoint:
                 _lib.check(self.L.pyqed_heom_adjoint_contract(adj.plan, xp, up, w, G[s].data_ptr(),
                                                               self._work.data_ptr(), self._wb, stream))
                 lam.add_(acc, alpha=dt / 6)
-        torch.cuda.synchronize()
-        Gh = G.cpu().numpy()
-        lam_h = lam.cpu().numpy()
-        out = dict(rho=rhoT, J=J, gH=[], grho0=[], G=[], gfield=[])
-        for k in range(self.n):
-            p = fwd.prep[k]
-            d = p["d"]
-            to = int(fwd.traj_offset[k])
-            Gk = Gh[:nt, :, to:to + d * d].reshape(nt, 3, d, d)
-            Gtot = self._from_work(k, Gk.sum(axis=(0, 1)))
-            out["gH"].append(1j * Gtot.conj().T)
-            o = int(fwd.state_offset[k])
-            out["grho0"].append(self._from_work(k, lam_h[o:o + d * d].reshape(d, d)))
-            out["G"].append(Gk)
-            mu = p["sdip"]
-            out["gfield"].append(None if mu is None else np.real(-1j * np.einsum("ab,tcba->tc", mu, Gk)))
-        return out
 
     def close(self):
         self.fwd.close()
