@@ -294,11 +294,13 @@ def kernel_name(stage, cls, precision, eng):
     mfma = "true" if cls >= 2 else "false"
     herm = "true" if eng.hermitian else "false"
     nt = 2 if cls == 3 else 1
-    # single-instance form: packed classes 1 to 3 when the class's streamed work is one instance; launches
-    # with more items than resident blocks (at most 8 on each of 256 CUs) loop over them
+    # packed classes whose streamed work is one instance: the lean kernel in class 1, else the single-instance
+    # form, whose launches with more items than resident blocks (at most 8 on each of 256 CUs) loop over them
     if eng.packed and eng.class_single()[cls] >= 0:
+        if cls == 1:
+            return f"heom_lean_kernel<{T}, {stage}, true>"
         if eng.classes()["items"][cls] > 8 * 256:
-            return f"heom_proj_loop_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {nt}>"
+            return f"heom_proj_loop_kernel<{T}, {TI}, {T}, {stage}, {nt}>"
         return f"heom_proj_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {herm}, {pack}, {nt}, true>"
     return f"heom_proj_kernel<{T}, {TI}, {T}, {stage}, {mfma}, {herm}, {pack}, {nt}, false>"
 

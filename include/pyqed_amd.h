@@ -195,9 +195,9 @@ int pyqed_heom_plan_set_variant(pyqed_heom_plan* plan, int32_t variant);
  * (host arrays [4], either may be NULL). */
 int pyqed_heom_plan_classes(const pyqed_heom_plan* plan, int64_t* items, int64_t* elems);
 /* Per kernel class (host array [4]): for classes 1 to 3 of a packed plan whose streamed work is a
- * single instance, that instance's index (the class then runs the single-instance kernel: instance
- * record from the kernel arguments, loaded once per block, neighbour lists at a fixed stride); -1
- * otherwise, and always for class 0.
+ * single instance, that instance's index (class 1 then runs the lean kernel, whatever its tiling,
+ * classes 2 and 3 the single-instance kernel: instance record from the kernel arguments, loaded once per
+ * block, neighbour lists at a fixed stride); -1 otherwise, and always for class 0.
  * No counterpart in the reference; used to name the kernels a benchmark's launches run. */
 int pyqed_heom_plan_class_single(const pyqed_heom_plan* plan, int32_t* inst);
 /* RK4-state elements (size in y) of the streamed work per kernel class (host array [4]): equal to

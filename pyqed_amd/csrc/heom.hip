@@ -111,6 +111,19 @@ __device__ __forceinline__ V ro_load(const V* q) {
 
 __device__ __forceinline__ int32_t ro_int(const int32_t* q, int64_t i) { return ((const PQA_CONST int32_t*)q)[i]; }
 
+// Tables of a site-projector hierarchy with d <= 11 that has its class to itself (heom_lean_kernel), made once
+// with the plan in the precision of the run.
+struct LeanTables {
+  const int2* ent;        // [nmax][stride]: entries in site order; x: neighbour * d + site, y: site << 16 | index of
+                          // the coefficient pair
+  const uint8_t* start;   // [nmax][16]: first entry of every site's group, and the number of entries at [d]
+  const void* damp;       // [nmax] complex: sum_k n_k gamma_k
+  const void* pair;       // per (exponential, n, sign): row and column coefficient times sqrt(n), complex
+  const int32_t* ij;      // packed plans: (i << 8) | j of every packed index
+  int32_t stride;
+  uint32_t dmag;          // floor(e / d) = (e dmag) >> 20 for e < 2^11
+};
+
 struct StageParams {
   const InstDev* insts;
   const WorkItem* items;
@@ -155,6 +168,7 @@ struct StageParams {
   InstDev inst0;
   int32_t one_per, fix_stride;
   const int2* ent_fix;
+  LeanTables lean;  // heom_lean_kernel
 };
 
 // LDS carve-up shared by both kernels.
@@ -871,9 +885,7 @@ constexpr int proj_waves(bool mfma, bool f32, bool pack, int stage, int nt) {
 // that the table-driven forms keep their registers.  1: a block has one item, as in launches whose blocks are
 // all resident at once; 2: a block runs through several items, loads the instance once and keeps its prefetch
 // going from item to item.  Measured per step, 16 sites at depth 3: FP64 120 us with form 1 and 110 with
-// form 2 (138 with a header per item of four ADOs per wavefront and all blocks launched), mixed 76 and 75 (86);
-// 7 sites at depth 4, one item per block: mixed 30.1 and 32.1 us (the second prefetch is code that every
-// launch fetches).
+// form 2 (138 with a header per item of four ADOs per wavefront and all blocks launched), mixed 76 and 75 (86).
 template <typename T, typename TI, typename TO, int STAGE, bool MFMA, bool HERM, bool PACK, int NT, int ONE>
 __device__ __forceinline__ void proj_body(const StageParams& p) {
   constexpr bool kDelta = std::is_same<TO, float>::value;  // mixed precision: FP32 RK4 increment
@@ -1436,10 +1448,10 @@ void heom_proj_kernel(StageParams p) {
 }
 
 // a single instance's class, a block running through several items
-template <typename T, typename TI, typename TO, int STAGE, bool MFMA, int NT>
-__global__ __launch_bounds__(kThreads, proj_waves(MFMA, std::is_same<T, float>::value, true, STAGE, NT))
+template <typename T, typename TI, typename TO, int STAGE, int NT>
+__global__ __launch_bounds__(kThreads, proj_waves(true, std::is_same<T, float>::value, true, STAGE, NT))
 void heom_proj_loop_kernel(StageParams p) {
-  proj_body<T, TI, TO, STAGE, MFMA, true, true, NT, 2>(p);
+  proj_body<T, TI, TO, STAGE, true, true, true, NT, 2>(p);
 }
 
 // ------------------------------------------------------------------ block-cooperative wide kernel
@@ -1943,6 +1955,228 @@ __global__ __launch_bounds__(kThreads, PQA_PIPE_WAVES) void heom_pipe_kernel(Sta
   }
 }
 
+// ------------------------------------------------------------------ small site-projector hierarchies
+// The VALU projector kernel for a hierarchy that has its class to itself: a wavefront per ADO, a block per four
+// ADOs.  Its launches are short chains of memory round trips and of instructions that are fetched anew in every
+// launch, so everything that does not change from launch to launch is in tables (site order, group starts,
+// damping, coefficient pairs, element indices), no table is loaded before the neighbour rows are requested but
+// the entries themselves, the waves meet once, for H, behind those requests, and results go to memory without a
+// tile in LDS.  The arithmetic of an element and its order are the projector kernel's.  us per step, projector
+// kernel and this one: 7 sites at depth 4 FP64 34.0, 28.1, mixed 29.6, 22.3; depth 3 FP64 26.0, 19.3 (of which
+// 13.6 are four empty launches); 11 sites at depth 4 FP64 155, 129, mixed 109, 80; 10 sites at depth 5 FP64 398,
+// 364, mixed 250, 160.  With the tile 1 to 3% more.  FP64 at depth 4 is bound by LDS reads, small ones by launches.
+constexpr int kLeanD = PQA_MFMA_DMIN - 1;
+constexpr int kLeanQ = 2;  // elements per lane, d d <= 64 kLeanQ
+static_assert(kLeanD * kLeanD <= 64 * kLeanQ && kLeanD < 16, "lean kernel: elements per lane, group starts");
+
+// Consecutive blocks that an XCD takes at a time.  Up to 4 blocks per CU, all resident at once, an eighth of them
+// each; beyond that runs of 16, because the ADOs of the last tier have half the neighbours of the others and
+// come last (us per step with eighths and with runs of 16: 10 sites at depth 5 FP64 421, 364; mixed 171, 160;
+// 11 sites at depth 4 FP64 152, 129).
+__host__ __device__ inline int lean_chunk(int nblk) { return nblk > 1024 ? 16 : (nblk + 7) / 8; }
+
+__host__ __device__ inline size_t lean_wave_bytes(int d, int stride, size_t ts, bool herm) {
+  const size_t el = (size_t)d * (d + 1) + (size_t)(herm ? 1 : 2) * stride * (d + 1) + 2 * (size_t)stride;
+  return (2 * ts * el + (herm ? 4 : 8) * (size_t)stride + 4 * 16 + 15) & ~size_t(15);
+}
+__host__ __device__ inline size_t lean_lds_bytes(int d, int stride, size_t ts, bool herm) {
+  return ((2 * ts * (size_t)d * (d + 1) + 15) & ~size_t(15)) + (kThreads / 64) * lean_wave_bytes(d, stride, ts, herm);
+}
+
+// PACK: packed Hermitian plans (stages 0-3); else non-Hermitian full-matrix plans (right-hand sides, STAGE 4)
+template <typename T, int STAGE, bool PACK>
+__global__ __launch_bounds__(kThreads) void heom_lean_kernel(StageParams p) {
+  static_assert(PACK ? STAGE < 4 : STAGE == 4 && std::is_same<T, double>::value, "lean kernel forms");
+  constexpr bool kDelta = std::is_same<T, float>::value;
+  constexpr bool kPM = kDelta && PACK;
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int d = p.inst0.d, d2 = p.inst0.d2, rs = d + 1, S = p.lean.stride;
+  const uint32_t dmag = p.lean.dmag;
+  // blocks of one XCD take runs of consecutive ADOs, whose neighbours they share in that XCD's L2
+  const int nblk = (p.inst0.nmax + kThreads / 64 - 1) / (kThreads / 64);
+  const int chunk = lean_chunk(nblk), bx = blockIdx.x >> 3;
+  const int blk = ((bx / chunk) * 8 + (blockIdx.x & 7)) * chunk + bx % chunk;
+  const int a = blk * (kThreads / 64) + wv;
+  const bool act = a < p.inst0.nmax;  // wave-uniform
+  cpx<T>* sH = (cpx<T>*)smem;
+  char* wb = smem + ((2 * sizeof(T) * (size_t)d * rs + 15) & ~size_t(15)) + wv * lean_wave_bytes(d, S, sizeof(T), PACK);
+  cpx<T>* X = (cpx<T>*)wb;
+  cpx<T>* R = X + d * rs;
+  cpx<T>* Cc = R + S * rs;  // non-Hermitian plans only
+  cpx<T>* cl = PACK ? Cc : Cc + S * rs;
+  cpx<T>* cr = cl + S;
+  int32_t* row = (int32_t*)(cr + S);  // neighbour * d + site
+  int32_t* cst = row + S;             // neighbour * d d + site (non-Hermitian plans)
+  int32_t* gs = PACK ? cst : cst + S;
+  const cpx_store<T>* xi = (const cpx_store<T>*)p.xin + p.inst0.off;
+  const int64_t base = (int64_t)a * d2;
+  const int ne = PACK ? (d * rs) >> 1 : d2;
+  // ---- first round trip
+  int2 en = make_int2(0, 0);
+  int start = 0, ijv[kLeanQ];
+  cpx_store<T> xv[kLeanQ];
+  cpx<T> damp = mk<T>(0, 0);
+  Pre<kDelta> pr[kLeanQ];
+  PreM pm[kLeanQ];
+  if (act) {
+    if (lane < S) en = p.lean.ent[(int64_t)a * S + lane];
+    if (lane <= d) start = p.lean.start[(int64_t)a * 16 + lane];
+    damp = ro_load((const cpx<T>*)p.lean.damp + a);
+#pragma unroll
+    for (int q = 0; q < kLeanQ; ++q) {
+      const int e = lane + 64 * q;
+      if (e < d2) xv[q] = xi[base + e];
+      if (e < ne) {
+        if (PACK) ijv[q] = p.lean.ij[e];
+        const int64_t g = PACK ? p.inst0.poff + (int64_t)a * p.inst0.dp + e : p.inst0.off + base + e;
+        if constexpr (kPM) pm[q] = rk4_prefetch_m<STAGE>(p, g);
+        else pr[q] = rk4_prefetch<STAGE, kDelta>(p, StateRef{g, false});
+      }
+    }
+  }
+  double2 h = make_double2(0, 0);
+  if (tid < d2) {
+    h = p.mat[p.inst0.h_off + tid];
+    if (p.inst0.flags & F_SDIP) {
+      const int col = p.col_override >= 0 ? p.col_override : stage_col(STAGE & 3);
+      const double fs = p.field ? ro_load(p.field + 6 * p.step + col) : 0.0;
+      const double2 m = p.mat[p.inst0.h_off + d2 + tid];
+      h.x += m.x * fs;
+      h.y += m.y * fs;
+    }
+  }
+  // ---- second round trip: row s (and, unless Hermitian, column s) of every neighbour, coefficient pairs
+  constexpr int kCh = PACK ? 3 : 2;  // values per lane in flight (rows, and as many of the columns)
+  const int nent = __builtin_amdgcn_readlane(start, d), nval = act ? nent * d : 0;
+  cpx_store<T> v[kCh], u[PACK ? 1 : kCh];
+  cpx<T> pl, pc;
+  auto issue = [&](int q0) {
+#pragma unroll
+    for (int q = 0; q < kCh; ++q) {
+      const int idx = q0 + lane + 64 * q;
+      if (idx < nval) {
+        const int t = (int)(((uint32_t)idx * dmag) >> 20), jj = idx - t * d;
+        v[q] = xi[(int64_t)row[t] * d + jj];
+        if constexpr (!PACK) u[q] = xi[(int64_t)cst[t] + jj * d];
+      }
+    }
+  };
+  auto stash = [&](int q0) {
+#pragma unroll
+    for (int q = 0; q < kCh; ++q) {
+      const int idx = q0 + lane + 64 * q;
+      if (idx < nval) {
+        const int o = idx + (int)(((uint32_t)idx * dmag) >> 20);  // row t starts at t (d + 1)
+        R[o] = mk<T>(v[q].x, v[q].y);
+        if constexpr (!PACK) Cc[o] = mk<T>(u[q].x, u[q].y);
+      }
+    }
+  };
+  if (act) {
+    if (lane < nent) {
+      row[lane] = en.x;
+      if (!PACK) cst[lane] = (en.x - (en.y >> 16)) * d + (en.y >> 16);
+    }
+    if (lane <= d) gs[lane] = start;
+    wave_sync();
+    issue(0);
+    if (lane < nent) {
+      const cpx<T>* c = (const cpx<T>*)p.lean.pair + 2 * (en.y & 0xffff);
+      pl = c[0];
+      pc = c[1];
+    }
+#pragma unroll
+    for (int q = 0; q < kLeanQ; ++q) {
+      const int e = lane + 64 * q;
+      if (e < d2) X[e + (int)(((uint32_t)e * dmag) >> 20)] = mk<T>(xv[q].x, xv[q].y);
+    }
+  }
+  if (tid < d2) sH[tid + (int)(((uint32_t)tid * dmag) >> 20)] = mk<T>((T)h.x, (T)h.y);
+  __syncthreads();
+  if (!act) return;
+  // ---- commutator and damping while the rows are in flight
+  cpx<T> o[kLeanQ];
+#pragma unroll
+  for (int q = 0; q < kLeanQ; ++q) {
+    const int e = lane + 64 * q;
+    if (e < ne) {
+      int i, j;
+      if (PACK) {
+        i = ijv[q] >> 8, j = ijv[q] & 255;
+      } else {
+        i = (int)(((uint32_t)e * dmag) >> 20), j = e - i * d;
+      }
+      cpx<T> c = mk<T>(0, 0);
+      if (PACK && STAGE >= 1 && (p.inst0.flags & F_REALH)) {
+        for (int k = 0; k < d; ++k) {
+          const T hik = sH[i * rs + k].x, hkj = sH[k * rs + j].x;
+          const cpx<T> xkj = X[k * rs + j], xik = X[i * rs + k];
+          c.x += hik * xkj.x - xik.x * hkj;
+          c.y += hik * xkj.y - xik.y * hkj;
+        }
+      } else {
+        for (int k = 0; k < d; ++k) {
+          cmac(c, sH[i * rs + k], X[k * rs + j]);
+          cmsub(c, X[i * rs + k], sH[k * rs + j]);
+        }
+      }
+      o[q] = mul_mi(c);
+      cmsub(o[q], damp, X[i * rs + j]);
+    }
+  }
+  if (lane < nent) {
+    cl[lane] = pl;
+    cr[lane] = pc;
+  }
+  stash(0);
+  for (int q0 = 64 * kCh; q0 < nval; q0 += 64 * kCh) {
+    issue(q0);
+    stash(q0);
+  }
+  wave_sync();
+  // ---- neighbour terms, RK4 update
+  const bool save = STAGE == 3 && a == 0 && p.traj && p.save_slot >= 0;
+  const int64_t tb = p.save_slot * p.traj_stride + p.inst0.traj_off;
+  cpx_store<T>* xo = (cpx_store<T>*)p.xout + p.inst0.off + base;
+#pragma unroll
+  for (int q = 0; q < kLeanQ; ++q) {
+    const int e = lane + 64 * q;
+    if (e < ne) {
+      int i, j;
+      if (PACK) {
+        i = ijv[q] >> 8, j = ijv[q] & 255;
+      } else {
+        i = (int)(((uint32_t)e * dmag) >> 20), j = e - i * d;
+      }
+      for (int t = gs[i]; t < gs[i + 1]; ++t) cmac(o[q], cl[t], R[t * rs + j]);
+      for (int t = gs[j]; t < gs[j + 1]; ++t)
+        cmac(o[q], cr[t], PACK ? (i != j ? conjg(R[t * rs + i]) : R[t * rs + i]) : Cc[t * rs + i]);
+      if constexpr (PACK) {
+        const int64_t g = p.inst0.poff + (int64_t)a * p.inst0.dp + e;
+        double2 r;
+        if constexpr (kPM) {
+          if (STAGE <= 2) pm[q].y = y_from_input_m<STAGE>(X[i * rs + j], pm[q]);
+          r = rk4_upper_m<STAGE>(p, g, (double)o[q].x, (double)o[q].y, pm[q]);
+        } else {
+          r = rk4_upper<STAGE, kDelta>(p, g, (double)o[q].x, (double)o[q].y, pr[q]);
+        }
+        st(xo + i * d + j, mk<T>((T)r.x, (T)r.y));
+        if (i != j) st(xo + j * d + i, mk<T>((T)r.x, (T)(-r.y)));
+        if (save) {
+          p.traj[tb + i * d + j] = r;
+          if (i != j) p.traj[tb + j * d + i] = make_double2(r.x, -r.y);
+        }
+      } else {
+        const int64_t g = p.inst0.off + base + e;
+        rk4_store<T, STAGE, PACK, kDelta>(p, g, g, StateRef{g, false}, (double)o[q].x, (double)o[q].y, pr[q],
+                                          (cpx_store<T>*)p.xout, false, 0, 0);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------ LDS-resident kernel
 // One workgroup owns one small instance for the whole run: y, ynew and both
 // stage buffers live in LDS, so HBM is touched only to load the initial state,
@@ -2417,6 +2651,10 @@ struct pyqed_heom_plan {
   int one_inst[kClasses] = {-1, -1, -1, -1};
   int fix_stride[kClasses] = {0, 0, 0, 0};
   int2* d_entfix[kClasses] = {nullptr, nullptr, nullptr, nullptr};
+  // the lean kernel's instance (or -1: class 1 runs the projector kernel) and tables
+  int lean_inst = -1;
+  LeanTables lean64 = {}, lean32 = {};
+  char* d_lean = nullptr;
   double2* d_coef = nullptr;
   int32_t* d_mode = nullptr;
   double2* d_mat = nullptr;
@@ -2502,6 +2740,84 @@ size_t pipe_lds_bytes(const pyqed_heom_plan* P, int c) {
   return proj_block_bytes(q.d2pad, q.Kmax, q.Lmax, sizeof(float), false) + (kThreads / 64) * pipe_wave_bytes(q.d2pad, q.rowbuf);
 }
 
+// Tables of the lean kernel for instance `only` (P->lean64, lean32 hold offsets into the returned buffer until it
+// is uploaded).  The damping is summed as the projector kernel's wavefront sums it, in the run's precision, and
+// the coefficient pairs are the products that it forms.  Empty where an index would not fit its field.
+std::vector<char> lean_tables(pyqed_heom_plan* P, int only, const int32_t* rowptr, const int2* ent, const int32_t* site,
+                              const double2* coefp) {
+  const InstDev& I = P->inst[only];
+  const int S = I.K + std::min(I.K, I.L), npair = I.K * (I.L + 2) * 2;
+  if (S > kMaxEnt || npair > 65536 || (int64_t)I.nmax * S * (int64_t)sizeof(int2) > (int64_t(1) << 28)) return {};
+  std::vector<char> buf;
+  auto part = [&](size_t bytes) {
+    const size_t o = (buf.size() + 255) & ~size_t(255);
+    buf.resize(o + bytes);
+    return o;
+  };
+  const size_t oe = part((size_t)I.nmax * S * sizeof(int2)), os = part((size_t)I.nmax * 16), oij = part(4 * 64 * kLeanQ);
+  const size_t od64 = part(16 * (size_t)I.nmax), od32 = part(8 * (size_t)I.nmax);
+  const size_t op64 = part(32 * (size_t)npair), op32 = part(16 * (size_t)npair);
+  int2* le = (int2*)(buf.data() + oe);
+  uint8_t* ls = (uint8_t*)(buf.data() + os);
+  double* d64 = (double*)(buf.data() + od64);
+  float* d32 = (float*)(buf.data() + od32);
+  for (int a = 0; a < I.nmax; ++a) {
+    const int2* e = ent + rowptr[a];
+    const int n = rowptr[a + 1] - rowptr[a];
+    if (n > S) return {};
+    uint8_t* first = ls + (size_t)a * 16;
+    int at[16] = {0};
+    for (int t = 0; t < n; ++t) ++at[site[e[t].y & 0xffff] + 1];
+    for (int s = 0; s < I.d; ++s) at[s + 1] += at[s];
+    for (int s = 0; s <= I.d; ++s) first[s] = (uint8_t)at[s];
+    double v64[2][kMaxEnt];
+    float v32[2][kMaxEnt];
+    for (int t = 0; t < n; ++t) {
+      const int k = e[t].y & 0xffff, nf = (e[t].y >> 16) & 0x7f, plus = e[t].y < 0, s = site[k];
+      // stable: entries of a site keep the table's order
+      le[(size_t)a * S + at[s]++] = make_int2(e[t].x * I.d + s, s << 16 | ((k * (I.L + 2) + nf) * 2 + plus));
+      const double2 g = plus ? make_double2(0, 0) : coefp[5 * k];
+      v64[0][t] = g.x * (double)nf, v64[1][t] = g.y * (double)nf;
+      v32[0][t] = (float)g.x * (float)nf, v32[1][t] = (float)g.y * (float)nf;
+    }
+    // the butterfly's tree without the terms past the list, which are zero
+    for (int o = 32, m = n; o > 0 && m > 1; o >>= 1) {
+      for (int t = 0; t + o < m; ++t)
+        for (int c = 0; c < 2; ++c) v64[c][t] += v64[c][t + o], v32[c][t] += v32[c][t + o];
+      m = std::min(m, o);
+    }
+    for (int c = 0; c < 2; ++c) {
+      d64[2 * (size_t)a + c] = n ? v64[c][0] : 0.0;
+      d32[2 * (size_t)a + c] = n ? v32[c][0] : 0.0f;
+    }
+  }
+  double* p64 = (double*)(buf.data() + op64);
+  float* p32 = (float*)(buf.data() + op32);
+  for (int k = 0; k < I.K; ++k)
+    for (int nf = 0; nf < I.L + 2; ++nf)
+      for (int plus = 0; plus < 2; ++plus)
+        for (int c = 0; c < 2; ++c) {  // row, column
+          const double2 v = coefp[5 * k + 1 + 2 * plus + c];
+          const double sq = std::sqrt((double)nf);
+          const size_t o = 2 * ((size_t)((k * (I.L + 2) + nf) * 2 + plus) * 2 + c);
+          p64[o] = v.x * sq, p64[o + 1] = v.y * sq;
+          p32[o] = (float)v.x * (float)sq, p32[o + 1] = (float)v.y * (float)sq;
+        }
+  int32_t* ij = (int32_t*)(buf.data() + oij);
+  for (int i = 0, q = 0; i < I.d; ++i)
+    for (int j = i; j < I.d; ++j) ij[q++] = i << 8 | j;
+  LeanTables t;
+  t.ent = (const int2*)oe, t.start = (const uint8_t*)os, t.ij = (const int32_t*)oij;
+  t.damp = (const void*)od64, t.pair = (const void*)op64;
+  t.stride = S;
+  t.dmag = (uint32_t)(((1 << 20) + I.d - 1) / I.d);
+  P->lean64 = t;
+  t.damp = (const void*)od32, t.pair = (const void*)op32;
+  P->lean32 = t;
+  P->lean_inst = only;
+  return buf;
+}
+
 // LDS of the resident kernel for an instance of n_el elements whose base operators and tables take
 // `extra` bytes (resident_extra_bytes): header, base operators, tables, state and stage buffers.
 size_t resident_lds_bytes(const pyqed_heom_plan* P, int64_t n_el, size_t extra, size_t tsize) {
@@ -2550,6 +2866,7 @@ void destroy_plan(pyqed_heom_plan* P) {
   (void)hipFree(P->d_rowptr);
   (void)hipFree(P->d_ent);
   for (int c = 0; c < kClasses; ++c) (void)hipFree(P->d_entfix[c]);
+  (void)hipFree(P->d_lean);
   (void)hipFree(P->d_coef);
   (void)hipFree(P->d_mode);
   (void)hipFree(P->d_mat);
@@ -2576,8 +2893,8 @@ std::complex<double> cz(const double* p, int i) { return std::complex<double>(p[
 // has at most L, so by element count alone the first XCD of a single hierarchy got all the long ADOs (24-site
 // chain at depth 3: 1.7 times the average work; step 623 -> 562 us mixed, 1415 -> 1204 us FP64; 14 sites at
 // depth 4 in FP64 685 -> 523 us).  Up to 4 items per CU all items are resident at once and the ranges are of
-// equal length: a longer range would only queue (7 sites at depth 4 in FP64: 36 us, 49 us by cost).  `blocks_per_cu` sets the
-// persistent grid of the streamed kernels.
+// equal length: a longer range would only queue (7 sites at depth 4 in FP64 on the
+// projector kernel: 36 us, 49 us by cost).  `blocks_per_cu` sets the persistent grid of the streamed kernels.
 void build_items(pyqed_heom_plan* P);
 
 void retile(pyqed_heom_plan* P, int64_t target, int blocks_per_cu) {
@@ -2949,6 +3266,10 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
     const InstDev& I = P->inst[only];
     const int S = I.K + std::min(I.K, I.L);  // entries per ADO at most (K plus, min(K, L) minus)
     if ((int64_t)I.nmax * S * (int64_t)sizeof(int2) > (int64_t(1) << 28)) continue;
+    if (c == 1) {  // the lean kernel, with tables of its own
+      P->one_inst[c] = only;
+      continue;
+    }
     std::vector<int2>& f = entfix[c];
     f.assign((size_t)I.nmax * S, make_int2(-1, 0));
     bool fits = true;
@@ -2964,11 +3285,27 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
     P->one_inst[c] = only;
     P->fix_stride[c] = S;
   }
+  std::vector<char> lean;
+  if (P->packed ? P->one_inst[1] >= 0 : !P->hermitian) {
+    int only = -1, count = 0;
+    for (int i = 0; i < n_inst; ++i)
+      if (!is_res[i] && P->inst[i].path == 1) only = i, ++count;
+    if (count == 1) lean = lean_tables(P, only, rowptr.data() + P->inst[only].rowptr_off, ent.data() + P->inst[only].ent_off,
+                                       sites.data() + P->inst[only].site_off, coefp.data() + P->inst[only].coefp_off);
+  }
   retile(P, 0, 8);
   // ---- upload
   int rc = 0;
   for (int c = 1; c < kClasses && rc == 0; ++c)
     if (!entfix[c].empty()) rc = upload(entfix[c], &P->d_entfix[c]);
+  if (!rc && !lean.empty() && !(rc = upload(lean, &P->d_lean)))
+    for (LeanTables* t : {&P->lean64, &P->lean32}) {  // offsets from the buffer's start until now
+      t->ent = (const int2*)(P->d_lean + (intptr_t)t->ent);
+      t->start = (const uint8_t*)(P->d_lean + (intptr_t)t->start);
+      t->damp = P->d_lean + (intptr_t)t->damp;
+      t->pair = P->d_lean + (intptr_t)t->pair;
+      t->ij = (const int32_t*)(P->d_lean + (intptr_t)t->ij);
+    }
   if (rc || (rc = upload(P->inst, &P->d_inst)) || (rc = upload_items(P)) ||
       (rc = upload(rowptr, &P->d_rowptr)) || (rc = upload(ent, &P->d_ent)) || (rc = upload(coef, &P->d_coef)) ||
       (rc = upload(mode, &P->d_mode)) || (rc = upload(mat, &P->d_mat)) || (rc = upload(P->resident, &P->d_res)) ||
@@ -3294,7 +3631,7 @@ int launch_stage_ti(pyqed_heom_plan* P, const StageParams& p0, hipStream_t st, i
       p.colbuf = P->pd[c].colbuf;
       p.Kmax = P->pd[c].Kmax;
       p.Lmax = P->pd[c].Lmax;
-      if (P->one_inst[c] >= 0) {  // the class's items are consecutive ADO ranges of one instance
+      if (c > 1 && P->one_inst[c] >= 0) {  // the class's items are consecutive ADO ranges of one instance
         one = true;
         p.inst0 = P->inst[P->one_inst[c]];
         p.one_per = P->items[P->cls_begin[c]].nado;
@@ -3307,13 +3644,23 @@ int launch_stage_ti(pyqed_heom_plan* P, const StageParams& p0, hipStream_t st, i
     p.use_xcd = 1;
     std::memcpy(p.xr, P->xr[c], sizeof(p.xr));
     const int grid = stream_grid(P, c);
-    int rc;
+    int rc = PYQED_OK;
     // the projector kernel keeps neighbour rows (and columns) in LDS; when they do not fit, the
     // generic kernel (which any instance can use) takes the class
     const size_t plds = c == 0 ? 0 : proj_lds_bytes(P, c, sizeof(T));
     LaunchTimer timer(P, st, S < 4 ? kClasses * S + c : -1);  // right-hand-side launches are not timed
     constexpr bool F32 = std::is_same<T, float>::value;
-    if (c == 0 || plds > (size_t)P->max_lds) {
+    constexpr bool kLeanForm = PACK ? S < 4 : S == 4 && !F32;
+    const bool lean = kLeanForm && c == 1 && P->lean_inst >= 0 && (PACK || !P->hermitian);
+    if (lean) {
+      if constexpr (kLeanForm) {
+        p.inst0 = P->inst[P->lean_inst];
+        p.lean = F32 ? P->lean32 : P->lean64;
+        const int nblk = (p.inst0.nmax + kThreads / 64 - 1) / (kThreads / 64), run = 8 * lean_chunk(nblk);
+        rc = launch(heom_lean_kernel<T, S, PACK>, run * ((nblk + run - 1) / run),
+                    lean_lds_bytes(p.inst0.d, p.lean.stride, sizeof(T), PACK), st, p);
+      }
+    } else if (c == 0 || plds > (size_t)P->max_lds) {
       rc = launch(heom_stage_kernel<T, TI, T, S, PACK>, grid, stream_lds_bytes(P, sizeof(T)), st, p);
     } else if constexpr (PACK) {  // packed plans are Hermitian
       const size_t wlds = c == 3 ? proj_block_bytes(P->pd[3].d2pad, P->pd[3].Kmax, P->pd[3].Lmax, sizeof(float), true) +
@@ -3322,12 +3669,10 @@ int launch_stage_ti(pyqed_heom_plan* P, const StageParams& p0, hipStream_t st, i
       if (c == 3 && F32 && (P->variant & 2) && wlds <= (size_t)P->max_lds)
         rc = launch(heom_wide_kernel<S>, grid, wlds, st, p);
       else if (one)
-        rc = c == 1   ? launch_single(heom_proj_kernel<T, TI, T, S, false, true, true, 1, true>,
-                                      heom_proj_loop_kernel<T, TI, T, S, false, 1>, P, c, plds, st, p)
-             : c == 2 ? launch_single(heom_proj_kernel<T, TI, T, S, true, true, true, 1, true>,
-                                      heom_proj_loop_kernel<T, TI, T, S, true, 1>, P, c, plds, st, p)
-                      : launch_single(heom_proj_kernel<T, TI, T, S, true, true, true, 2, true>,
-                                      heom_proj_loop_kernel<T, TI, T, S, true, 2>, P, c, plds, st, p);
+        rc = c == 2 ? launch_single(heom_proj_kernel<T, TI, T, S, true, true, true, 1, true>,
+                                    heom_proj_loop_kernel<T, TI, T, S, 1>, P, c, plds, st, p)
+                    : launch_single(heom_proj_kernel<T, TI, T, S, true, true, true, 2, true>,
+                                    heom_proj_loop_kernel<T, TI, T, S, 2>, P, c, plds, st, p);
       else if (c == 1)
         rc = launch(heom_proj_kernel<T, TI, T, S, false, true, true, 1>, grid, plds, st, p);
       else if (c == 2)

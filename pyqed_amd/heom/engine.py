@@ -272,7 +272,7 @@ class HeomEngine:
 
     def class_single(self):
         """Per kernel class: for classes 1 to 3 of a packed plan whose streamed work is one instance, its
-        index (the class then runs the single-instance kernel), else -1."""
+        index (class 1 then runs the lean kernel, 2 and 3 the single-instance kernel), else -1."""
         out = np.zeros(NCLASSES, np.int32)
         _lib.check(self.L.pyqed_heom_plan_class_single(self.plan, out.ctypes.data))
         return out.tolist()
