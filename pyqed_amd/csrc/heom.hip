@@ -56,6 +56,7 @@ using namespace pqa;
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kResThreads = 1024;  // resident instances of more than kThreads elements
 constexpr int kMaxD = 32;
 // Streamed work classes: 0 generic, 1 site projector with VALU commutator, 2 site projector with MFMA
 // commutator on one 16 x 16 tile (d <= 16), 3 the same on 2 x 2 tiles (17 <= d <= 32)
@@ -298,6 +299,35 @@ __device__ __forceinline__ cpx<T> element_rhs(const StageParams& p, const InstDe
   cpx<T> damp = mk<T>(0, 0);
   const int r0 = rowp[a], r1 = rowp[a + 1];
   const bool dense = (I.flags & F_DENSE) != 0;
+  if (!dense) {
+    // four entries at a time, their loads in flight together (us per step, 5 sites at depth 3: 45.5 one by one, 35.9)
+    constexpr int kE = 4;
+    for (int t0 = r0; t0 < r1; t0 += kE) {
+      int2 e4[kE];
+      cpx<T> cf[kE], v[kE];
+#pragma unroll
+      for (int u = 0; u < kE; ++u) e4[u] = ent[min(t0 + u, r1 - 1)];
+#pragma unroll
+      for (int u = 0; u < kE; ++u) {
+        cf[u] = mk<T>(0, 0);
+        if (t0 + u < r1) {
+          const int k = e4[u].y & 0xffff, nf = (e4[u].y >> 16) & 0x7f;
+          const bool plus = e4[u].y < 0;
+          const cpx<T>* C = l.C + 5 * k;
+          if (!plus) damp = damp + C[0] * (T)nf;
+          const cpx<T> cL = plus ? C[3] : C[1], cR = plus ? C[4] : C[2];
+          const int m = l.M[k];
+          cf[u] = (cL * l.Q[m * d + i] + cR * l.Q[m * d + j]) * l.S[nf];
+        }
+        if (cf[u].x != (T)0 || cf[u].y != (T)0) v[u] = ldc<T>(xin, (int64_t)e4[u].x * d2 + i * d + j);
+      }
+#pragma unroll
+      for (int u = 0; u < kE; ++u)
+        if (cf[u].x != (T)0 || cf[u].y != (T)0) cmac(r, cf[u], v[u]);
+    }
+    cmsub(r, damp, ldc<T>(own, i * d + j));
+    return r;
+  }
   for (int t = r0; t < r1; ++t) {
     const int2 en = ent[t];
     const int k = en.y & 0xffff;
@@ -310,29 +340,24 @@ __device__ __forceinline__ cpx<T> element_rhs(const StageParams& p, const InstDe
     const T sq = l.S[nf];
     const int m = l.M[k];
     const int64_t nb = (int64_t)en.x * d2;
-    if (!dense) {
-      cpx<T> coef = (cL * l.Q[m * d + i] + cR * l.Q[m * d + j]) * sq;
-      if (coef.x != (T)0 || coef.y != (T)0) cmac(r, coef, ldc<T>(xin, nb + i * d + j));
-    } else {
-      // dense coupling: cL (Q X)_{ij} + cR (X Q)_{ij}, Q read from the FP64 matrix pool
-      const double2* Qm = p.mat + I.q_off + (int64_t)m * d2;
-      const double2* Cm = (I.flags & F_CDIP) ? Qm + (int64_t)I.ncoup * d2 : nullptr;
-      cpx<T> s1 = mk<T>(0, 0), s2 = mk<T>(0, 0);
-      for (int q = 0; q < d; ++q) {
-        double2 qa = Qm[i * d + q], qb = Qm[q * d + j];
-        if (Cm) {
-          double2 ca = Cm[i * d + q], cb = Cm[q * d + j];
-          qa.x += ca.x * fc;
-          qa.y += ca.y * fc;
-          qb.x += cb.x * fc;
-          qb.y += cb.y * fc;
-        }
-        cmac(s1, mk<T>((T)qa.x, (T)qa.y), ldc<T>(xin, nb + q * d + j));
-        cmac(s2, ldc<T>(xin, nb + i * d + q), mk<T>((T)qb.x, (T)qb.y));
+    // dense coupling: cL (Q X)_{ij} + cR (X Q)_{ij}, Q read from the FP64 matrix pool
+    const double2* Qm = p.mat + I.q_off + (int64_t)m * d2;
+    const double2* Cm = (I.flags & F_CDIP) ? Qm + (int64_t)I.ncoup * d2 : nullptr;
+    cpx<T> s1 = mk<T>(0, 0), s2 = mk<T>(0, 0);
+    for (int q = 0; q < d; ++q) {
+      double2 qa = Qm[i * d + q], qb = Qm[q * d + j];
+      if (Cm) {
+        double2 ca = Cm[i * d + q], cb = Cm[q * d + j];
+        qa.x += ca.x * fc;
+        qa.y += ca.y * fc;
+        qb.x += cb.x * fc;
+        qb.y += cb.y * fc;
       }
-      cpx<T> v = cL * s1 + cR * s2;
-      r = r + v * sq;
+      cmac(s1, mk<T>((T)qa.x, (T)qa.y), ldc<T>(xin, nb + q * d + j));
+      cmac(s2, ldc<T>(xin, nb + i * d + q), mk<T>((T)qb.x, (T)qb.y));
     }
+    cpx<T> v = cL * s1 + cR * s2;
+    r = r + v * sq;
   }
   cmsub(r, damp, ldc<T>(own, i * d + j));
   return r;
@@ -2181,13 +2206,18 @@ __global__ __launch_bounds__(kThreads) void heom_lean_kernel(StageParams p) {
 // One workgroup owns one small instance for the whole run: y, ynew and both
 // stage buffers live in LDS, so HBM is touched only to load the initial state,
 // write trajectory samples and store the final state.
-template <typename T, bool PACK>
-__global__ __launch_bounds__(kThreads) void heom_resident_kernel(StageParams p) {
+// An element's right-hand side is a chain of dependent LDS reads, so instances of more elements than kThreads run
+// on kResThreads (NTH): us per step with 256 and 1024 threads, FP64 and mixed, 3 sites at depth 3 (756 elements)
+// 22.4, 12.0 and 17.4, 11.5; 5 sites at depth 2 (1650) 48.8, 20.4 and 38.1, 18.6.
+// Instances of up to kThreads elements keep one element per thread in registers (F_TINY), in that form only.
+template <typename T, bool PACK, int NTH>
+__global__ __launch_bounds__(NTH) void heom_resident_kernel(StageParams p) {
   extern __shared__ __align__(16) char smem[];
   const Lds<T> l = carve<T>(smem, p);
   const InstDev I = p.insts[p.resident[blockIdx.x]];
   const int n = I.nmax * I.d2, d2 = I.d2, d = I.d;
-  const int tid = threadIdx.x, nth = blockDim.x;
+  constexpr int nth = NTH;
+  const int tid = threadIdx.x;
   const double dt = p.dt;
   // ---- LDS: base operators (FP64), the instance's neighbour records, then the state and stage buffers
   const bool dense = (I.flags & F_DENSE) != 0, sd = (I.flags & F_SDIP) != 0, cd = (I.flags & F_CDIP) != 0;
@@ -2319,7 +2349,7 @@ __global__ __launch_bounds__(kThreads) void heom_resident_kernel(StageParams p) 
       for (int e = tid; e < d2; e += nth) p.traj[slot * p.traj_stride + I.traj_off + e] = make_double2(Y[e].x, Y[e].y);
     }
   };
-  if (I.flags & F_TINY) {
+  if (NTH == kThreads && (I.flags & F_TINY)) {
     // Tiny instances: thread e owns element e for the whole run.  Its indices, damping, the element
     // offsets of its neighbour entries and their coefficients sit in registers; d and the entry count
     // are bounded at compile time (D, E) and the four stages are unrolled, so a stage is one round of
@@ -2638,7 +2668,8 @@ struct pyqed_heom_plan {
   int cls_begin[kClasses + 1] = {0};  // class c occupies [cls_begin[c], cls_begin[c+1])
   int n_items_stream = 0;
   int xr[kClasses][9] = {{0}};
-  std::vector<int32_t> resident;
+  std::vector<int32_t> resident;  // instances of at most kThreads elements first
+  int n_res_small = 0;
   int64_t res_elems = 0, stream_elems = 0;
   int num_cu = 256, max_lds = 65536;
   // device copies
@@ -3249,6 +3280,9 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
   P->is_res = is_res;
   for (int i = 0; i < n_inst; ++i)
     if (is_res[i]) P->resident.push_back(i);
+  P->n_res_small = (int)(std::stable_partition(P->resident.begin(), P->resident.end(), [&](int i) {
+                           return (int64_t)P->inst[i].nmax * P->inst[i].d2 <= kThreads;
+                         }) - P->resident.begin());
   for (int i = 0; i < n_inst; ++i)
     if (!is_res[i]) P->cls_state[P->inst[i].path] += (int64_t)P->inst[i].nmax * P->inst[i].dp;
   if (stream_lds_bytes(P, sizeof(double)) > (size_t)P->max_lds) {
@@ -3853,13 +3887,26 @@ int run_typed(pyqed_heom_plan* P, double2* y, char* ws, const double* field, int
     r.step = step0;
     r.nsteps = nsteps;
     r.save_every = save_every;
-    size_t lds = 0;
-    for (int i : P->resident)
-      lds = std::max(lds, resident_lds_bytes(P, (int64_t)P->inst[i].nmax * P->inst[i].d2, P->res_extra[i], sizeof(T)));
-    // four waves per instance: an element's right-hand side is a chain of dependent LDS reads, so
-    // even small instances run faster with one element per lane than with one wave and cheaper barriers
-    int rc = P->packed ? launch(heom_resident_kernel<T, true>, (int)P->resident.size(), lds, P->side, r)
-                       : launch(heom_resident_kernel<T, false>, (int)P->resident.size(), lds, P->side, r);
+    // the list holds the instances of more than kThreads elements last; with as many of them as CUs the chip is
+    // full with kThreads each, and all run in one launch
+    const int nres = (int)P->resident.size(), nbig = nres - P->n_res_small;
+    const int cut = nbig <= P->num_cu ? P->n_res_small : nres;
+    auto lds_of = [&](int lo, int hi) {
+      size_t lds = 0;
+      for (int q = lo; q < hi; ++q) {
+        const int i = P->resident[q];
+        lds = std::max(lds, resident_lds_bytes(P, (int64_t)P->inst[i].nmax * P->inst[i].d2, P->res_extra[i], sizeof(T)));
+      }
+      return lds;
+    };
+    int rc = PYQED_OK;
+    if (cut > 0)
+      rc = P->packed ? launch(heom_resident_kernel<T, true, kThreads>, cut, lds_of(0, cut), P->side, r)
+                     : launch(heom_resident_kernel<T, false, kThreads>, cut, lds_of(0, cut), P->side, r);
+    r.resident += cut;
+    if (!rc && cut < nres)
+      rc = P->packed ? launch(heom_resident_kernel<T, true, kResThreads>, nres - cut, lds_of(cut, nres), P->side, r, kResThreads)
+                     : launch(heom_resident_kernel<T, false, kResThreads>, nres - cut, lds_of(cut, nres), P->side, r, kResThreads);
     if (rc) return rc;
     PQA_HIP(hipEventRecord(P->ev_join, P->side));
   }
