@@ -25,8 +25,8 @@ from .spectral import TIME, spectral_sum
 
 class LindbladSolver:
     """form (keyword only): "auto" runs d*d <= 1024 on the Liouville-space kernel (vec(rho) and its
-    generator in LDS) and larger d on the matrix-form kernel (pyqed_lindblad_run); "liouville" or
-    "matrix" force one of them."""
+    generator in LDS) and larger d on the matrix-form kernel (pyqed_lindblad_run), which also takes driven
+    Hermitian Hamiltonians from d = 8 on; "liouville" or "matrix" force one of them."""
 
     def __init__(self, H=None, c_ops=None, e_ops=None, *, form="auto"):
         if form not in ("auto", "liouville", "matrix"):
@@ -67,7 +67,16 @@ class LindbladSolver:
         else:
             H0 = np.asarray(self.H, np.complex128)
             drives = []
-        if self.form == "matrix" or (self.form == "auto" and d * d > 1024):
+        # A driven step has a generator of its own, so the Liouville-space kernel reads drives + 1 matrices of N x N,
+        # N = d d, in every stage; the matrix form works on d x d.  us per step with one drive, Liouville and matrix
+        # form, two collapse operators: d = 6 8 and 24, d = 8 30 and 24, d = 11 46 and 24, d = 16 222 and 27, d = 24
+        # 1470 and 37, d = 32 3740 and 37; with twelve (7 to 15 us each in matrix form): d = 11 48 and 95, d = 16
+        # 222 and 100, d = 17 281 and 174 (32 instances), d = 24 1460 and 77.  The matrix form's commutator is
+        # H rho - rho H^dagger, so H and the drives have to be Hermitian.
+        driven_matrix = (drives and Nt > 0 and len(rho0s) > 0 and d >= 8 and 24 * len(c_ops) <= d * d
+                         and all(np.shape(a) == (d, d) for a in [H0, *drives, *c_ops])
+                         and all(np.array_equal(h, dag(h)) for h in [H0, *drives]))
+        if self.form == "matrix" or (self.form == "auto" and (d * d > 1024 or driven_matrix)):
             return propagate_matrix(H0, c_ops, drives, rho0s, dt, Nt, field if drives else None, e_ops,
                                     keep_states=keep_states)
         gens = [lindblad_generator(H0, c_ops)] + [1j * op2sop(Hi) for Hi in drives]
