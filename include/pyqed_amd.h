@@ -315,6 +315,10 @@ int pyqed_liouville_adjoint(int32_t N, int32_t nterm, const void* A, int32_t n_i
                             const void* rhoT_bar, double* grad_field, void* grad_A, void* rho0_bar,
                             void* ckpt, int64_t ckpt_bytes, void* stream);
 
+/* rho_k <- V rho_k V^dagger for n matrices (device complex double [n][d][d], V [d][d], d <= 32): the states of a
+ * Redfield run from the eigenbasis to the caller's (oqs.py:57-81). */
+int pyqed_basis_change(int32_t d, int64_t n, const void* V, void* rho, void* stream);
+
 /* pyqed_liouville_adjoint with a workspace of pyqed_liouville_adjoint_work_bytes (at least the checkpoints that
  * pyqed_liouville_adjoint takes; work replaces ckpt).  For N <= 16 and few instances the sweep is cut along
  * time: the segments' propagators give every segment's first state and last adjoint state, then all segments

@@ -49,10 +49,17 @@ def run_workspace(torch, N, nterm, n_inst, nsteps, n_obs, keep_states, save_ever
         return None
 
 
-def propagate(gens, rho0s, dt, nsteps, field=None, e_ops=(), save_every=1, keep_states=True):
+def change_basis(torch, L, V, states):
+    """states (device, d x d matrices, d <= 32) <- V rho V^dagger in place."""
+    d = V.shape[0]
+    Vd = torch.as_tensor(np.ascontiguousarray(np.asarray(V, np.complex128)), device=states.device)
+    _lib.check(L.pyqed_basis_change(d, states.numel() // (d * d), Vd.data_ptr(), states.data_ptr(), _lib.stream_ptr(torch)))
+
+
+def propagate(gens, rho0s, dt, nsteps, field=None, e_ops=(), save_every=1, keep_states=True, basis=None):
     """Run pyqed_liouville_run.  gens: [nterm, N, N]; rho0s: [n_inst, d, d]; field: [n_inst, nsteps,
     nterm-1] or None.  Returns (observables [n_inst, nsteps+1, n_obs], states [n_inst, nsave, d, d],
-    final [n_inst, d, d]) as host arrays."""
+    final [n_inst, d, d]) as host arrays, the states as V rho V^dagger when basis = V is given (d <= 32)."""
     torch = _lib.require_gpu()
     L = _lib.lib()
     gens = np.ascontiguousarray(np.asarray(gens, np.complex128))
@@ -78,6 +85,8 @@ def propagate(gens, rho0s, dt, nsteps, field=None, e_ops=(), save_every=1, keep_
     _lib.check(L.pyqed_liouville_run_work(N, nterm, A.data_ptr(), n_inst, rho.data_ptr(), _lib.ptr(f), nsteps, float(dt),
                                           n_obs, _lib.ptr(obs), _lib.ptr(obs_out), _lib.ptr(rho_out), save_every,
                                           _lib.ptr(work), 0 if work is None else work.numel(), _lib.stream_ptr(torch)))
+    if nsave and basis is not None:
+        change_basis(torch, L, basis, rho_out)
     torch.cuda.synchronize()
     o = obs_out.cpu().numpy() if n_obs else np.zeros((n_inst, nsteps + 1, 0), complex)
     st = rho_out.cpu().numpy().reshape(n_inst, -1, d, d)[:, :nsave] if nsave else np.zeros((n_inst, 0, d, d), complex)
@@ -120,9 +129,10 @@ def redfield_operators(H, a_ops, spectra):
     return Heff, lefts, rights, evecs
 
 
-def run_matrix(Heff, lefts, rights, drives, rho0s, dt, nsteps, field=None, e_ops=(), save_every=1, keep_states=True):
+def run_matrix(Heff, lefts, rights, drives, rho0s, dt, nsteps, field=None, e_ops=(), save_every=1, keep_states=True,
+               basis=None):
     """pyqed_lindblad_run for d rho/dt = -i (Hs rho - rho Hs^dag) + sum_k lefts[k] rho rights[k],
-    Hs = Heff - sum_i f_i drives[i]."""
+    Hs = Heff - sum_i f_i drives[i]; returns as propagate."""
     torch = _lib.require_gpu()
     L = _lib.lib()
     Heff = np.asarray(Heff, np.complex128)
@@ -162,6 +172,8 @@ def run_matrix(Heff, lefts, rights, drives, rho0s, dt, nsteps, field=None, e_ops
                                     _lib.ptr(Hd), _lib.ptr(HdD), n_inst, rho.data_ptr(), _lib.ptr(f), nsteps, float(dt),
                                     n_obs, _lib.ptr(obs), _lib.ptr(obs_out), _lib.ptr(rho_out), save_every,
                                     work.data_ptr(), work.numel(), _lib.stream_ptr(torch)))
+    if nsave and basis is not None:
+        change_basis(torch, L, basis, rho_out)
     torch.cuda.synchronize()
     o = obs_out.cpu().numpy() if n_obs else np.zeros((n_inst, nsteps + 1, 0), complex)
     st = rho_out.cpu().numpy().reshape(n_inst, -1, d, d)[:, :nsave] if nsave else np.zeros((n_inst, 0, d, d), complex)

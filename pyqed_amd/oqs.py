@@ -312,17 +312,18 @@ class RedfieldSolver:
             Heff, lefts, rights, ev = redfield_operators(self.H, self.c_ops, self.spectra)
             self.evecs = ev
             e_eig = [dag(ev) @ np.asarray(e, np.complex128) @ ev for e in (e_ops or [])]
-            obs, states, _ = run_matrix(Heff, lefts, rights, (), (dag(ev) @ rho0 @ ev)[None], dt, Nt, None, e_eig)
+            obs, states, _ = run_matrix(Heff, lefts, rights, (), (dag(ev) @ rho0 @ ev)[None], dt, Nt, None, e_eig,
+                                       basis=ev if d <= 32 else None)
         else:
             if self.R is None:
                 self.redfield_tensor()
             ev = self.evecs
             e_eig = [dag(ev) @ np.asarray(e, np.complex128) @ ev for e in (e_ops or [])]
             obs, states, _ = propagate(np.asarray(self.R, np.complex128)[None], (dag(ev) @ rho0 @ ev)[None], dt, Nt,
-                                       None, e_eig)
+                                       None, e_eig, basis=ev)
         result = Result(dt=dt, Nt=Nt, rho0=rho0)
         result.observables = obs[0, 1:]
-        result.rholist = [ev @ states[0, k] @ dag(ev) for k in range(states.shape[1])]
+        result.rholist = list(states[0]) if d <= 32 else [ev @ r @ dag(ev) for r in states[0]]
         return result
 
 
