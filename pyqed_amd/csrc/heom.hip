@@ -2686,6 +2686,8 @@ struct pyqed_heom_plan {
   int lean_inst = -1;
   LeanTables lean64 = {}, lean32 = {};
   char* d_lean = nullptr;
+  char* d_arena = nullptr;  // the small tables (Arena)
+  size_t arena_bytes = 0;
   double2* d_coef = nullptr;
   int32_t* d_mode = nullptr;
   double2* d_mat = nullptr;
@@ -2736,6 +2738,50 @@ int upload(const std::vector<V>& h, V** d) {
   PQA_HIP(hipMalloc((void**)d, sizeof(V) * h.size()));
   PQA_HIP(hipMemcpy(*d, h.data(), sizeof(V) * h.size(), hipMemcpyHostToDevice));
   return PYQED_OK;
+}
+
+// The tables of a plan on their way to the device: those of up to kArenaTable bytes go into one allocation with one
+// copy (P->d_arena), larger ones each into their own, without a second copy on the host.  An allocation, its copy and
+// its release cost about 15 us each: an engine of a resident two-level hierarchy took 398 us to make and 141 to
+// close with a buffer per table and two streams, and takes 174 and 11; of 7 sites at depth 4 561 and 144, now 407
+// and 72.
+constexpr size_t kArenaTable = size_t(1) << 18;
+
+struct Arena {
+  std::vector<char> host;
+  std::vector<std::pair<void**, size_t>> at;  // pointer to set, offset (a page each, as allocations have)
+
+  template <typename V>
+  int add(const std::vector<V>& h, V** d) {
+    if (h.empty() || sizeof(V) * h.size() > kArenaTable) return upload(h, d);
+    const size_t o = (host.size() + 4095) & ~size_t(4095);
+    host.resize(o + sizeof(V) * h.size());
+    std::memcpy(host.data() + o, h.data(), sizeof(V) * h.size());
+    at.push_back({(void**)d, o});
+    return PYQED_OK;
+  }
+  int send(char** buf) {
+    const int rc = upload(host, buf);
+    if (!rc)
+      for (auto& a : at) *a.first = *buf + a.second;
+    return rc;
+  }
+};
+
+// The resident instances run beside the streamed ones on a stream of their own, alone on the caller's; the small
+// classes on their own stream when the other classes have work too.  Neither changes with the tiling.
+bool side_resident(const pyqed_heom_plan* P) { return !P->resident.empty() && P->n_items_stream > 0; }
+bool side_small(const pyqed_heom_plan* P) {
+  constexpr int cs = PQA_SIDE_CLASSES;
+  return P->cls_begin[cs] > P->cls_begin[0] && P->cls_begin[kClasses] > P->cls_begin[cs];
+}
+
+// Release a table unless it is part of the plan's arena.
+template <typename V>
+void release(const pyqed_heom_plan* P, V*& d) {
+  const char* q = (const char*)d;
+  if (d && !(P->d_arena && q >= P->d_arena && q < P->d_arena + P->arena_bytes)) (void)hipFree(d);
+  d = nullptr;
 }
 
 // Workspace of a run: ynew in the RK4 state layout (complex double), then the two stage buffers
@@ -2866,11 +2912,9 @@ size_t resident_extra_bytes(int d, int ncoup, bool dense, int nmax, int64_t nent
 
 // The work queue and, per instance, the range [first, last) of its items: tile() lists the items of one
 // instance consecutively.
-int upload_items(pyqed_heom_plan* P) {
-  (void)hipFree(P->d_items);
-  (void)hipFree(P->d_inst_items);
-  P->d_items = nullptr;
-  P->d_inst_items = nullptr;
+int upload_items(pyqed_heom_plan* P, Arena* arena = nullptr) {
+  release(P, P->d_items);
+  release(P, P->d_inst_items);
   std::vector<int2> rng(P->n_inst, make_int2(0, 0));
   std::vector<char> seen(P->n_inst, 0);
   for (int it = 0; it < (int)P->items.size(); ++it) {
@@ -2879,9 +2923,9 @@ int upload_items(pyqed_heom_plan* P) {
     seen[i] = 1;
     rng[i].y = it + 1;
   }
-  int rc = upload(P->items, &P->d_items);
+  int rc = arena ? arena->add(P->items, &P->d_items) : upload(P->items, &P->d_items);
   if (rc) return rc;
-  return upload(rng, &P->d_inst_items);
+  return arena ? arena->add(rng, &P->d_inst_items) : upload(rng, &P->d_inst_items);
 }
 
 int group_size(int d2) {
@@ -2892,19 +2936,20 @@ int group_size(int d2) {
 
 void destroy_plan(pyqed_heom_plan* P) {
   if (!P) return;
-  (void)hipFree(P->d_inst);
-  (void)hipFree(P->d_items);
-  (void)hipFree(P->d_rowptr);
-  (void)hipFree(P->d_ent);
-  for (int c = 0; c < kClasses; ++c) (void)hipFree(P->d_entfix[c]);
-  (void)hipFree(P->d_lean);
-  (void)hipFree(P->d_coef);
-  (void)hipFree(P->d_mode);
-  (void)hipFree(P->d_mat);
-  (void)hipFree(P->d_res);
-  (void)hipFree(P->d_site);
-  (void)hipFree(P->d_inst_items);
-  (void)hipFree(P->d_coefp);
+  release(P, P->d_inst);
+  release(P, P->d_items);
+  release(P, P->d_rowptr);
+  release(P, P->d_ent);
+  for (int c = 0; c < kClasses; ++c) release(P, P->d_entfix[c]);
+  release(P, P->d_lean);
+  release(P, P->d_coef);
+  release(P, P->d_mode);
+  release(P, P->d_mat);
+  release(P, P->d_res);
+  release(P, P->d_site);
+  release(P, P->d_inst_items);
+  release(P, P->d_coefp);
+  (void)hipFree(P->d_arena);
   if (P->side) (void)hipStreamDestroy(P->side);
   if (P->ev_fork) (void)hipEventDestroy(P->ev_fork);
   if (P->ev_join) (void)hipEventDestroy(P->ev_join);
@@ -3330,9 +3375,18 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
   retile(P, 0, 8);
   // ---- upload
   int rc = 0;
+  Arena arena;
   for (int c = 1; c < kClasses && rc == 0; ++c)
-    if (!entfix[c].empty()) rc = upload(entfix[c], &P->d_entfix[c]);
-  if (!rc && !lean.empty() && !(rc = upload(lean, &P->d_lean)))
+    if (!entfix[c].empty()) rc = arena.add(entfix[c], &P->d_entfix[c]);
+  if (rc || (rc = arena.add(lean, &P->d_lean)) || (rc = arena.add(P->inst, &P->d_inst)) || (rc = upload_items(P, &arena)) ||
+      (rc = arena.add(rowptr, &P->d_rowptr)) || (rc = arena.add(ent, &P->d_ent)) || (rc = arena.add(coef, &P->d_coef)) ||
+      (rc = arena.add(mode, &P->d_mode)) || (rc = arena.add(mat, &P->d_mat)) || (rc = arena.add(P->resident, &P->d_res)) ||
+      (rc = arena.add(sites, &P->d_site)) || (rc = arena.add(coefp, &P->d_coefp)) || (rc = arena.send(&P->d_arena))) {
+    destroy_plan(P);
+    return rc;
+  }
+  P->arena_bytes = arena.host.size();
+  if (!lean.empty())
     for (LeanTables* t : {&P->lean64, &P->lean32}) {  // offsets from the buffer's start until now
       t->ent = (const int2*)(P->d_lean + (intptr_t)t->ent);
       t->start = (const uint8_t*)(P->d_lean + (intptr_t)t->start);
@@ -3340,20 +3394,17 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
       t->pair = P->d_lean + (intptr_t)t->pair;
       t->ij = (const int32_t*)(P->d_lean + (intptr_t)t->ij);
     }
-  if (rc || (rc = upload(P->inst, &P->d_inst)) || (rc = upload_items(P)) ||
-      (rc = upload(rowptr, &P->d_rowptr)) || (rc = upload(ent, &P->d_ent)) || (rc = upload(coef, &P->d_coef)) ||
-      (rc = upload(mode, &P->d_mode)) || (rc = upload(mat, &P->d_mat)) || (rc = upload(P->resident, &P->d_res)) ||
-      (rc = upload(sites, &P->d_site)) ||
-      (rc = upload(coefp, &P->d_coefp))) {
-    destroy_plan(P);
-    return rc;
-  }
-  if (hipStreamCreateWithFlags(&P->side, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&P->ev_fork, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&P->ev_join, hipEventDisableTiming) != hipSuccess ||
-      hipStreamCreateWithFlags(&P->side0, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&P->ev_fork0, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&P->ev_join0, hipEventDisableTiming) != hipSuccess) {
+  // The streams that run_typed uses.  Packed plans with streamed work have both also where they use neither: their
+  // chains of launches are 1% faster beside two idle streams (us per step: 7 sites at depth 4 FP64 28.4 without, 28.1
+  // with; 16 sites at depth 3 114.1, 113.2), and such plans run many steps; the others save 160 us a plan.
+  const auto stream = [](hipStream_t* s, hipEvent_t* fork, hipEvent_t* join) {
+    return hipStreamCreateWithFlags(s, hipStreamNonBlocking) == hipSuccess &&
+           hipEventCreateWithFlags(fork, hipEventDisableTiming) == hipSuccess &&
+           hipEventCreateWithFlags(join, hipEventDisableTiming) == hipSuccess;
+  };
+  const bool chains = P->packed && P->n_items_stream > 0;
+  if (((chains || side_resident(P)) && !stream(&P->side, &P->ev_fork, &P->ev_join)) ||
+      ((chains || side_small(P)) && !stream(&P->side0, &P->ev_fork0, &P->ev_join0))) {
     destroy_plan(P);
     return fail(PYQED_EHIP, "stream/event creation failed");
   }
@@ -3880,9 +3931,13 @@ int run_typed(pyqed_heom_plan* P, double2* y, char* ws, const double* field, int
   p.nstate = P->n_state;
   p.traj = traj;
   p.field = field;
+  const bool beside = side_resident(P);
   if (!P->resident.empty()) {
-    PQA_HIP(hipEventRecord(P->ev_fork, st));
-    PQA_HIP(hipStreamWaitEvent(P->side, P->ev_fork, 0));
+    const hipStream_t rst = beside ? P->side : st;
+    if (beside) {
+      PQA_HIP(hipEventRecord(P->ev_fork, st));
+      PQA_HIP(hipStreamWaitEvent(P->side, P->ev_fork, 0));
+    }
     StageParams r = p;
     r.step = step0;
     r.nsteps = nsteps;
@@ -3901,14 +3956,14 @@ int run_typed(pyqed_heom_plan* P, double2* y, char* ws, const double* field, int
     };
     int rc = PYQED_OK;
     if (cut > 0)
-      rc = P->packed ? launch(heom_resident_kernel<T, true, kThreads>, cut, lds_of(0, cut), P->side, r)
-                     : launch(heom_resident_kernel<T, false, kThreads>, cut, lds_of(0, cut), P->side, r);
+      rc = P->packed ? launch(heom_resident_kernel<T, true, kThreads>, cut, lds_of(0, cut), rst, r)
+                     : launch(heom_resident_kernel<T, false, kThreads>, cut, lds_of(0, cut), rst, r);
     r.resident += cut;
     if (!rc && cut < nres)
-      rc = P->packed ? launch(heom_resident_kernel<T, true, kResThreads>, nres - cut, lds_of(cut, nres), P->side, r, kResThreads)
-                     : launch(heom_resident_kernel<T, false, kResThreads>, nres - cut, lds_of(cut, nres), P->side, r, kResThreads);
+      rc = P->packed ? launch(heom_resident_kernel<T, true, kResThreads>, nres - cut, lds_of(cut, nres), rst, r, kResThreads)
+                     : launch(heom_resident_kernel<T, false, kResThreads>, nres - cut, lds_of(cut, nres), rst, r, kResThreads);
     if (rc) return rc;
-    PQA_HIP(hipEventRecord(P->ev_join, P->side));
+    if (beside) PQA_HIP(hipEventRecord(P->ev_join, P->side));
   }
   if (P->n_items_stream > 0) {
     // packed mode: stage 0 reads x1, the full-matrix copy of y that stage 3 leaves there
@@ -3920,9 +3975,8 @@ int run_typed(pyqed_heom_plan* P, double2* y, char* ws, const double* field, int
       const int rc = launch(heom_unpack_kernel<T>, std::max(1, std::min(P->n_items_stream, P->num_cu * 8)), 0, st, u);
       if (rc) return rc;
     }
-    // the small classes on their own stream when the other classes have work too
     constexpr int cs = PQA_SIDE_CLASSES;
-    const bool split = P->cls_begin[cs] > P->cls_begin[0] && P->cls_begin[kClasses] > P->cls_begin[cs];
+    const bool split = side_small(P);
     if (split) {
       PQA_HIP(hipEventRecord(P->ev_fork0, st));
       PQA_HIP(hipStreamWaitEvent(P->side0, P->ev_fork0, 0));
@@ -3944,7 +3998,7 @@ int run_typed(pyqed_heom_plan* P, double2* y, char* ws, const double* field, int
       PQA_HIP(hipStreamWaitEvent(st, P->ev_join0, 0));
     }
   }
-  if (!P->resident.empty()) PQA_HIP(hipStreamWaitEvent(st, P->ev_join, 0));
+  if (beside) PQA_HIP(hipStreamWaitEvent(st, P->ev_join, 0));
   return PYQED_OK;
 }
 
