@@ -2791,7 +2791,7 @@ int64_t ws_state_bytes(const pyqed_heom_plan* P) { return ((P->n_state * 16 + 25
 // of its dense generator (power_run): elements of that generator's vector, 0 for other plans.
 constexpr int kPowerMax = 640;
 int power_size(const pyqed_heom_plan* P) {
-  return P->n_inst == 1 && !P->resident.empty() && P->n_elems <= kPowerMax ? (int)P->n_elems : 0;
+  return power_vector && P->n_inst == 1 && !P->resident.empty() && P->n_elems <= kPowerMax ? (int)P->n_elems : 0;
 }
 int64_t workspace_bytes(const pyqed_heom_plan* P, size_t xsize) {
   const int64_t stream = ws_state_bytes(P) + 2 * P->n_elems * (int64_t)xsize;

@@ -45,9 +45,11 @@ int small_adjoint(const LiouvilleRun& r, hipStream_t st);
 int small_adjoint_split(const LiouvilleRun& r, void* work, hipStream_t st);
 
 // dv/dt = A v for one vector of N <= 1024 elements by powers of the RK4 step matrix (propagator.hip): nsteps
-// steps in place; every `every` steps the first n_out elements go to out + slot out_stride (out may be NULL).
-int64_t power_vector_bytes(int N);
-int power_vector(int N, const double2* A, double2* v, int64_t nsteps, double dt, double2* out, int n_out, int64_t out_stride,
-                 int64_t every, void* work, hipStream_t st);
+// steps in place, kRowSeg rows at a time; every `every` steps the first n_out elements go to out + slot out_stride
+// (out may be NULL).  Weak: a program linked without propagator.hip has no such runs (power_size).
+constexpr int64_t kRowSeg = 1024;
+inline int64_t power_vector_bytes(int N) { return 16 * ((int64_t)(3 + 7) * N * N + kRowSeg * N); }
+__attribute__((weak)) int power_vector(int N, const double2* A, double2* v, int64_t nsteps, double dt, double2* out, int n_out,
+                                       int64_t out_stride, int64_t every, void* work, hipStream_t st);
 
 }  // namespace pqa

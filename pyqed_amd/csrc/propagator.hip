@@ -389,9 +389,6 @@ int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps,
   return PYQED_OK;
 }
 
-// One vector of N <= 1024 elements by powers of its step matrix, kRowSeg rows at a time.
-constexpr int64_t kRowSeg = 1024;
-
 // rho_k <- V rho_k V^dagger for a run of d x d matrices: a block per matrix, the three factors in LDS.  Bound by
 // the states' own bytes; the caller's copy of them to the host is longer (400 states of 16 x 16, 1.6 MB: on the host
 // the two products took 1.2 ms of a 1.7 ms call, here 6 us).
@@ -432,8 +429,6 @@ __global__ __launch_bounds__(kBasisThreads) void basis_change_kernel(int d, int6
 }  // namespace
 
 namespace pqa {
-
-int64_t power_vector_bytes(int N) { return 16 * ((int64_t)(3 + 7) * N * N + kRowSeg * N); }
 
 int power_vector(int N, const double2* A, double2* v, int64_t nsteps, double dt, double2* out, int n_out, int64_t out_stride,
                  int64_t every, void* work, hipStream_t st) {
