@@ -48,7 +48,9 @@ int small_adjoint_split(const LiouvilleRun& r, void* work, hipStream_t st);
 // steps in place, kRowSeg rows at a time; every `every` steps the first n_out elements go to out + slot out_stride
 // (out may be NULL).  Weak: a program linked without propagator.hip has no such runs (power_size).
 constexpr int64_t kRowSeg = 1024;
-inline int64_t power_vector_bytes(int N) { return 16 * ((int64_t)(3 + 7) * N * N + kRowSeg * N); }
+// complex elements of the matrices: seven and the powers
+inline int64_t power_matrix_elems(int N, int levels) { return (int64_t)(7 + levels) * N * N; }
+inline int64_t power_vector_bytes(int N) { return 16 * (power_matrix_elems(N, 7) + kRowSeg * N); }
 __attribute__((weak)) int power_vector(int N, const double2* A, double2* v, int64_t nsteps, double dt, double2* out, int n_out,
                                        int64_t out_stride, int64_t every, void* work, hipStream_t st);
 
