@@ -2793,6 +2793,10 @@ constexpr int kPowerMax = 640;
 int power_size(const pyqed_heom_plan* P) {
   return power_vector && P->n_inst == 1 && !P->resident.empty() && P->n_elems <= kPowerMax ? (int)P->n_elems : 0;
 }
+// Steps from which a call takes powers.  Forming them costs as N^3, a step of the resident kernel 2 us up to N = 256 and
+// 8 to 9 us beyond.  us per call of 63 steps by the resident kernel and of 64 by powers: N = 84 178 and 107, 144 188 and
+// 135, 252 219 and 189, 324 555 and 337, 336 572 and 346, 448 573 and 749, 576 634 and 1288 (1298 for 150 steps).
+int64_t power_steps(int N) { return std::max<int64_t>(64, (int64_t)N * N / 2400); }
 int64_t workspace_bytes(const pyqed_heom_plan* P, size_t xsize) {
   const int64_t stream = ws_state_bytes(P) + 2 * P->n_elems * (int64_t)xsize;
   const int64_t N = xsize == sizeof(double2) ? power_size(P) : 0;
@@ -3893,7 +3897,7 @@ __global__ __launch_bounds__(kThreads) void heom_repack_kernel(StageParams p, co
 // A small hierarchy alone in its plan, without fields: the whole hierarchy is a vector of N <= kPowerMax
 // elements under a constant generator, so its steps are rows of matrix products (propagator.hip) instead of a
 // chain of four LDS rounds per step.  Spin-boson at depth 5 (N = 84), 1000 steps in FP64: 2430 us by the
-// resident kernel, 130 us in 30 launches here (launch latency: N = 84 has 36 tiles).
+// resident kernel, 150 us in 30 launches here (launch latency: N = 84 has 36 tiles).
 int power_run(pyqed_heom_plan* P, double2* y, char* ws, int64_t nsteps, double dt, double2* traj, int64_t save_every, hipStream_t st) {
   const int N = power_size(P);
   const InstDev& I = P->inst[0];
@@ -4018,8 +4022,7 @@ extern "C" int pyqed_heom_run(pyqed_heom_plan* P, int32_t precision, void* y, vo
                                   std::to_string(need) + " bytes)");
   if (nsteps == 0) return PYQED_OK;
   hipStream_t st = (hipStream_t)stream;
-  // forming the powers takes as long as about 40 steps of the resident kernel
-  if (precision == PYQED_PREC_FP64 && !field && nsteps >= 64 && power_size(P))
+  if (precision == PYQED_PREC_FP64 && !field && power_size(P) && nsteps >= power_steps(power_size(P)))
     return power_run(P, (double2*)y, (char*)workspace, nsteps, dt, (double2*)traj, save_every, st);
   if (precision == PYQED_PREC_FP64)
     return run_typed<double>(P, (double2*)y, (char*)workspace, field, step0, nsteps, dt, (double2*)traj, save_every,
