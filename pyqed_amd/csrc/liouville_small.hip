@@ -29,6 +29,7 @@ namespace pqa {
 namespace {
 
 constexpr int kWin = 64;  // values of a group's field window in LDS
+constexpr double kTame = 1e150, kHold = 0x1p1000;
 
 typedef cpx<double> Z;
 
@@ -229,6 +230,12 @@ __global__ __launch_bounds__(64) void small_forward_kernel(SmParams p) {
   const int N = p.r.N, col = COLS ? (int)(q.b % p.cols) : 0;
   Rows<NT, G, false> R;
   R.init(c.sA, q.li, p.r.nterm);
+  // columns: is everything the segment multiplies with of ordinary size?
+  bool tame = true;
+  if (COLS) {
+    for (int e = threadIdx.x; e < p.r.nterm * NT * Grp<NT, G>::kStride; e += 64) tame = tame && fabs(c.sA[e].x) < kTame && fabs(c.sA[e].y) < kTame;
+    tame = __ballot(!tame) == 0;
+  }
   Z v = mk(0.0, 0.0);
   const int64_t end = p.r.ckpt ? (q.inst * (p.nsegs + 1) + q.seg) * N : q.inst * N;  // where the state comes from
   if (COLS) {
@@ -257,17 +264,25 @@ __global__ __launch_bounds__(64) void small_forward_kernel(SmParams p) {
   // the longest segment of the wavefront sets the trip count; shorter ones stop changing
   for (int64_t s = 0; s < p.r.seg && s < p.r.nsteps; ++s) {
     const bool act = s < q.len;
-    R.combine(field_row<NT, G>(p, q, f, s, false), act);
+    const double* fr = field_row<NT, G>(p, q, f, s, false);
+    R.combine(fr, act);
     const Z n = rk4<NT, G>(R, v, c.x, q.li, p.r.dt);
     if (!act) continue;
     v = n;
-    if (COLS) continue;
+    if (COLS) {
+      for (int i = 0; i < p.r.nterm - 1; ++i) tame = tame && fabs(fr[i]) < kTame;
+      continue;
+    }
     const int64_t t = q.s0 + s + 1;
     if (p.r.n_obs) observe(t);
     if (p.r.rho_out && t % p.r.save_every == 0 && q.row)
       p.r.rho_out[(q.inst * (p.r.nsteps / p.r.save_every) + t / p.r.save_every - 1) * N + q.li] = make_double2(v.x, v.y);
   }
   if (COLS) {
+    // A mode that this dt makes unstable and the state never excites: its column overflows, and steps would leave it
+    // at exactly zero.  Held within 2^1000, zero times it stays zero.  NaN and Inf of the inputs pass.
+    if (tame && !(fabs(v.x) < kHold)) v.x = copysign(kHold, v.x);
+    if (tame && !(fabs(v.y) < kHold)) v.y = copysign(kHold, v.y);
     if (q.row) p.Q[((q.inst * p.nsegs + q.seg) * N + q.li) * N + col] = make_double2(v.x, v.y);
   } else if (q.row && q.seg == p.nsegs - 1) {
     p.r.rho[q.inst * N + q.li] = make_double2(v.x, v.y);

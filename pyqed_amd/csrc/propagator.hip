@@ -18,9 +18,10 @@
 // of 22 us form and square matrices (the FP64 matrix cores; 9 before), 1000 steps of N = 84 130 -> 150, of N = 64
 // 105 -> 110.
 //
-// kCap bounds the powers: the entries of D_j for a mode that this dt makes unstable grow like |P|^(2^j) and must stay
-// finite even if the state never excites that mode (0 x Inf would be NaN where stepping gives 0); |P|^64 overflows only
-// beyond |lambda dt| of about 35, twelve times the stability limit of RK4.
+// The entries of D_j for a mode that this dt makes unstable grow like |P|^(2^j).  Such a mode may belong to a coherence
+// that the state never excites, as one with a far level that nothing couples to, and steps then leave it at exactly
+// zero.  0 x Inf would be NaN, so a square's components are held within 2^1000 (kHold): zero stays zero, and a mode
+// that is excited still overflows, in the rows.
 //
 // States are rows, so the matrices are kept transposed (G_j = D_j^T): v' = v + v G.
 #include <hip/hip_runtime.h>
@@ -38,6 +39,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kCap = 64;            // largest number of steps in one power
 constexpr int kDeepN = 64;          // rows of more elements are summed in short pieces (launch_power)
+constexpr double kHold = 0x1p1000;
 constexpr int power_threads(int split) { return split == 8 ? 512 : 256; }
 constexpr int64_t kTilesFull = 1024;  // wavefront tiles that give every SIMD of the chip one
 constexpr int64_t kScratchBytes = int64_t(256) << 20;  // states kept when the caller keeps none
@@ -65,6 +67,7 @@ struct PwParams {
   double2* w;         // set when X B = zt zt: also writes w = 1/2 + zt/6 + (X B)/24
   double2* wlo;
   double addc;
+  bool hold;          // keep out within kHold
 };
 
 // a value and its remainder
@@ -207,6 +210,11 @@ __device__ __forceinline__ void matrix_task(const PwParams& p, int blk, double2*
   } else {
     x = add(x, Two{p.addc * o.x, p.addc * ol.x});
     y = add(y, Two{p.addc * o.y, p.addc * ol.y});
+    // a generator with a NaN or Inf makes all of the first power NaN: that has to stay
+    if (p.hold && isfinite(o.x) && isfinite(o.y)) {
+      if (!(fabs(x.h) < kHold)) x = Two{copysign(kHold, x.h), 0.0};
+      if (!(fabs(y.h) < kHold)) y = Two{copysign(kHold, y.h), 0.0};
+    }
   }
   p.out[e] = make_double2(x.h, y.h);
   p.outlo[e] = make_double2(x.l, y.l);
@@ -503,6 +511,7 @@ int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps,
   p.outlo = lo[1];
   if ((rc = launch_power(p, false, true, st))) return rc;
   p.addc = 2.0;
+  p.hold = true;
   // the launch that squares power j into power j + 1 also advances rows by power j
   auto level = [&](int j, bool rows, bool square) {
     p.G = G + j * NN;
