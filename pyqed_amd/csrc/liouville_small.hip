@@ -16,9 +16,10 @@
 // short chain over segments gives the state at every segment's start and, for gradients, the adjoint state
 // at every segment's end, and then all segments run at once.  The work grows by about N + 1 but the chain
 // falls from nsteps to nsteps / seg + 2 seg steps.  One N = 9 instance, 1000 driven steps: 1868 -> 137 us
-// forward, 15.3 -> 0.26 ms for the gradients; 4000 steps: 7670 -> 255 us and 61.7 -> 0.49 ms.  The gradients'
-// error against extended precision (Lambda system, 100..1200 steps) is 0.65, 0.87 and 0.58 times the uncut
-// sweep's of liouville.hip for parameters, amplitudes and initial state.
+// forward, 15.3 -> 0.26 ms for the gradients; 4000 steps: 7670 -> 255 us and 61.7 -> 0.49 ms.  Error
+// against extended precision relative to the uncut run and sweep of liouville.hip (Lambda system, 100..1200 steps, 14
+// fields, geometric mean): parameters 0.75, amplitudes 0.47, initial state 0.38; with amplitudes held for 250 steps and
+// more (root mean square) final state 0.35, amplitudes 0.7, initial state 0.15.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -39,7 +40,7 @@ struct SmParams {
   int64_t groups;    // of this launch
   int64_t seg_buf;   // adjoint: element offset of the segment states within ckpt
   int cols;          // forward: N when the groups are propagator columns (instance, segment, column), else 1
-  double2* Q;        // [n_inst][nsegs][N][N] segment propagators
+  double2* Q;        // [n_inst][nsegs][N][N] segment propagators less the identity
   double2* lamT;     // [n_inst][nsegs][N] adjoint states at the segments' ends (split), else NULL
   double2* part;     // [n_inst][nsegs][nterm][N][N] gradient parts (split), else NULL
 };
@@ -175,7 +176,7 @@ __device__ __forceinline__ const double* field_row(const SmParams& p, const Grp<
   return f.w + (s - f.lo) * nt1;
 }
 
-// One RK4 step of the lane's element v; x: the group's LDS vector
+// What one RK4 step adds to the lane's element v; x: the group's LDS vector
 template <int NT, int G>
 __device__ __forceinline__ Z rk4(const Rows<NT, G, false>& R, Z v, Z* x, int li, double dt) {
   const double dt2 = dt / 2.0;
@@ -188,7 +189,7 @@ __device__ __forceinline__ Z rk4(const Rows<NT, G, false>& R, Z v, Z* x, int li,
   };
   const Z k1 = mul(v), k2 = mul(v + k1 * dt2), k3 = mul(v + k2 * dt2), k4 = mul(v + k3 * dt);
   const Z t = k1 + k2 * 2.0 + k3 * 2.0 + k4;
-  return v + mk(t.x / 6.0 * dt, t.y / 6.0 * dt);
+  return mk(t.x / 6.0 * dt, t.y / 6.0 * dt);
 }
 
 // LDS: [generators][per group: vector NT][per group: field window kWin or nterm - 1 values]
@@ -236,7 +237,9 @@ __global__ __launch_bounds__(64) void small_forward_kernel(SmParams p) {
     for (int e = threadIdx.x; e < p.r.nterm * NT * Grp<NT, G>::kStride; e += 64) tame = tame && fabs(c.sA[e].x) < kTame && fabs(c.sA[e].y) < kTame;
     tame = __ballot(!tame) == 0;
   }
-  Z v = mk(0.0, 0.0);
+  // Columns are summed without their unit vector: segments under one field share a propagator, and rounding of the
+  // sum to the unit's ulp would repeat in each and add up.  The increment rounds to its own.
+  Z v = mk(0.0, 0.0), sum = v;
   const int64_t end = p.r.ckpt ? (q.inst * (p.nsegs + 1) + q.seg) * N : q.inst * N;  // where the state comes from
   if (COLS) {
     if (q.row && q.li == col) v.x = 1.0;
@@ -268,11 +271,13 @@ __global__ __launch_bounds__(64) void small_forward_kernel(SmParams p) {
     R.combine(fr, act);
     const Z n = rk4<NT, G>(R, v, c.x, q.li, p.r.dt);
     if (!act) continue;
-    v = n;
     if (COLS) {
+      sum = sum + n;
+      v = mk((q.li == col ? 1.0 : 0.0) + sum.x, sum.y);
       for (int i = 0; i < p.r.nterm - 1; ++i) tame = tame && fabs(fr[i]) < kTame;
       continue;
     }
+    v = v + n;
     const int64_t t = q.s0 + s + 1;
     if (p.r.n_obs) observe(t);
     if (p.r.rho_out && t % p.r.save_every == 0 && q.row)
@@ -281,9 +286,9 @@ __global__ __launch_bounds__(64) void small_forward_kernel(SmParams p) {
   if (COLS) {
     // A mode that this dt makes unstable and the state never excites: its column overflows, and steps would leave it
     // at exactly zero.  Held within 2^1000, zero times it stays zero.  NaN and Inf of the inputs pass.
-    if (tame && !(fabs(v.x) < kHold)) v.x = copysign(kHold, v.x);
-    if (tame && !(fabs(v.y) < kHold)) v.y = copysign(kHold, v.y);
-    if (q.row) p.Q[((q.inst * p.nsegs + q.seg) * N + q.li) * N + col] = make_double2(v.x, v.y);
+    if (tame && !(fabs(sum.x) < kHold)) sum.x = copysign(kHold, sum.x);
+    if (tame && !(fabs(sum.y) < kHold)) sum.y = copysign(kHold, sum.y);
+    if (q.row) p.Q[((q.inst * p.nsegs + q.seg) * N + q.li) * N + col] = make_double2(sum.x, sum.y);
   } else if (q.row && q.seg == p.nsegs - 1) {
     p.r.rho[q.inst * N + q.li] = make_double2(v.x, v.y);
   }
@@ -323,7 +328,7 @@ __global__ __launch_bounds__(64) void small_chain_kernel(SmParams p, int dirs) {
       else cmac(a, cur[k], x[k]);
       cur[k] = nxt[k];
     }
-    v = a + b;
+    v = v + (a + b);
     wave_order();
   }
 }
@@ -372,7 +377,7 @@ __global__ __launch_bounds__(64) void small_adjoint_kernel(SmParams p, int64_t s
       if (s + 1 == most) break;
       R.combine(field_row<NT, G>(p, q, f, s, false), act);
       const Z n = rk4<NT, G>(R, v, c.x, q.li, dt);
-      if (act) v = n;
+      if (act) v = v + n;
     }
     // the lane reads back its own elements only: v holds the last one, the others come a step ahead
     double2 ahead = make_double2(0.0, 0.0);
@@ -480,7 +485,7 @@ __global__ __launch_bounds__(64) void small_checkpoint_kernel(SmParams p) {
   for (int64_t s = 0; s < p.r.nsteps; ++s) {
     if (s % p.r.seg == 0 && q.row) p.r.ckpt[(q.inst * (p.nsegs + 1) + s / p.r.seg) * N + q.li] = make_double2(v.x, v.y);
     R.combine(field_row<NT, G>(p, q, f, s, false), true);
-    v = rk4<NT, G>(R, v, c.x, q.li, p.r.dt);
+    v = v + rk4<NT, G>(R, v, c.x, q.li, p.r.dt);
   }
 }
 
