@@ -321,8 +321,8 @@ int pyqed_basis_change(int32_t d, int64_t n, const void* V, void* rho, void* str
 
 /* pyqed_liouville_adjoint with a workspace of pyqed_liouville_adjoint_work_bytes (at least the checkpoints that
  * pyqed_liouville_adjoint takes; work replaces ckpt).  For N <= 16 and few instances the sweep is cut along
- * time: the segments' propagators give every segment's first state and last adjoint state, then all segments
- * are swept at once. */
+ * time where that takes at most 4 GiB and the workspace holds it: the segments' propagators give every
+ * segment's first state and last adjoint state, then all segments are swept at once. */
 int pyqed_liouville_adjoint_work_bytes(int32_t N, int32_t nterm, int32_t n_inst, int64_t nsteps, int32_t ckpt_every,
                                        int64_t* bytes);
 int pyqed_liouville_adjoint_work(int32_t N, int32_t nterm, const void* A, int32_t n_inst, const void* rho0,

@@ -72,11 +72,15 @@ class LindbladAdjoint:
         r0b = torch.zeros((1, self.N), dtype=torch.complex128, device=dev)
         wb = _lib.C.c_int64()
         _lib.check(L.pyqed_liouville_adjoint_work_bytes(self.N, nterm, 1, self.nsteps, self.ckpt_every, _lib.C.byref(wb)))
-        work = torch.empty(wb.value, dtype=torch.uint8, device=dev)
+        try:
+            work = torch.empty(wb.value, dtype=torch.uint8, device=dev)
+        except torch.OutOfMemoryError:  # no room to cut the sweep along time: the checkpoints alone
+            nck = (self.nsteps + self.ckpt_every - 1) // self.ckpt_every + 1
+            work = torch.empty((nck + self.ckpt_every) * self.N * 16, dtype=torch.uint8, device=dev)
         _lib.check(L.pyqed_liouville_adjoint_work(self.N, nterm, A.data_ptr(), 1, rho.data_ptr(), _lib.ptr(f), self.nsteps,
                                                   self.dt, self.ckpt_every, bar.data_ptr(),
                                                   gf.data_ptr() if nterm > 1 else None, gA.data_ptr(), r0b.data_ptr(),
-                                                  work.data_ptr(), wb.value, _lib.stream_ptr(torch)))
+                                                  work.data_ptr(), work.numel(), _lib.stream_ptr(torch)))
         torch.cuda.synchronize()
         gA0 = gA[0, 0].cpu().numpy()
         g_theta = np.array([np.real(np.sum(np.conj(gA0) * Gj)) for Gj in self.G])

@@ -31,6 +31,7 @@ namespace {
 
 constexpr int kWin = 64;  // values of a group's field window in LDS
 constexpr double kTame = 1e150, kHold = 0x1p1000;
+constexpr int64_t kSplitBytes = int64_t(4) << 30;  // largest workspace of a cut run, 1.4% of a GPU's 288 GB
 
 typedef cpx<double> Z;
 
@@ -572,7 +573,9 @@ int64_t small_split(int N, int nterm, int n_inst, int64_t nsteps, bool adjoint) 
   if (load > (adjoint ? (N <= 4 ? 0.5 : 1.5) : (N <= 4 ? 0.15 : 0.5))) return 0;
   int64_t seg = 4;
   while (seg * seg * (adjoint ? 10 : 5) < nsteps && seg < 64) ++seg;
-  return (nsteps + seg - 1) / seg < 6 ? 0 : seg;
+  if ((nsteps + seg - 1) / seg < 6) return 0;
+  // a cut run holds its propagators and a cut gradient every state besides, whatever checkpoints it was asked for
+  return small_split_bytes(N, nterm, n_inst, nsteps, seg, adjoint) > kSplitBytes ? 0 : seg;
 }
 
 int64_t small_split_bytes(int N, int nterm, int n_inst, int64_t nsteps, int64_t seg, bool adjoint) {
