@@ -21,11 +21,12 @@ accumulated per step and field column by pyqed_heom_adjoint_contract.  J is real
 dJ = Re sum conj(rhoT_bar) d rho(T) (rhoT_bar = dJ/dRe rho + i dJ/dIm rho; for J = Re Tr(O rho(T)),
 rhoT_bar = O^H).
 
-Memory: where the stage inputs of all steps (4 nt states) fit `HeomAdjoint.keep_bytes`, the forward run keeps
-them and nothing is recomputed.  Beyond that the forward run keeps the state every `ckpt_every` steps and the
-backward sweep recomputes one segment at a time, the last one excepted: its stage inputs where 4 ckpt_every
-states fit (nt / ckpt_every + 4 ckpt_every states in all), else its states, with the stage inputs formed again
-step by step (nt / ckpt_every + ckpt_every states).
+Memory: a sweep that keeps stage inputs holds 4 m + 1 states of the m steps it keeps, 4 b + 1 of the adjoint over b <= 32
+of them, three more states and the contraction's workspace of b steps.  Where all nt steps fit `HeomAdjoint.keep_bytes`
+that way, the forward run keeps them and nothing is recomputed.  Beyond that the forward run keeps the state every
+`ckpt_every` steps and the backward sweep recomputes one segment at a time, the last one excepted: its stage inputs
+where m = ckpt_every fits, else its states, with the stage inputs formed again step by step (nt / ckpt_every +
+ckpt_every states and eight more: keep_bytes = 0 holds a gradient to that).
 """
 import ctypes as C
 
@@ -37,7 +38,8 @@ from .. import _lib
 class HeomAdjoint:
     """Forward run and streamed adjoint of one or more HEOM instances (HeomEngine instance dicts)."""
 
-    # Stage inputs kept for the backward sweep, 1.4% of a GPU's 288 GB.  A step costs 8 launches with all of them
+    # What the backward sweep may hold in stage inputs, both directions', and their contraction: 1.4% of a GPU's 288 GB,
+    # whatever ckpt_every is.  A step costs 8 launches with all of them
     # kept, 12 with a segment's, 16 and a copy with none: on 680 ADOs of 7 x 7, where a launch takes about 7 us
     # whatever it does, and on large hierarchies, where it takes its bytes, the fewer the faster.
     keep_bytes = 4 << 30
@@ -106,6 +108,18 @@ class HeomAdjoint:
         return self.fwd.reduced_states()
 
     # ------------------------------------------------------------------ gradient
+    @staticmethod
+    def kept_steps(nt, ckpt_every, state, contraction, keep):
+        """(steps whose stage inputs are held at a time, those of an adjoint sweep over them) for states of `state` bytes,
+        a contraction workspace of `contraction` bytes a step and a limit of `keep` bytes; (ckpt_every, 0) where none fit."""
+        for seg in (nt, min(ckpt_every, nt)):
+            b = min(seg, 32)
+            while b:
+                if (4 * seg + 1 + 4 * b + 1 + 3) * state + b * contraction <= keep:
+                    return (nt if seg == nt else ckpt_every), b
+                b //= 2
+        return ckpt_every, 0
+
     def gradient(self, rhoT_bar, field=None):
         """Backward sweep.  rhoT_bar: list (one per instance) of d x d cotangents of rho(T).
 
@@ -129,12 +143,10 @@ class HeomAdjoint:
         stream = _lib.stream_ptr(torch)
         fp = None if f is None else f.data_ptr()
         # steps whose stage inputs are kept at a time (X), and of those the steps of an adjoint sweep (U)
-        state = 16 * n
-        seg = nt if 4 * nt * state <= self.keep_bytes else ck
+        seg, cb = self.kept_steps(nt, ck, 16 * n, self._wb, self.keep_bytes)
         X = None
-        if nt and 4 * seg * state <= self.keep_bytes:
+        if cb:
             try:
-                cb = min(seg, 32)
                 X = torch.empty((4 * min(seg, nt) + 1, n), dtype=torch.complex128, device=dev)
                 U = torch.empty((4 * cb + 1, n), dtype=torch.complex128, device=dev)
                 acc = torch.empty(n, dtype=torch.complex128, device=dev)
