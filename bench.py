@@ -729,6 +729,22 @@ def cavity_problem(d=64, n=256, seed=21):
     return H, c_ops, np.array(rhos), [num, a + a.conj().T]
 
 
+def matrix_form_flops(Heff, c_ops):
+    """Flops of one RK4 step of the matrix form: H X, X H^dagger, X c^dagger and c T in every stage, 16 x 16 blocks.  The
+    real and the imaginary part of an operator's block take two real products of 2 16^3 flops with every tile of the
+    other factor, and a part that is zero takes none."""
+    d = Heff.shape[0]
+    nt = -(-d // 16)
+
+    def parts(op):
+        a = np.zeros((16 * nt, 16 * nt), np.complex128)
+        a[:d, :d] = op
+        a = a.reshape(nt, 16, nt, 16)
+        return int(sum(np.any(x != 0, axis=(1, 3)).sum() for x in (a.real, a.imag)))
+
+    return 4 * 2 * 2 * 16 ** 3 * nt * (2 * parts(Heff) + 2 * sum(parts(c) for c in c_ops))
+
+
 def bench_lindblad_matrix(args, torch):
     """LindbladSolver.run for a d = 64 system (beyond the Liouville kernel's d*d <= 1024): the matrix-form
     kernel, n_inst initial states per launch, two observables every step (oqs.py:1596-1696)."""
@@ -772,14 +788,8 @@ def bench_lindblad_matrix(args, torch):
     ev[1].record(st)
     torch.cuda.synchronize()
     launch_ms = ev[0].elapsed_time(ev[1])
-    # complex products of an RK4 step over the operators' 16 x 16 blocks that are not zero
     nt = -(-d // 16)
-
-    def blocks(op):
-        a = np.zeros((16 * nt, 16 * nt), np.complex128)
-        a[:d, :d] = op
-        return int(np.any(a.reshape(nt, 16, nt, 16) != 0, axis=(1, 3)).sum())
-    flops = 4 * 8 * 16 ** 3 * nt * (2 * blocks(Heff) + 2 * sum(blocks(c) for c in c_ops)) * nsteps * n
+    flops = matrix_form_flops(Heff, c_ops) * nsteps * n
     achieved = flops / (launch_ms / 1e3) / 1e12
     kernel = (f"lindblad_resident_kernel<{nt}, false>" if nt <= 4 and n >= (0, 1, 16, 96, 96)[nt] else
               "lindblad_product_kernel (8 launches per step)")
@@ -796,7 +806,8 @@ def bench_lindblad_matrix(args, torch):
         "roofline": {"bound": "mfma", "kernel": kernel, "launch_ms": launch_ms,
                      "flops_per_launch": flops, "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None,
-                     "note": "FP64 MFMA; flops of the products over 16 x 16 operator blocks that are not zero"},
+                     "note": "FP64 MFMA; flops of the real products over the real and imaginary parts of 16 x 16 operator "
+                             "blocks that are not zero"},
         "trace_deviation": trace_dev,
     }
     if not args.no_cpu:
