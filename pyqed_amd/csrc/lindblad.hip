@@ -38,6 +38,7 @@ namespace {
 
 constexpr int kLThreads = 256;
 constexpr int64_t kFullChip = 256;  // CUs: workgroups from which a launch fills the chip
+constexpr int64_t kGridBlocks = (int64_t(1) << 32) / kLThreads - 1;  // a grid's threads are counted in 32 bits
 constexpr int kScanBlocks = 64;  // workgroups of the non-finite scan
 
 typedef double doublex4 __attribute__((ext_vector_type(4)));
@@ -801,13 +802,13 @@ extern "C" int pyqed_lindblad_run(int32_t d, int32_t nc, const void* Heff, const
   // 32 x 32 wavefront tiles once they give every CU a workgroup, 16 x 16 tiles split four ways below
   const int64_t t16 = (int64_t)p.nt * p.nt, t32 = (int64_t)((p.nt + 1) / 2) * ((p.nt + 1) / 2);
   const bool big = p.nt > 1 && t32 * n_inst >= 4 * kFullChip;
-  // instances per launch, so that no grid exceeds 2^31 - 1 workgroups
+  // instances per launch, so that no grid holds 2^32 threads or more
   const int64_t d2 = (int64_t)d * d;
   const int64_t hs_blocks = ndrive > 0 ? std::min<int64_t>((d2 + 4 * kLThreads - 1) / (4 * kLThreads), 64) : 0;
   if ((int64_t)n_obs + hs_blocks > INT32_MAX / 4) return fail(PYQED_EINVAL, "lindblad_run: too many observables");
   p.side_blocks = (int)(n_obs + hs_blocks);
-  const int64_t per_inst = std::max<int64_t>(std::max(nc, 1) * t16 + p.side_blocks, 1);
-  const int64_t chunk = std::max<int64_t>(1, (int64_t)INT32_MAX / per_inst / 2);
+  const int64_t tiles = std::max(nc, 1) * (big ? (t32 + 3) / 4 : t16);
+  const int64_t chunk = std::max<int64_t>(1, kGridBlocks / (tiles + p.side_blocks + 1));
   for (int64_t i0 = 0; i0 < n_inst; i0 += chunk) {
     p.inst0 = (int)i0;
     p.n_inst = (int)std::min<int64_t>(chunk, n_inst - i0);

@@ -366,22 +366,25 @@ __global__ __launch_bounds__(kThreads) void liouville_step_kernel(int N, const d
 __global__ __launch_bounds__(kThreads) void liouville_observe_kernel(PwParams p, int gsz, int n_obs, const double2* obs,
                                                                      double2* obs_out, int64_t out_rows, int64_t t0) {
   const int li = threadIdx.x % gsz;
-  const int64_t r = blockIdx.x * (int64_t)(kThreads / gsz) + threadIdx.x / gsz;
-  const bool live = r < (int64_t)p.cnt * p.n_inst;
-  const int64_t i = live ? r / p.cnt : 0, s = live ? p.s_in + (r - i * p.cnt) : p.s_in;
-  const double2* v = row_ptr(p, i, s);
-  for (int o = 0; o < n_obs; ++o) {
-    double re = 0.0, im = 0.0;
-    for (int e = li; e < p.N; e += gsz) {
-      const double2 a = obs[(int64_t)o * p.N + e], x = v[e];
-      re += a.x * x.x - a.y * x.y;
-      im += a.x * x.y + a.y * x.x;
+  const int64_t per = kThreads / gsz, nr = (int64_t)p.cnt * p.n_inst;
+  for (int64_t r0 = blockIdx.x * per; r0 < nr; r0 += gridDim.x * per) {  // the same trips for every lane
+    const int64_t r = r0 + threadIdx.x / gsz;
+    const bool live = r < nr;
+    const int64_t i = live ? r / p.cnt : 0, s = live ? p.s_in + (r - i * p.cnt) : p.s_in;
+    const double2* v = row_ptr(p, i, s);
+    for (int o = 0; o < n_obs; ++o) {
+      double re = 0.0, im = 0.0;
+      for (int e = li; e < p.N; e += gsz) {
+        const double2 a = obs[(int64_t)o * p.N + e], x = v[e];
+        re += a.x * x.x - a.y * x.y;
+        im += a.x * x.y + a.y * x.x;
+      }
+      for (int w = gsz / 2; w > 0; w >>= 1) {
+        re += __shfl_xor(re, w, gsz);
+        im += __shfl_xor(im, w, gsz);
+      }
+      if (live && li == 0) obs_out[(i * out_rows + t0 + s) * n_obs + o] = make_double2(re, im);
     }
-    for (int w = gsz / 2; w > 0; w >>= 1) {
-      re += __shfl_xor(re, w, gsz);
-      im += __shfl_xor(im, w, gsz);
-    }
-    if (live && li == 0) obs_out[(i * out_rows + t0 + s) * n_obs + o] = make_double2(re, im);
   }
 }
 
@@ -573,8 +576,8 @@ int run_power(int N, const double2* A, int n_inst, double2* rho, int64_t nsteps,
     if (n_obs) {
       p.cnt = (int)(S + 1 - p.s_in);
       const int64_t per = kThreads / gsz, nr = (int64_t)p.cnt * n_inst;
-      hipLaunchKernelGGL(liouville_observe_kernel, dim3((unsigned)((nr + per - 1) / per)), dim3(kThreads), 0, st, p, gsz, n_obs, obs,
-                         obs_out, nsteps + 1, t0);
+      hipLaunchKernelGGL(liouville_observe_kernel, dim3((unsigned)std::min<int64_t>((nr + per - 1) / per, 1 << 20)), dim3(kThreads), 0, st, p,
+                         gsz, n_obs, obs, obs_out, nsteps + 1, t0);
       PQA_HIP(hipGetLastError());
     }
     if (pick && (t0 + S) / pick->every > t0 / pick->every) {
