@@ -26,7 +26,9 @@ from .spectral import TIME, spectral_sum
 class LindbladSolver:
     """form (keyword only): "auto" runs d*d <= 1024 on the Liouville-space kernel (vec(rho) and its
     generator in LDS) and larger d on the matrix-form kernel (pyqed_lindblad_run), which also takes driven
-    Hermitian Hamiltonians from d = 8 on; "liouville" or "matrix" force one of them."""
+    Hamiltonians from d = 8 on where H and the drives equal their adjoints to the last bit (a rotated V E V^dagger
+    rarely does, 0.5 * (H + H^dagger) does; at d = 24 a step is 40 times as fast) and 24 len(c_ops) <= d * d; "liouville" or
+    "matrix" force one of them."""
 
     def __init__(self, H=None, c_ops=None, e_ops=None, *, form="auto"):
         if form not in ("auto", "liouville", "matrix"):
@@ -77,8 +79,14 @@ class LindbladSolver:
                          and all(np.shape(a) == (d, d) for a in [H0, *drives, *c_ops])
                          and all(np.array_equal(h, dag(h)) for h in [H0, *drives]))
         if self.form == "matrix" or (self.form == "auto" and (d * d > 1024 or driven_matrix)):
-            return propagate_matrix(H0, c_ops, drives, rho0s, dt, Nt, field if drives else None, e_ops,
-                                    keep_states=keep_states)
+            try:
+                return propagate_matrix(H0, c_ops, drives, rho0s, dt, Nt, field if drives else None, e_ops,
+                                        keep_states=keep_states)
+            except RuntimeError as e:
+                # its workspace is 5 + n_c matrices an instance; the Liouville-space kernel needs the states alone
+                import torch
+                if self.form == "matrix" or d * d > 1024 or not isinstance(e, torch.OutOfMemoryError):
+                    raise
         gens = [lindblad_generator(H0, c_ops)] + [1j * op2sop(Hi) for Hi in drives]
         return propagate(np.array(gens), rho0s, dt, Nt, field if drives else None, e_ops, keep_states=keep_states)
 
