@@ -136,7 +136,11 @@ int pyqed_heom_tables_build(int32_t K, int32_t L, int64_t* keys, int32_t* plus, 
  *              aligned to 128 bytes), then ADO after ADO (full d x d matrices,
  *              or upper triangles with PYQED_PLAN_PACKED), updated in place
  *              (ADO 0 of each instance is the reduced rho).
- *   workspace  device, >= ws_bytes for `precision` (plan_query); scratch.
+ *   workspace  device, >= ws_bytes for `precision` (plan_query); scratch.  A plan of one small hierarchy runs
+ *              undriven FP64 calls of max(64, N^2 / 2400) steps and more, N <= 640 its elements, by powers of its
+ *              dense generator, which takes most of that size; with less than it, but 16 bytes for every element
+ *              of the state (rounded up to 256) and 32 for every full-matrix element, the run steps.  The two
+ *              agree to rounding, not bit for bit, so results depend at that level on how a run is cut into calls.
  *   field      device [(step0+nsteps)*6] double or NULL: for step s,
  *              field[6s+0..2] = f_s(t), f_s(t+dt/2), f_s(t+dt) and
  *              field[6s+3..5] = f_c at the same times (t = s*dt).

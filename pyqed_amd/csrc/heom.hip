@@ -2797,10 +2797,10 @@ int power_size(const pyqed_heom_plan* P) {
 // 8 to 9 us beyond.  us per call of 63 steps by the resident kernel and of 64 by powers: N = 84 178 and 107, 144 188 and
 // 135, 252 219 and 189, 324 555 and 337, 336 572 and 346, 448 573 and 749, 576 634 and 1288 (1298 for 150 steps).
 int64_t power_steps(int N) { return std::max<int64_t>(64, (int64_t)N * N / 2400); }
+int64_t step_bytes(const pyqed_heom_plan* P, size_t xsize) { return ws_state_bytes(P) + 2 * P->n_elems * (int64_t)xsize; }
 int64_t workspace_bytes(const pyqed_heom_plan* P, size_t xsize) {
-  const int64_t stream = ws_state_bytes(P) + 2 * P->n_elems * (int64_t)xsize;
   const int64_t N = xsize == sizeof(double2) ? power_size(P) : 0;
-  return N ? std::max(stream, 16 * (N * N + N) + power_vector_bytes((int)N)) : stream;
+  return std::max(step_bytes(P, xsize), N ? 16 * (N * N + N) + power_vector_bytes((int)N) : 0);
 }
 
 size_t stream_lds_bytes(const pyqed_heom_plan* P, size_t tsize) {
@@ -4014,7 +4014,7 @@ extern "C" int pyqed_heom_run(pyqed_heom_plan* P, int32_t precision, void* y, vo
   if (!P || !y || !workspace) return fail(PYQED_EINVAL, "heom_run: null plan, state or workspace");
   if (nsteps < 0 || step0 < 0) return fail(PYQED_EINVAL, "heom_run: negative step count");
   if (save_every <= 0) save_every = 1;
-  const int64_t need = workspace_bytes(P, precision == PYQED_PREC_FP64 ? sizeof(double2) : sizeof(float2));
+  const int64_t need = step_bytes(P, precision == PYQED_PREC_FP64 ? sizeof(double2) : sizeof(float2));
   if (precision != PYQED_PREC_FP64 && precision != PYQED_PREC_MIXED)
     return fail(PYQED_EINVAL, "heom_run: precision must be PYQED_PREC_FP64 or PYQED_PREC_MIXED");
   if (ws_bytes < need)
@@ -4022,7 +4022,8 @@ extern "C" int pyqed_heom_run(pyqed_heom_plan* P, int32_t precision, void* y, vo
                                   std::to_string(need) + " bytes)");
   if (nsteps == 0) return PYQED_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (precision == PYQED_PREC_FP64 && !field && power_size(P) && nsteps >= power_steps(power_size(P)))
+  if (precision == PYQED_PREC_FP64 && !field && power_size(P) && nsteps >= power_steps(power_size(P)) &&
+      ws_bytes >= workspace_bytes(P, sizeof(double2)))
     return power_run(P, (double2*)y, (char*)workspace, nsteps, dt, (double2*)traj, save_every, st);
   if (precision == PYQED_PREC_FP64)
     return run_typed<double>(P, (double2*)y, (char*)workspace, field, step0, nsteps, dt, (double2*)traj, save_every,

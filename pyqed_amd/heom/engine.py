@@ -24,6 +24,7 @@ import numpy as np
 from .. import _lib
 
 PRECISIONS = {"fp64": _lib.PREC_FP64, "mixed": _lib.PREC_MIXED, "fp32": _lib.PREC_MIXED}
+POWER_STEPS = 64  # no shorter call takes powers of a small hierarchy's generator (pyqed_heom_run)
 NCLASSES = 4  # streamed kernel classes of a plan (pyqed_heom_plan_classes)
 
 
@@ -168,7 +169,7 @@ class HeomEngine:
         self.device = torch.device("cuda", torch.cuda.current_device())
         self.y = torch.zeros(self.n_elems, dtype=torch.complex128, device=self.device)
         self._ws = None
-        self._ws_prec = None
+        self._no_room = False
         self._tuned = set()
         self.variant = 0
         self.autotune_cache = True
@@ -203,13 +204,26 @@ class HeomEngine:
         self.y[torch.as_tensor(idx, device=self.device)] = torch.as_tensor(np.concatenate(vals), device=self.device)
         self.step = 0
 
-    def workspace(self, prec):
+    def workspace(self, prec, nsteps=POWER_STEPS, driven=False):
+        """Scratch of a call of nsteps steps.  plan_query's FP64 size holds the powers of a small hierarchy's generator
+        (up to 98 MB for a state of 164 KB): calls that only step do without, as do all where the device has no room."""
         torch = self.torch
         need = self.ws_bytes[prec]
+        # stepping: the state, and two stage buffers of 8 bytes an element in mixed precision, 16 in FP64
+        step = 2 * self.ws_bytes[_lib.PREC_MIXED] - -(-16 * self.n_elems // 256) * 256
+        if prec == _lib.PREC_FP64 and (driven or nsteps < POWER_STEPS or self._no_room):
+            need = min(need, step)
         if self._ws is None or self._ws.numel() < need:
             # captured graphs hold the old workspace's address: drop them before it is released
             self._drop_graphs()
-            self._ws = torch.empty(max(need, 256), dtype=torch.uint8, device=self.device)
+            try:
+                self._ws = torch.empty(max(need, 256), dtype=torch.uint8, device=self.device)
+            except torch.OutOfMemoryError:
+                if step >= need:
+                    raise
+                self._no_room = True
+                if self._ws is None or self._ws.numel() < step:
+                    self._ws = torch.empty(max(step, 256), dtype=torch.uint8, device=self.device)
         return self._ws
 
     def _drop_graphs(self):
@@ -325,7 +339,7 @@ class HeomEngine:
                     if tb:
                         self.set_class_tiling(c, *tb)
                 self._tuned_hit = True
-        ws = self.workspace(prec)
+        ws = self.workspace(prec, nsteps, field is not None)
         _lib.check(self.L.pyqed_heom_run(
             self.plan, prec, self.y.data_ptr(), ws.data_ptr(), ws.numel(),
             None if field is None else field.data_ptr(), self.step, nsteps, float(dt),
@@ -358,7 +372,7 @@ class HeomEngine:
                              "system or coupling dipole (time-dependent fields) must use advance()")
         if getattr(self, "_graphs", None) is None:
             self._graphs = {}
-        self.workspace(PRECISIONS[precision])
+        self.workspace(PRECISIONS[precision], chunk)
         if self.autotune_cache and precision not in self._tuned:
             self.advance(0, dt, precision)  # apply the cached tiling before looking up or capturing a graph
         key = (precision, chunk, float(dt))
