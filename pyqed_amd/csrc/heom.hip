@@ -2202,6 +2202,39 @@ __global__ __launch_bounds__(kThreads) void heom_lean_kernel(StageParams p) {
   }
 }
 
+// The lean kernel's entries, group starts and damping, a wavefront per ADO, as the projector kernel forms them in every
+// launch.  Made on the device: 10 sites at depth 4 (10626 ADOs, 2 MB) took 510 us on the host and 130 to copy, so that
+// a plan cost 8 of the steps that its kernel saved.
+__global__ __launch_bounds__(kThreads) void heom_lean_tables_kernel(InstDev I, const int32_t* rowptr, const int2* ent, const int32_t* site,
+                                                                    const double2* coefp, LeanTables t, double2* damp64, float2* damp32) {
+  const int lane = threadIdx.x & 63, a = blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (a >= I.nmax) return;
+  const int r0 = rowptr[I.rowptr_off + a], n = min(rowptr[I.rowptr_off + a + 1] - r0, t.stride);
+  int2 en = make_int2(0, 0);
+  if (lane < n) en = ent[I.ent_off + r0 + lane];
+  const int k = en.y & 0xffff, nf = (en.y >> 16) & 0x7f, plus = en.y < 0;
+  const int my_site = lane < n ? site[I.site_off + k] : 0x7fffffff;
+  int first;
+  const int pos = site_order(my_site, I.d, lane, (I.flags & F_SITESORT) != 0, first);
+  if (lane < t.stride)
+    const_cast<int2*>(t.ent)[(int64_t)a * t.stride + (lane < n ? pos : lane)] =
+        lane < n ? make_int2(en.x * I.d + my_site, my_site << 16 | ((k * (I.L + 2) + nf) * 2 + plus)) : make_int2(0, 0);
+  if (lane <= I.d) const_cast<uint8_t*>(t.start)[(int64_t)a * 16 + lane] = (uint8_t)first;
+  cpx<double> g = mk(0.0, 0.0);
+  cpx<float> h = mk(0.f, 0.f);
+  if (lane < n && !plus) {
+    const double2 c = coefp[I.coefp_off + 5 * k];
+    g = mk(c.x, c.y) * (double)nf;
+    h = mk((float)c.x, (float)c.y) * (float)nf;
+  }
+  g = wave_sum(g);
+  h = wave_sum(h);
+  if (lane == 0) {
+    damp64[a] = make_double2(g.x, g.y);
+    damp32[a] = make_float2(h.x, h.y);
+  }
+}
+
 // ------------------------------------------------------------------ LDS-resident kernel
 // One workgroup owns one small instance for the whole run: y, ynew and both
 // stage buffers live in LDS, so HBM is touched only to load the initial state,
@@ -2685,7 +2718,9 @@ struct pyqed_heom_plan {
   // the lean kernel's instance (or -1: class 1 runs the projector kernel) and tables
   int lean_inst = -1;
   LeanTables lean64 = {}, lean32 = {};
-  char* d_lean = nullptr;
+  char* d_lean = nullptr;       // entries, group starts and damping
+  char* d_lean_pairs = nullptr;
+  size_t lean_bytes = 0;
   char* d_arena = nullptr;  // the small tables (Arena)
   size_t arena_bytes = 0;
   double2* d_coef = nullptr;
@@ -2743,8 +2778,8 @@ int upload(const std::vector<V>& h, V** d) {
 // The tables of a plan on their way to the device: those of up to kArenaTable bytes go into one allocation with one
 // copy (P->d_arena), larger ones each into their own, without a second copy on the host.  An allocation, its copy and
 // its release cost about 15 us each: an engine of a resident two-level hierarchy took 398 us to make and 141 to
-// close with a buffer per table and two streams, and takes 174 and 11; of 7 sites at depth 4 561 and 144, now 407
-// and 72.
+// close with a buffer per table and two streams, and takes 174 and 11; of 7 sites at depth 4 561 and 144, now 300
+// and 55.
 constexpr size_t kArenaTable = size_t(1) << 18;
 
 struct Arena {
@@ -2757,6 +2792,18 @@ struct Arena {
     const size_t o = (host.size() + 4095) & ~size_t(4095);
     host.resize(o + sizeof(V) * h.size());
     std::memcpy(host.data() + o, h.data(), sizeof(V) * h.size());
+    at.push_back({(void**)d, o});
+    return PYQED_OK;
+  }
+  // room for a table that is made on the device
+  int reserve(size_t n, char** d) {
+    if (n == 0) return PYQED_OK;
+    if (n > kArenaTable) {
+      PQA_HIP(hipMalloc((void**)d, n));
+      return PYQED_OK;
+    }
+    const size_t o = (host.size() + 4095) & ~size_t(4095);
+    host.resize(o + n);
     at.push_back({(void**)d, o});
     return PYQED_OK;
   }
@@ -2821,57 +2868,27 @@ size_t pipe_lds_bytes(const pyqed_heom_plan* P, int c) {
   return proj_block_bytes(q.d2pad, q.Kmax, q.Lmax, sizeof(float), false) + (kThreads / 64) * pipe_wave_bytes(q.d2pad, q.rowbuf);
 }
 
-// Tables of the lean kernel for instance `only` (P->lean64, lean32 hold offsets into the returned buffer until it
-// is uploaded).  The damping is summed as the projector kernel's wavefront sums it, in the run's precision, and
-// the coefficient pairs are the products that it forms.  Empty where an index would not fit its field.
-std::vector<char> lean_tables(pyqed_heom_plan* P, int only, const int32_t* rowptr, const int2* ent, const int32_t* site,
-                              const double2* coefp) {
+// The lean kernel's tables for instance `only`: sizes and strides (P->lean64, lean32; pointers hold offsets into their
+// allocation until it is made), and the returned coefficient pairs, the products that the projector kernel forms, and
+// packed indices, which are small.  Empty where an index would not fit its field.
+std::vector<char> lean_tables(pyqed_heom_plan* P, int only, const double2* coefp) {
   const InstDev& I = P->inst[only];
   const int S = I.K + std::min(I.K, I.L), npair = I.K * (I.L + 2) * 2;
   if (S > kMaxEnt || npair > 65536 || (int64_t)I.nmax * S * (int64_t)sizeof(int2) > (int64_t(1) << 28)) return {};
-  std::vector<char> buf;
-  auto part = [&](size_t bytes) {
-    const size_t o = (buf.size() + 255) & ~size_t(255);
-    buf.resize(o + bytes);
+  size_t bytes = 0;
+  auto part = [&](size_t n) {
+    const size_t o = (bytes + 255) & ~size_t(255);
+    bytes = o + n;
     return o;
   };
-  const size_t oe = part((size_t)I.nmax * S * sizeof(int2)), os = part((size_t)I.nmax * 16), oij = part(4 * 64 * kLeanQ);
+  LeanTables t;
+  t.ent = (const int2*)part((size_t)I.nmax * S * sizeof(int2));
+  t.start = (const uint8_t*)part((size_t)I.nmax * 16);
   const size_t od64 = part(16 * (size_t)I.nmax), od32 = part(8 * (size_t)I.nmax);
-  const size_t op64 = part(32 * (size_t)npair), op32 = part(16 * (size_t)npair);
-  int2* le = (int2*)(buf.data() + oe);
-  uint8_t* ls = (uint8_t*)(buf.data() + os);
-  double* d64 = (double*)(buf.data() + od64);
-  float* d32 = (float*)(buf.data() + od32);
-  for (int a = 0; a < I.nmax; ++a) {
-    const int2* e = ent + rowptr[a];
-    const int n = rowptr[a + 1] - rowptr[a];
-    if (n > S) return {};
-    uint8_t* first = ls + (size_t)a * 16;
-    int at[16] = {0};
-    for (int t = 0; t < n; ++t) ++at[site[e[t].y & 0xffff] + 1];
-    for (int s = 0; s < I.d; ++s) at[s + 1] += at[s];
-    for (int s = 0; s <= I.d; ++s) first[s] = (uint8_t)at[s];
-    double v64[2][kMaxEnt];
-    float v32[2][kMaxEnt];
-    for (int t = 0; t < n; ++t) {
-      const int k = e[t].y & 0xffff, nf = (e[t].y >> 16) & 0x7f, plus = e[t].y < 0, s = site[k];
-      // stable: entries of a site keep the table's order
-      le[(size_t)a * S + at[s]++] = make_int2(e[t].x * I.d + s, s << 16 | ((k * (I.L + 2) + nf) * 2 + plus));
-      const double2 g = plus ? make_double2(0, 0) : coefp[5 * k];
-      v64[0][t] = g.x * (double)nf, v64[1][t] = g.y * (double)nf;
-      v32[0][t] = (float)g.x * (float)nf, v32[1][t] = (float)g.y * (float)nf;
-    }
-    // the butterfly's tree without the terms past the list, which are zero
-    for (int o = 32, m = n; o > 0 && m > 1; o >>= 1) {
-      for (int t = 0; t + o < m; ++t)
-        for (int c = 0; c < 2; ++c) v64[c][t] += v64[c][t + o], v32[c][t] += v32[c][t + o];
-      m = std::min(m, o);
-    }
-    for (int c = 0; c < 2; ++c) {
-      d64[2 * (size_t)a + c] = n ? v64[c][0] : 0.0;
-      d32[2 * (size_t)a + c] = n ? v32[c][0] : 0.0f;
-    }
-  }
+  P->lean_bytes = bytes;
+  bytes = 0;
+  const size_t op64 = part(32 * (size_t)npair), op32 = part(16 * (size_t)npair), oij = part(4 * 64 * kLeanQ);
+  std::vector<char> buf(bytes);
   double* p64 = (double*)(buf.data() + op64);
   float* p32 = (float*)(buf.data() + op32);
   for (int k = 0; k < I.K; ++k)
@@ -2887,8 +2904,7 @@ std::vector<char> lean_tables(pyqed_heom_plan* P, int only, const int32_t* rowpt
   int32_t* ij = (int32_t*)(buf.data() + oij);
   for (int i = 0, q = 0; i < I.d; ++i)
     for (int j = i; j < I.d; ++j) ij[q++] = i << 8 | j;
-  LeanTables t;
-  t.ent = (const int2*)oe, t.start = (const uint8_t*)os, t.ij = (const int32_t*)oij;
+  t.ij = (const int32_t*)oij;
   t.damp = (const void*)od64, t.pair = (const void*)op64;
   t.stride = S;
   t.dmag = (uint32_t)(((1 << 20) + I.d - 1) / I.d);
@@ -2912,6 +2928,15 @@ size_t resident_lds_bytes(const pyqed_heom_plan* P, int64_t n_el, size_t extra, 
 size_t resident_extra_bytes(int d, int ncoup, bool dense, int nmax, int64_t nent) {
   const size_t nq = dense ? 0 : (size_t)ncoup * d;
   return 16 * (2 * (size_t)d * d + 2 * nq) + (2 * 16 + 8) * (size_t)nent + 16 * (size_t)nmax + 4 * (size_t)(nmax + 1);
+}
+
+int fill_lean_tables(pyqed_heom_plan* P) {
+  const InstDev& I = P->inst[P->lean_inst];
+  hipLaunchKernelGGL(heom_lean_tables_kernel, dim3((I.nmax + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0, nullptr, I,
+                     P->d_rowptr, P->d_ent, P->d_site, P->d_coefp, P->lean64, (double2*)P->lean64.damp, (float2*)P->lean32.damp);
+  PQA_HIP(hipGetLastError());
+  PQA_HIP(hipStreamSynchronize(nullptr));  // before any stream's first run
+  return PYQED_OK;
 }
 
 // The work queue and, per instance, the range [first, last) of its items: tile() lists the items of one
@@ -2946,6 +2971,7 @@ void destroy_plan(pyqed_heom_plan* P) {
   release(P, P->d_ent);
   for (int c = 0; c < kClasses; ++c) release(P, P->d_entfix[c]);
   release(P, P->d_lean);
+  release(P, P->d_lean_pairs);
   release(P, P->d_coef);
   release(P, P->d_mode);
   release(P, P->d_mat);
@@ -3373,8 +3399,7 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
     int only = -1, count = 0;
     for (int i = 0; i < n_inst; ++i)
       if (!is_res[i] && P->inst[i].path == 1) only = i, ++count;
-    if (count == 1) lean = lean_tables(P, only, rowptr.data() + P->inst[only].rowptr_off, ent.data() + P->inst[only].ent_off,
-                                       sites.data() + P->inst[only].site_off, coefp.data() + P->inst[only].coefp_off);
+    if (count == 1) lean = lean_tables(P, only, coefp.data() + P->inst[only].coefp_off);
   }
   retile(P, 0, 8);
   // ---- upload
@@ -3382,7 +3407,7 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
   Arena arena;
   for (int c = 1; c < kClasses && rc == 0; ++c)
     if (!entfix[c].empty()) rc = arena.add(entfix[c], &P->d_entfix[c]);
-  if (rc || (rc = arena.add(lean, &P->d_lean)) || (rc = arena.add(P->inst, &P->d_inst)) || (rc = upload_items(P, &arena)) ||
+  if (rc || (rc = arena.add(lean, &P->d_lean_pairs)) || (rc = arena.reserve(P->lean_bytes, &P->d_lean)) || (rc = arena.add(P->inst, &P->d_inst)) || (rc = upload_items(P, &arena)) ||
       (rc = arena.add(rowptr, &P->d_rowptr)) || (rc = arena.add(ent, &P->d_ent)) || (rc = arena.add(coef, &P->d_coef)) ||
       (rc = arena.add(mode, &P->d_mode)) || (rc = arena.add(mat, &P->d_mat)) || (rc = arena.add(P->resident, &P->d_res)) ||
       (rc = arena.add(sites, &P->d_site)) || (rc = arena.add(coefp, &P->d_coefp)) || (rc = arena.send(&P->d_arena))) {
@@ -3390,14 +3415,19 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
     return rc;
   }
   P->arena_bytes = arena.host.size();
-  if (!lean.empty())
-    for (LeanTables* t : {&P->lean64, &P->lean32}) {  // offsets from the buffer's start until now
+  if (!lean.empty()) {
+    for (LeanTables* t : {&P->lean64, &P->lean32}) {  // offsets until now
       t->ent = (const int2*)(P->d_lean + (intptr_t)t->ent);
       t->start = (const uint8_t*)(P->d_lean + (intptr_t)t->start);
       t->damp = P->d_lean + (intptr_t)t->damp;
-      t->pair = P->d_lean + (intptr_t)t->pair;
-      t->ij = (const int32_t*)(P->d_lean + (intptr_t)t->ij);
+      t->pair = P->d_lean_pairs + (intptr_t)t->pair;
+      t->ij = (const int32_t*)(P->d_lean_pairs + (intptr_t)t->ij);
     }
+    if ((rc = fill_lean_tables(P))) {
+      destroy_plan(P);
+      return rc;
+    }
+  }
   // The streams that run_typed uses.  Packed plans with streamed work have both also where they use neither: their
   // chains of launches are 1% faster beside two idle streams (us per step: 7 sites at depth 4 FP64 28.4 without, 28.1
   // with; 16 sites at depth 3 114.1, 113.2), and such plans run many steps; the others save 160 us a plan.
