@@ -205,13 +205,14 @@ class HeomEngine:
         self.step = 0
 
     def workspace(self, prec, nsteps=POWER_STEPS, driven=False):
-        """Scratch of a call of nsteps steps.  plan_query's FP64 size holds the powers of a small hierarchy's generator
-        (up to 98 MB for a state of 164 KB): calls that only step do without, as do all where the device has no room."""
+        """Scratch of a call of nsteps steps.  plan_query's FP64 size holds the powers of a small hierarchy's generator,
+        up to 98 MB for a state of 10 KB.  Above 16 MB, calls that only step do without, and every call does where the
+        device has no room; below, one size serves all, so that a long call after a short one allocates nothing."""
         torch = self.torch
         need = self.ws_bytes[prec]
         # stepping: the state, and two stage buffers of 8 bytes an element in mixed precision, 16 in FP64
         step = 2 * self.ws_bytes[_lib.PREC_MIXED] - -(-16 * self.n_elems // 256) * 256
-        if prec == _lib.PREC_FP64 and (driven or nsteps < POWER_STEPS or self._no_room):
+        if prec == _lib.PREC_FP64 and (self._no_room or need > 16 << 20 and (driven or nsteps < POWER_STEPS)):
             need = min(need, step)
         if self._ws is None or self._ws.numel() < need:
             # captured graphs hold the old workspace's address: drop them before it is released
