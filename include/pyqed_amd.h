@@ -201,7 +201,8 @@ int pyqed_heom_plan_classes(const pyqed_heom_plan* plan, int64_t* items, int64_t
 /* Per kernel class (host array [4]): for classes 1 to 3 of a packed plan whose streamed work is a
  * single instance, that instance's index (class 1 then runs the lean kernel, whatever its tiling,
  * classes 2 and 3 the single-instance kernel: instance record from the kernel arguments, loaded once per
- * block, neighbour lists at a fixed stride); -1 otherwise, and always for class 0.
+ * block, neighbour lists at a fixed stride; FP64 launches of class 3 that do not fit LDS run the generic
+ * kernel); -1 otherwise, and always for class 0.
  * No counterpart in the reference; used to name the kernels a benchmark's launches run. */
 int pyqed_heom_plan_class_single(const pyqed_heom_plan* plan, int32_t* inst);
 /* RK4-state elements (size in y) of the streamed work per kernel class (host array [4]): equal to
@@ -293,7 +294,8 @@ int pyqed_liouville_run_work(int32_t N, int32_t nterm, const void* A, int32_t n_
  *   rho_out      device [n_inst][nsteps/save_every][d][d] or NULL
  *   work         device, >= pyqed_lindblad_work_bytes(d, nc, ndrive, n_inst) bytes; with
  *                pyqed_lindblad_table_bytes(d, nc) more, 16 x 16 blocks of the operators that are exactly
- *                zero are found once per call and skipped (same results) */
+ *                zero are found once per call and skipped (the same results; a run that overflows on the way
+ *                spreads its infinities through the other blocks only) */
 int pyqed_lindblad_work_bytes(int32_t d, int32_t nc, int32_t ndrive, int32_t n_inst, int64_t* bytes);
 int pyqed_lindblad_table_bytes(int32_t d, int32_t nc, int64_t* bytes);
 int pyqed_lindblad_run(int32_t d, int32_t nc, const void* Heff, const void* HeffD, const void* C, const void* CD,

@@ -3013,7 +3013,9 @@ void retile(pyqed_heom_plan* P, int64_t target, int blocks_per_cu) {
     // the single-instance kernels pay nothing per item, so their items are as small as they get (one ADO per
     // wavefront) and the tail of a launch is short.  Step in us with 1, 2, 4 and 8 ADOs per wavefront and item:
     // 24 sites at depth 3 mixed 521, 566, 591, 806, FP64 1093, 1165, 1187, 1667; 14 sites at depth 4 mixed 229,
-    // 229, 255, 346; 16 sites at depth 3 mixed 75, 87, 138, 244
+    // 229, 255, 346; 16 sites at depth 3 mixed 75, 87, 138, 244.  Where the wide class's FP64 rows do not fit LDS (from 26
+    // sites with two exponentials each on) the generic kernel takes the items, and small ones are the faster there
+    // too: one ADO per wavefront and 8192 elements, 28 sites at depth 3 12.2 and 15.2 ms, at depth 2 1.3 and 3.8 ms
     P->cls_target[c] = automatic && P->one_inst[c] >= 0 ? 1 : P->tile_target;
     P->cls_bpc[c] = P->blocks_per_cu;
   }
@@ -3428,9 +3430,10 @@ extern "C" int pyqed_heom_plan_create(const pyqed_heom_instance* in, int32_t n_i
       return rc;
     }
   }
-  // The streams that run_typed uses.  Packed plans with streamed work have both also where they use neither: their
-  // chains of launches are 1% faster beside two idle streams (us per step: 7 sites at depth 4 FP64 28.4 without, 28.1
-  // with; 16 sites at depth 3 114.1, 113.2), and such plans run many steps; the others save 160 us a plan.
+  // The streams that run_typed uses.  Packed plans with streamed work keep both also where they use neither, as all
+  // plans once did: a step of 16 sites at depth 3 in FP64 takes 112.3 us with them and 114.5 without (112.1 to 112.5 and
+  // 114.4 to 114.7 in six processes in turn), of 7 sites at depth 4 28.6 and 28.7.  Why idle streams help is not known;
+  // the figure alone decides, and a plan pays 160 us for it, 70 steps' worth.  The other plans save those.
   const auto stream = [](hipStream_t* s, hipEvent_t* fork, hipEvent_t* join) {
     return hipStreamCreateWithFlags(s, hipStreamNonBlocking) == hipSuccess &&
            hipEventCreateWithFlags(fork, hipEventDisableTiming) == hipSuccess &&

@@ -20,7 +20,7 @@
 // local operators), so a bit table made once per call marks the 16 x 16 operator blocks that hold a
 // nonzero real or imaginary part; blocks, and the real products of a part, that are exactly zero are
 // skipped.  A non-finite value anywhere in the inputs marks every block, so that it spreads as in the
-// full product.
+// full product; one that a run makes on its way spreads through the marked blocks only.
 //
 // Measured (MI355X) against one workgroup per instance with 4 x 4 register blocks on the vector ALU, which
 // left 255 CUs idle for a single instance and was bound by its LDS reads otherwise: a step of one dense
@@ -789,7 +789,9 @@ extern "C" int pyqed_lindblad_run(int32_t d, int32_t nc, const void* Heff, const
   // dimension.  us per step with two collapse operators, launches against resident, dense / banded operators:
   // d = 16: 30-39 / 23, 29-38 / 19; d = 32: 39 / 48, 36 / 31 for one instance, 96 / 48, 78 / 32 for 256;
   // d = 48: 98 / 138, 71 / 54 for 64, 137 / 138, 97 / 55 for 128; d = 64: 129 / 231, 82 / 75 for 64,
-  // 224 / 233, 131 / 75 for 128, 368 / 233, 181 / 75 for 256.
+  // 224 / 233, 131 / 75 for 128, 368 / 233, 181 / 75 for 256.  The numbers of instances are those from which dense
+  // operators are the faster; which operators a call has is known on the device alone, and banded ones would gain up
+  // to a quarter by going over earlier (d = 48 and 64 from 64 instances on).
   constexpr int kResFrom[5] = {0, 1, 16, 96, 96};
   if (p.nt <= 4 && n_inst >= kResFrom[p.nt] && nc <= 256) {
     switch (p.nt) {

@@ -14,9 +14,9 @@
 // run relative to the stepping kernels' (states, Frobenius norm; in brackets the largest element), 30 Lindblad systems
 // of d = 2..16 and Redfield oscillators of d = 3..20 with 100..1000 steps: 0.53 (0.72) on geometric mean, at most
 // 0.85 (1.7); populations of 12 small hierarchies (heom.hip) 0.24 (0.37), at most 0.61 (1.0).  Powers formed in
-// FP64 had 2.2 to 2.4 (1.9 to 2.9) at N = 256.  Their cost: 400 steps of N = 256 100 -> 190 us, of which 10 launches
-// of 22 us form and square matrices (the FP64 matrix cores; 9 before), 1000 steps of N = 84 130 -> 150, of N = 64
-// 105 -> 110.
+// FP64 had 2.2 to 2.4 (1.9 to 2.9) at N = 256.  Their cost in kernel time: 400 steps of N = 256 125 -> 220 us, of which
+// 8 launches of 19 to 22 us form and square matrices (the FP64 matrix cores; 8 to 10 before), 1000 steps of N = 84
+// 115 -> 145, of N = 64 100 -> 125.
 //
 // The entries of D_j for a mode that this dt makes unstable grow like |P|^(2^j).  Such a mode may belong to a coherence
 // that the state never excites, as one with a far level that nothing couples to, and steps then leave it at exactly
